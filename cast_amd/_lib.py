@@ -65,6 +65,8 @@ SIGNATURES: dict[str, list] = {
     "rcsa_route_check": [_P, _P, _P, _P, _I, _I, _I, _I, _P, _P],
     "rcsa_quantize_rows_int8": [_P, c_int, _I, _I, _I, _P, _P, _P],
     "rcsa_int8_linear": [_P, _P, _P, _P, _P, _I, _I, _I, _P, _I, _P],
+    "rcsa_order_lists_max_blocks": [],
+    "rcsa_order_lists": [_P, _P] + [_I] * 6 + [_P] + [_I] * 6 + [_P, _P, _P, _I, _P, _P],
     "rcsa_pack_tokens": [_P, c_int, _I, _I, _I, _I, _I, _I, _I, _P, _I, _P, _P],
     "rcsa_unpack_tokens": [_P, _I, _I, _I, _I, _P, _I, _P, _P],
     "rcsa_status_string": [c_int],
@@ -94,7 +96,8 @@ def load() -> ctypes.CDLL:
         fn.argtypes = argtypes
         fn.restype = (ctypes.c_char_p if name == "rcsa_status_string"
                       else c_int64 if name in ("rcsa_attn_workspace_bytes",
-                                               "rcsa_attn_noalloc_scratch_bytes")
+                                               "rcsa_attn_noalloc_scratch_bytes",
+                                               "rcsa_order_lists_max_blocks")
                       else c_int)
     _lib = lib
     return lib

@@ -34,11 +34,24 @@ def longcat_active(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, indices: t
             and k.shape[2] % block_size == 0:
         # the validity as bits (32 keys a word): the attention then reads 8 bytes
         # per wavefront and block instead of staging the bytes (about 6% faster)
+        indices, counts, bits, ordered = _lists_and_bits(k, indices, counts, key_valid,
+                                                         block_size)
         return ops.sparse_attn_bf16(q, k, v, indices, counts, None, block_m=block_size,
-                                    block_n=block_size,
-                                    block_mask=ops.valid_bits(key_valid, block_size))
+                                    block_n=block_size, block_mask=bits, ordered=ordered)
     return ops.sparse_attn_bf16(q, k, v, indices, counts, key_valid.to(torch.uint8).contiguous(),
                                 block_m=block_size, block_n=block_size)
+
+
+def _lists_and_bits(k, indices, counts, key_valid, block_n):
+    """The lists in ascending order where that helps (and they have the attention's
+    form; otherwise it refuses them itself) and the validity bits, in one launch."""
+    B, H, L, D = k.shape
+    if (k.is_cuda and indices.is_cuda and counts.is_cuda and key_valid.is_cuda
+            and indices.ndim == 4 and counts.shape == indices.shape[:3]
+            and indices.shape[:2] in ((B, H), (1, H), (B, 1), (1, 1))
+            and ops.order_helps(B * H, L, 4 * D, block_n, indices.shape[3])):
+        return (*ops.order_lists(indices, counts, L // block_n, valid=key_valid), True)
+    return indices, counts, ops.valid_bits(key_valid, block_n), False
 
 
 def longcat_asymmetric(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor,

@@ -18,7 +18,7 @@ from ._lib import RCSA_BF16, RCSA_F32, RCSA_ORDER_INDEX, RCSA_ORDER_RANK, check
 __all__ = [
     "pool_query", "pool_key", "block_scores", "select_topk", "quantize_key",
     "sparse_attn_bf16", "sparse_attn_int8", "pack_tokens", "unpack_tokens", "row_budgets",
-    "quantize_key_select",
+    "quantize_key_select", "order_lists",
 ]
 
 
@@ -560,12 +560,74 @@ def _check_block_mask(block_mask, Lk, block_n, device, fn):
     return block_mask.contiguous()
 
 
+_L2_BYTES = 4 << 20  # one XCD's L2
+
+
+def order_helps(n_bh: int, k_len: int, key_bytes: int, block_n: int, max_k: int) -> bool:
+    """Whether the attention orders its block lists: when the K and V rows
+    (``key_bytes`` per key) of the heads an XCD works on exceed its L2, ascending
+    lists let the query blocks of a head share what they stream (bf16, 24 heads x
+    28 query blocks x 85 of 303 key blocks listed at random: the attention takes
+    473 us ordered against 540 us as given, the ordering itself under 5).  Smaller
+    planes stay in L2 in any order."""
+    return (max_k > 2 and -(-n_bh // 8) * k_len * key_bytes > _L2_BYTES
+            and -(-k_len // block_n) <= _lib.load().rcsa_order_lists_max_blocks())
+
+
+def order_lists(indices: torch.Tensor, counts: torch.Tensor, n_kblocks: int, *,
+                rows: Optional[torch.Tensor] = None, valid: Optional[torch.Tensor] = None):
+    """Block lists in ascending block order (``rcsa_order_lists``): ``(indices, counts)``
+    of the entries in ``[0, n_kblocks)``, repeats kept.  indices int32 ``[B|1, H|1, N,
+    maxK]``, counts int32 ``[B|1, H|1, N]``; ``rows`` (int64) picks rows of them.  With
+    ``valid`` (one flag per key, a multiple of 32) a third value follows: its bits as
+    :func:`valid_bits` gives them, flat, from the same launch."""
+    fn = "order_lists"
+    _require_cuda(fn, indices, counts)
+    if indices.dtype != torch.int32 or counts.dtype != torch.int32:
+        raise TypeError(f"{fn}: indices/lens must be int32")
+    if indices.ndim != 4 or counts.ndim != 3 or indices.stride(3) != 1 \
+            or indices.shape[2] != counts.shape[2]:
+        raise ValueError(f"{fn}: indices must be [B, H, N, maxK], lens [B, H, N]")
+    B, H = torch.broadcast_shapes(indices.shape[:2], counts.shape[:2])
+    indices, counts = _expand_lists(indices, counts, B, H)
+    # a broadcast list is ordered once
+    b = 1 if indices.stride(0) == 0 and counts.stride(0) == 0 else B
+    h = 1 if indices.stride(1) == 0 and counts.stride(1) == 0 else H
+    n_src, max_k = indices.shape[2:]
+    n_rows = n_src
+    if rows is not None:
+        rows = rows.to(device=indices.device, dtype=torch.int64).contiguous()
+        n_rows = rows.numel()
+    out = torch.empty(b, h, n_rows, max_k, device=indices.device, dtype=torch.int32)
+    lens = torch.empty(b, h, n_rows, device=indices.device, dtype=torch.int32)
+    bits = None
+    if valid is not None:
+        valid = _bytes_mask(valid.reshape(-1), indices.device)
+        bits = torch.empty(valid.numel() // 32, device=indices.device, dtype=torch.int32)
+    check(_lib.load().rcsa_order_lists(
+        indices.data_ptr(), counts.data_ptr(), *indices.stride()[:3], *counts.stride(),
+        _ptr(rows), n_src, b, h, n_rows, max_k, int(n_kblocks), out.data_ptr(),
+        lens.data_ptr(), _ptr(valid), 0 if valid is None else valid.numel(), _ptr(bits),
+        _stream()), fn)
+    out, lens = out.expand(B, H, -1, -1), lens.expand(B, H, -1)
+    return (out, lens) if valid is None else (out, lens, bits)
+
+
 def valid_bits(valid: torch.Tensor, block_size: int) -> torch.Tensor:
     """Per-key validity flags ``[n_blocks * block_size]`` as the attention's
     ``block_mask``: int32 ``[n_blocks, block_size // 32]``, bit i of word w of
     block n = key n * block_size + 32 w + i (the form the key pooling pass writes)."""
     if block_size % 32 or valid.numel() % block_size:
         raise ValueError("valid_bits: block_size must be a multiple of 32 dividing the keys")
+    if valid.is_cuda and valid.numel() > 0:
+        flags = _bytes_mask(valid.reshape(-1), valid.device)
+        bits = torch.empty(flags.numel() // block_size, block_size // 32, device=valid.device,
+                           dtype=torch.int32)
+        with torch.cuda.device(valid.device):
+            check(_lib.load().rcsa_order_lists(
+                None, None, 0, 0, 0, 0, 0, 0, None, 0, 0, 0, 0, 0, 0, None, None,
+                flags.data_ptr(), flags.numel(), bits.data_ptr(), _stream()), "valid_bits")
+        return bits
     words = (valid.reshape(-1, block_size // 32, 32) != 0).to(torch.int64)
     bits = (words << torch.arange(32, device=valid.device)).sum(-1)
     return torch.where(bits >= 2 ** 31, bits - 2 ** 32, bits).to(torch.int32)
@@ -580,7 +642,7 @@ def _bhld_strides(x: torch.Tensor, token_major: bool):
 def sparse_attn_bf16(q, k, v, indices, counts, valid=None, *, block_m=128, block_n=128,
                      sm_scale=None, return_lse=False, out=None, n_split=None,
                      block_mask=None, q_token=None, kv_token=None, out_token=None,
-                     out_len=None):
+                     out_len=None, ordered=False):
     """bf16 block-sparse attention; the ``_attn_fwd_bsa_align`` contract.
 
     q/k/v [B, H, L, D] bf16, indices int32 [B|1, H|1, NQB, maxK], counts
@@ -597,6 +659,7 @@ def sparse_attn_bf16(q, k, v, indices, counts, valid=None, *, block_m=128, block
     v[:, flat] packing of P/matrix_curvature_phase_frame_weave.py:5677-5684)
     and writes the output (and LSE) to the token rows, ``[B, Lq_tokens, H, D]``
     (P/matrix_curvature_phase_frame_weave.py:6095).  Empty slots read zeros.
+    ``ordered``: the lists are ascending already (:func:`order_lists` is not run).
     ``out_token`` / ``out_len`` (with the maps) write output row r to row
     ``out_token[r]`` of ``[B, out_len, H, D]`` instead, e.g. a relay layer's
     query-frame rows (P/matrix_curvature_phase_frame_weave.py:8990-8994).
@@ -641,6 +704,8 @@ def sparse_attn_bf16(q, k, v, indices, counts, valid=None, *, block_m=128, block
         kv = None
     else:
         kv = _valid_u8(valid, Lk, q.device, fn)
+    if not ordered and order_helps(B * H, Lk, 4 * D, block_n, indices.shape[3]):
+        indices, counts = order_lists(indices, counts, -(-Lk // block_n))
     n_rows = n_out if gathered else Lq
     if out is None:
         out = (torch.empty(B, n_out, H, D, device=q.device, dtype=torch.bfloat16) if gathered
@@ -663,7 +728,7 @@ def sparse_attn_bf16(q, k, v, indices, counts, valid=None, *, block_m=128, block
 def sparse_attn_int8(q_i8, q_scale, k_i8, k_scale, v, indices, counts, valid=None, *,
                      block_m=128, block_n=128, sm_scale=None, return_lse=False, out=None,
                      n_split=None, block_mask=None, out_token=None, out_len=None,
-                     v_token=None):
+                     v_token=None, ordered=False):
     """int8-QK / bf16-PV block-sparse attention over quantiser outputs.
 
     ``block_mask`` (int32 ``[ceil(Lk / block_n), block_n // 32]``, e.g. from
@@ -675,7 +740,8 @@ def sparse_attn_int8(q_i8, q_scale, k_i8, k_scale, v, indices, counts, valid=Non
     ``v_token`` (a slot -> token map of the packed keys; needs ``block_mask``,
     D 128, 128-token blocks) reads V rows from a token-major ``[B, Lv_tokens, H, D]``
     v through the map inside the attention's copy ring (the v[:, flat] packing
-    of P/matrix_curvature_phase_frame_weave.py:5677-5684); empty slots read zeros."""
+    of P/matrix_curvature_phase_frame_weave.py:5677-5684); empty slots read zeros.
+    ``ordered``: the lists are ascending already (:func:`order_lists` is not run)."""
     fn = "sparse_attn_int8"
     _require_cuda(fn, q_i8, q_scale, k_i8, k_scale, v, indices, counts)
     _attn_common(q_i8, k_i8, v, indices, counts, fn)
@@ -711,6 +777,8 @@ def sparse_attn_int8(q_i8, q_scale, k_i8, k_scale, v, indices, counts, valid=Non
         kv = None
     else:
         kv = _valid_u8(valid, Lk, q_i8.device, fn)
+    if not ordered and order_helps(B * H, Lk, 3 * D, block_n, indices.shape[3]):
+        indices, counts = order_lists(indices, counts, nkb)
     if out_token is not None:
         om = _slot_map(out_token, block_m, q_i8.device, fn)
         if om.numel() < Lq or out_len is None or int(out_len) <= 0:

@@ -164,7 +164,8 @@ def rcsa_attention(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor,
                                    block_m=bs, block_n=bs, sm_scale=scale,
                                    return_lse=return_lse, n_split=n_split, block_mask=k_mask,
                                    out_token=q_slot_token if gathered else None,
-                                   out_len=q.shape[1] if gathered else None, v_token=v_token)
+                                   out_len=q.shape[1] if gathered else None, v_token=v_token,
+                                   ordered=order == "index")
     else:
         k_i8 = k_scale = kmean = None
         qb = q if q.dtype == torch.bfloat16 else q.to(torch.bfloat16)
@@ -174,7 +175,8 @@ def rcsa_attention(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor,
                                    sm_scale=scale, return_lse=return_lse, n_split=n_split,
                                    block_mask=k_mask,
                                    q_token=q_slot_token if gathered else None,
-                                   kv_token=k_slot_token if gathered else None)
+                                   kv_token=k_slot_token if gathered else None,
+                                   ordered=order == "index")
     out, lse = res if return_lse else (res, None)
     return RCSAResult(out, idx4, cnt3, score, qhat, khat, lse, q_i8, q_scale, k_i8, k_scale,
                       kmean, k_mask)
@@ -206,8 +208,17 @@ def relay_attention(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, layout, s
     if k.shape != q.shape or v.shape != q.shape:
         raise ValueError("relay_attention: q, k and v must be token-major [B, S, H, D] alike")
     rows = layout.query_block_ids.to(selected.device)
-    idx = selected.index_select(2, rows).to(torch.int32).contiguous()
-    cnt = counts.index_select(2, rows).to(torch.int32).contiguous()
+    n_kblocks = layout.key_slot_token.numel() // bs
+    ordered = (selected.dtype == torch.int32 and counts.dtype == torch.int32
+               and selected.stride(3) == 1 and selected.shape[:3] == counts.shape
+               and selected.shape[2] == layout.n_blocks
+               and ops.order_helps(B * H, n_kblocks * bs, (3 if int8 else 4) * D, bs,
+                                   selected.shape[3]))
+    if ordered:  # the query blocks' rows, ascending, in one launch
+        idx, cnt = ops.order_lists(selected, counts, n_kblocks, rows=rows)
+    else:
+        idx = selected.index_select(2, rows).to(torch.int32).contiguous()
+        cnt = counts.index_select(2, rows).to(torch.int32).contiguous()
     n_out = layout.query_indices.numel()
     scale = 1.0 / math.sqrt(D) if sm_scale is None else sm_scale
     if int8:
@@ -222,11 +233,13 @@ def relay_attention(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, layout, s
                                     block_m=bs, block_n=bs, sm_scale=scale,
                                     return_lse=return_lse, n_split=n_split,
                                     block_mask=k_mask, out_token=layout.query_out_row,
-                                    out_len=n_out, v_token=layout.key_slot_token)
+                                    out_len=n_out, v_token=layout.key_slot_token,
+                                    ordered=ordered)
     qb, kb, vb = (x if x.dtype == torch.bfloat16 else x.to(torch.bfloat16) for x in (q, k, v))
     return ops.sparse_attn_bf16(qb, kb, vb, idx, cnt, None, block_m=bs, block_n=bs,
                                 sm_scale=scale, return_lse=return_lse, n_split=n_split,
                                 block_mask=layout.key_block_mask,
                                 q_token=layout.query_slot_token,
                                 kv_token=layout.key_slot_token,
-                                out_token=layout.query_out_row, out_len=n_out)
+                                out_token=layout.query_out_row, out_len=n_out,
+                                ordered=ordered)

@@ -167,7 +167,8 @@ def _available_layers(weave):
                         if isinstance(k, tuple) and len(k) == 2 and int(k[0]) == step)
 
 
-def _attention(q, k, v, idx4, cnt3, slot, token_to_packed, mask, bs, int8: bool, kq=None):
+def _attention(q, k, v, idx4, cnt3, slot, token_to_packed, mask, bs, int8: bool, kq=None,
+               ordered=False):
     """Block-sparse attention of the packed blocks named by the slot map, the
     output in the token rows [B, L, H, D] (bf16).  The copy rings read the
     token-major sources through the slot map for D 128 and 128-token blocks;
@@ -180,14 +181,14 @@ def _attention(q, k, v, idx4, cnt3, slot, token_to_packed, mask, bs, int8: bool,
         return ops.sparse_attn_int8(q_i8, q_scale, k_i8, k_scale,
                                     vb if ring else ops.pack_tokens(vb, slot), idx4, cnt3, None,
                                     block_m=bs, block_n=bs, block_mask=mask, out_token=slot,
-                                    out_len=L, v_token=slot if ring else None)
+                                    out_len=L, v_token=slot if ring else None, ordered=ordered)
     qb, kb = (x if x.dtype == torch.bfloat16 else x.to(torch.bfloat16) for x in (q, k))
     if ring:
         return ops.sparse_attn_bf16(qb, kb, vb, idx4, cnt3, None, block_m=bs, block_n=bs,
-                                    block_mask=mask, q_token=slot, kv_token=slot)
+                                    block_mask=mask, q_token=slot, kv_token=slot, ordered=ordered)
     packed = [ops.pack_tokens(x, slot) for x in (qb, kb, vb)]
     out = ops.sparse_attn_bf16(*packed, idx4, cnt3, None, block_m=bs, block_n=bs,
-                               block_mask=mask)
+                               block_mask=mask, ordered=ordered)
     return ops.unpack_tokens(out, token_to_packed.to(device=q.device, dtype=torch.long))
 
 
@@ -313,7 +314,10 @@ def compact_cwca_attention(weave, module: Any, q: torch.Tensor, k: torch.Tensor,
 
     # ---- top-k at each row's degree, local blocks first (:5829-5832) ----
     row_k = degrees.to(torch.int32)
-    indices, _ = ops.select_topk(score, row_k, forced=local, max_k=width, order="rank")
+    # only the router reads the rank order; the attention takes ascending lists
+    ordered = route != "refine"
+    indices, _ = ops.select_topk(score, row_k, forced=local, max_k=width,
+                                 order="index" if ordered else "rank")
     selected = indices.view(B, H, blocks, width)
     counts = row_k[None, None].expand(B, H, -1).contiguous()
 
@@ -367,7 +371,7 @@ def compact_cwca_attention(weave, module: Any, q: torch.Tensor, k: torch.Tensor,
 
     # ---- attention and unpack (:6086-6095) ----
     out = _attention(q, k, v, selected.to(torch.int32).contiguous(), counts, slot,
-                     layout.compact_token_to_packed, mask, bs, int8, kq)
+                     layout.compact_token_to_packed, mask, bs, int8, kq, ordered)
     if provider is not None:  # the closed loop conserves blocks * mean_degree edges
         edges, mean_f = blocks * mean_degree, float(mean_degree)
     else:

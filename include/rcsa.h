@@ -576,6 +576,30 @@ int rcsa_route_check(const int32_t* base, const int32_t* selected, const int32_t
                      int64_t memory_blocks, int64_t max_k, int32_t* out, hipStream_t stream);
 
 /*
+ * Block lists in ascending block order, and key validity flags as bits.
+ *
+ * rcsa_order_lists: row r of (b, h) of block_indices (stride_b*: batch, head,
+ * row; entries contiguous) and its length (stride_l*) become list r of
+ * out_indices [B][H][n_rows][max_k] and out_lens [B][H][n_rows]: the first
+ * min(max(len, 0), max_k) entries that name a block in [0, n_kblocks), ascending,
+ * repeats kept, the rest -1.  rows (int64 [n_rows], NULL: r itself) picks source
+ * rows out of n_src_rows.  The attention's result over the ordered lists is that
+ * over the given ones up to the rounding of its sums; it reads them with fewer
+ * cache misses.  n_kblocks <= rcsa_order_lists_max_blocks(), max_k < 2^24.
+ * valid (one byte per key, n_valid of them) with valid_bits (ceil(n_valid / 32)
+ * words: bit i of word w = key 32 w + i), both or neither, in the same launch;
+ * block_indices may be NULL when only the bits are wanted.
+ */
+int64_t rcsa_order_lists_max_blocks(void);
+int rcsa_order_lists(const int32_t* block_indices, const int32_t* block_indices_lens,
+                     int64_t stride_bz, int64_t stride_bh, int64_t stride_bm,
+                     int64_t stride_lz, int64_t stride_lh, int64_t stride_lm,
+                     const int64_t* rows, int64_t n_src_rows, int64_t B, int64_t H,
+                     int64_t n_rows, int64_t max_k, int64_t n_kblocks, int32_t* out_indices,
+                     int32_t* out_lens, const uint8_t* valid, int64_t n_valid,
+                     uint32_t* valid_bits, hipStream_t stream);
+
+/*
  * Shared int8 Q/K/V projection (P/matrix_shared_int8_qkv.py:19-92): the
  * activations are quantised once per token and reused by the three int8
  * projections.  No reference kernel: the reference calls the upstream Matrix
