@@ -52,6 +52,7 @@ COMMON_FLAGS = [
 # only under the memory-clause scheduler.
 FILE_FLAGS = {
     "sparse_attn.hip": ["-mllvm", "-amdgpu-sched-strategy=max-ilp"],
+    "sparse_attn_shapes.hip": ["-mllvm", "-amdgpu-sched-strategy=max-ilp"],
     "sparse_attn_bf16_cu3.hip": ["-mllvm", "-amdgpu-sched-strategy=max-memory-clause"],
 }
 

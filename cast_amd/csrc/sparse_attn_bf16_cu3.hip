@@ -10,9 +10,9 @@ namespace rcsa {
 
 int launch_bf16_cu3(AttnArgs& a, dim3 grid, bool gather, hipStream_t s) {
   if (gather)
-    sparse_attn_kernel<false, 128, 128, 128, 3, 32, 1, true, true, 3><<<grid, dim3(256), 0, s>>>(a);
+    sparse_attn_kernel<false, 128, 128, 128, 32, 1, true, true, 3><<<grid, dim3(256), 0, s>>>(a);
   else
-    sparse_attn_kernel<false, 128, 128, 128, 3, 32, 1, false, false, 3><<<grid, dim3(256), 0, s>>>(a);
+    sparse_attn_kernel<false, 128, 128, 128, 32, 1, false, false, 3><<<grid, dim3(256), 0, s>>>(a);
   return launch_status();
 }
 

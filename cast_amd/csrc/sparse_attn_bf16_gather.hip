@@ -6,7 +6,7 @@
 namespace rcsa {
 
 int launch_bf16_gather(AttnArgs& a, dim3 grid, hipStream_t s) {
-  sparse_attn_kernel<false, 128, 128, 128, 3, 64, 2, true, true><<<grid, dim3(512), 0, s>>>(a);
+  sparse_attn_kernel<false, 128, 128, 128, 64, 2, true, true><<<grid, dim3(512), 0, s>>>(a);
   return launch_status();
 }
 

@@ -14,13 +14,13 @@ namespace rcsa {
 int launch_int8_cu3(AttnArgs& a, dim3 grid, bool gather, bool bits, hipStream_t s) {
   constexpr int kThreads = 128 / 32 * 64;  // BLOCK_M / 32 row groups, one key half
   if (gather)
-    sparse_attn_kernel<true, 128, 128, 128, 3, 32, 1, true, true, 3>
+    sparse_attn_kernel<true, 128, 128, 128, 32, 1, true, true, 3>
         <<<grid, dim3(kThreads), 0, s>>>(a);
   else if (bits)
-    sparse_attn_kernel<true, 128, 128, 128, 3, 32, 1, true, false, 3>
+    sparse_attn_kernel<true, 128, 128, 128, 32, 1, true, false, 3>
         <<<grid, dim3(kThreads), 0, s>>>(a);
   else
-    sparse_attn_kernel<true, 128, 128, 128, 3, 32, 1, false, false, 3>
+    sparse_attn_kernel<true, 128, 128, 128, 32, 1, false, false, 3>
         <<<grid, dim3(kThreads), 0, s>>>(a);
   return launch_status();
 }

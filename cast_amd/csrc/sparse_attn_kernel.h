@@ -15,8 +15,8 @@
 //
 // Staging: each selected K tile (row-major, 16-byte chunks XOR-swizzled) and
 // V tile (row-major, swizzled) is copied global -> LDS with direct-to-LDS
-// loads (no VGPR round trip), double buffered: the copy of block i+1 is in
-// flight while block i is computed.
+// loads (no VGPR round trip) into a 3-slot ring: the copies of the next two
+// steps are in flight while one is computed.
 //
 // Orientation: a wavefront computes S^T = K Q^T with 32x32 MFMAs, so a lane
 // owns ONE query row (column lane%32 of the MFMA output).  The K rows fed to
@@ -169,8 +169,9 @@ static __device__ uint8_t kAllValid[128] = {RCSA_ONES16, RCSA_ONES16, RCSA_ONES1
 // block); NKH key halves split every staged step between wavefronts.  WPE > 0:
 // several workgroups share a compute unit, WPE waves per SIMD in all (a
 // register budget of 512 / WPE); 0: one workgroup per compute unit.
-template <bool INT8, int D, int BM, int BN, int STAGES, int BNS, int NKH, int WPE = 0>
+template <bool INT8, int D, int BM, int BN, int BNS, int NKH, int WPE = 0>
 struct AttnCfg {
+  static constexpr int STAGES = 3;               // ring slots
   static constexpr int NRG = BM / 32;            // row groups
   static constexpr int NW = NRG * NKH;           // wavefronts: row group x key half
   static constexpr int NT = NW * 64;             // threads
@@ -189,23 +190,22 @@ struct AttnCfg {
   static constexpr int BUF = KBYTES + VBYTES;    // one ring slot: K tile then V tile
   static constexpr int KUNITS = KBYTES / 1024;   // 1 KiB direct-to-LDS copies
   static constexpr int VUNITS = VBYTES / 1024;
-  static constexpr int KUPW = (KUNITS + NW - 1) / NW;  // copies per wavefront
-  static constexpr int VUPW = (VUNITS + NW - 1) / NW;
+  static constexpr int KUPW = KUNITS / NW;       // copies per wavefront
+  static constexpr int VUPW = VUNITS / NW;
   static constexpr int DMA = KUPW + VUPW;
   static constexpr int K_RPU = 1024 / KROW;      // rows per copy
   static constexpr int V_RPU = 1024 / VROW;
   static constexpr int MW = NDT * 16 * 64 + 128; // floats of one row group's merge partial
   static constexpr int MPER = (NRG + STAGES - 1) / STAGES;  // partials per slot
-  // a 3-slot ring's slots are grown to hold the key-half merge partials (the
+  // the ring's slots are grown to hold the key-half merge partials (the
   // 64-key bf16 ring: 2 x 16.5 KiB in each 32.25 KiB slot); workgroups that
   // share a compute unit have one key half and no merge
-  static constexpr int SLOT = (WPE == 0 && STAGES == 3 && MPER * MW * 4 > BUF + 256)
+  static constexpr int SLOT = (WPE == 0 && NKH == 2 && MPER * MW * 4 > BUF + 256)
                                   ? MPER * MW * 4 : BUF + 256;
   static constexpr bool MERGE_IN_SLOTS = MPER * MW * 4 <= SLOT;
-  // the vmcnt accounting of a 3-deep ring needs the same copy count on every wavefront
-  static_assert(STAGES == 2 || (KUNITS % NW == 0 && VUNITS % NW == 0), "uneven copies");
+  // the ring's vmcnt accounting needs the same copy count on every wavefront
+  static_assert(KUNITS % NW == 0 && VUNITS % NW == 0, "uneven copies");
   static_assert(QSTEPS * 2 == CPR_K, "K chunk layout");
-  static_assert(STAGES == 2 || STAGES == 3, "ring depth");
   static_assert((NKH == 1 || NKH == 2) && HK % 32 == 0 && BN % BNS == 0, "key split");
   static_assert(BNS <= 256, "validity bytes of one step fit the slot tail");
   static_assert(WPE == 0 || NKH == 1, "workgroups sharing a compute unit merge no key halves");
@@ -233,30 +233,30 @@ constexpr int attn_waves_min() { return WPE > 0 ? WPE : (NT / 256 > 1 ? NT / 256
 template <int WPE>
 constexpr int attn_waves_max() { return WPE > 0 ? WPE : 8; }
 
-template <bool INT8, int D, int BM, int BN, int STAGES, int BNS, int NKH, bool MASK,
+template <bool INT8, int D, int BM, int BN, int BNS, int NKH, bool MASK,
           bool GATHER = false, int WPE = 0>
 __global__ void __launch_bounds__(BM * 2 * NKH)  // == AttnCfg::NT
 __attribute__((amdgpu_waves_per_eu(attn_waves_min<BM * 2 * NKH, WPE>(), attn_waves_max<WPE>())))
 sparse_attn_kernel(AttnArgs a) {
-  using C = AttnCfg<INT8, D, BM, BN, STAGES, BNS, NKH, WPE>;
+  using C = AttnCfg<INT8, D, BM, BN, BNS, NKH, WPE>;
   typedef typename std::conditional<INT8, v4i, v8bf>::type OpT;
-  // A 3-slot ring issues its copies between the PV MFMAs, every wavefront
-  // the same kOps copies per ring step (validity bytes included)
-  constexpr bool kDmaInPv = STAGES == 3;
+  // The ring issues its copies between the PV MFMAs, every wavefront the
+  // same kOps copies per ring step (validity bytes included)
+  constexpr int STAGES = C::STAGES;
   // Rings of several steps per key block run whole rounds of STAGES steps (up
   // to STAGES - 1 masked steps past the list, a fraction of a block); a ring of
   // one step per block stops at the list's end, and so do the gathered rings
   // (their scalar registers spill more with the padded loop, 56 -> 71 SGPRs in
   // the int8 kernel).
-  constexpr bool kPadRounds = kDmaInPv && BN / BNS > 1 && !GATHER;
+  constexpr bool kPadRounds = BN / BNS > 1 && !GATHER;
   // validity bytes ride along with the copies unless the caller passes the
   // validity bits (MASK: read with scalar loads instead)
-  constexpr bool kValidCopy = kDmaInPv && !MASK;
+  constexpr bool kValidCopy = !MASK;
   constexpr int kOps = C::DMA + (kValidCopy ? 1 : 0);
   // GATHER: every ring step also reads, one step ahead, the slot-map entries
   // of the VUPW V rows (bf16: and the same K rows) its lane copies
   constexpr int kTok = GATHER ? C::VUPW : 0;
-  static_assert(!GATHER || (kDmaInPv && MASK), "gathered sources ride the 3-slot ring with bits");
+  static_assert(!GATHER || MASK, "gathered sources ride the ring with bits");
   static_assert(!GATHER || INT8 || (C::KUPW == C::VUPW && C::K_RPU == C::V_RPU &&
                                     C::CPR_K == C::CPR_V), "bf16 K and V rows share tokens");
   typedef typename std::conditional<INT8, v16i, v16f>::type AccT;
@@ -265,7 +265,7 @@ sparse_attn_kernel(AttnArgs a) {
   // flight into the other slots (it would otherwise drain them first).
   __shared__ __attribute__((aligned(1024))) char s_0[C::SLOT];
   __shared__ __attribute__((aligned(1024))) char s_1[C::SLOT];
-  __shared__ __attribute__((aligned(1024))) char s_2[STAGES > 2 ? C::SLOT : 16];
+  __shared__ __attribute__((aligned(1024))) char s_2[C::SLOT];
   __shared__ __attribute__((aligned(16)))
   char s_m[NKH == 1 || C::MERGE_IN_SLOTS ? 16 : C::NRG * C::MW * 4];
 
@@ -325,9 +325,7 @@ sparse_attn_kernel(AttnArgs a) {
   }
   // Q must be resident before the ring starts: otherwise its pending loads
   // meet the loop's back edge and the compiler drains at the first MFMA.
-  // A 3-slot ring waits for them after issuing its two prologue stages
-  // (counted below); the other rings wait here.
-  if constexpr (!kDmaInPv) __builtin_amdgcn_s_waitcnt(vmcnt_imm(0));
+  // They are waited for after the two prologue stages are issued (below).
 
   v16f o_acc[C::NDT];
 #pragma unroll
@@ -373,15 +371,13 @@ sparse_attn_kernel(AttnArgs a) {
 #pragma unroll
   for (int i = 0; i < C::VUPW; ++i)
     v_lo[i] = (GATHER ? 0u : static_cast<uint32_t>(v_row(i) * vrow_bytes)) + v_col(i);
-  // Copy step n (BNS keys from key n*BNS; clamped to 0 when invalid) into a
-  // slot.  Rows past k_len re-read the last row (those keys are masked).
+  // Copy step n (BNS keys from key n*BNS) into a slot.
   // (Named source pointers: an inline pointer expression as this builtin's
   // source argument makes the host pass drop the kernel stub.)
-  // Branch-free variant for the 3-slot ring: the copies of a step go through
-  // buffer resources that end at the step's last valid row, so each lane
-  // keeps its loop-invariant offset and rows past K_LEN land as zeros (those
-  // keys are masked); the copies then sit in the caller's basic block
-  // between its MFMAs.
+  // Branch-free: the copies of a step go through buffer resources that end at
+  // the step's last valid row, so each lane keeps its loop-invariant offset
+  // and rows past K_LEN land as zeros (those keys are masked); the copies then
+  // sit in the caller's basic block between its MFMAs.
   const uint32_t krb = static_cast<uint32_t>(krow_bytes), vrb = static_cast<uint32_t>(vrow_bytes);
   // Gathered rows: lane l of copy i moves a chunk of slot v_row(i) =
   // v_row(0) + i V_RPU of the step, read from the slot map through a buffer
@@ -459,37 +455,14 @@ sparse_attn_kernel(AttnArgs a) {
   // next 16-byte boundary; bytes of keys past K_LEN are masked anyway)
   auto stage_valid_flat = [&](int n, char* dst) __attribute__((always_inline)) {
     static_assert(BNS <= 128, "validity bytes of a step: 32 lanes x 4");
-    const int key0 = (n < 0 ? 0 : n) * BNS;  // a listed block starts below K_LEN
+    const int key0 = (n < 0 ? 0 : n) * BNS;
     const bool has = a.kvalid != nullptr;
     char* const vb = has ? reinterpret_cast<char*>(const_cast<uint8_t*>(a.kvalid)) + key0
                          : reinterpret_cast<char*>(kAllValid);
-    const int left = n < 0 ? 0 : (has ? klen - key0 : BNS);
+    // (a block's later steps may begin past K_LEN: nothing is read for them)
+    const int left = n < 0 ? 0 : (has ? (klen > key0 ? klen - key0 : 0) : BNS);
     const int vnum = ((left + 3) & ~3) < BNS ? ((left + 3) & ~3) : BNS;
     buffer_copy4(vb, vnum, 4u * (lane & 31), dst + C::BUF);
-  };
-  auto stage = [&](int n, char* dst) __attribute__((always_inline)) {
-    const int64_t key0 = static_cast<int64_t>(n < 0 ? 0 : n) * BNS;
-    const bool tail = key0 + BNS > a.k_len;
-    const char* kb0 = kbase + key0 * krow_bytes;
-    const char* vb0 = vbase + key0 * vrow_bytes;
-#pragma unroll
-    for (int i = 0; i < C::KUPW; ++i) {
-      if (C::KUNITS % C::NW == 0 || wave * C::KUPW + i < C::KUNITS) {  // uniform per wavefront
-        const char* src = tail ? kbase + min(key0 + k_row(i), int64_t{klast}) * krow_bytes + k_col(i)
-                               : kb0 + k_lo[i];
-        __builtin_amdgcn_global_load_lds(
-            src, RCSA_LDS(void, dst + (wave * C::KUPW + i) * 1024), 16, 0, 0);
-      }
-    }
-#pragma unroll
-    for (int i = 0; i < C::VUPW; ++i) {
-      if (C::VUNITS % C::NW == 0 || wave * C::VUPW + i < C::VUNITS) {
-        const char* src = tail ? vbase + min(key0 + v_row(i), int64_t{klast}) * vrow_bytes + v_col(i)
-                               : vb0 + v_lo[i];
-        __builtin_amdgcn_global_load_lds(
-            src, RCSA_LDS(void, dst + C::KBYTES + (wave * C::VUPW + i) * 1024), 16, 0, 0);
-      }
-    }
   };
   // Ring step `it`: step SUB*n + it%SUB of list entry n = list[it / SUB]
   // (-1 = invalid entry), a scalar load.
@@ -504,17 +477,6 @@ sparse_attn_kernel(AttnArgs a) {
     return INT8 ? ld_const(a.k_scale + bh * a.k_scale_stride + (n < 0 ? 0 : n / C::SUB))
                 : 1.0f;
   };
-  // The BNS validity bytes of a step ride along with its copies (BNS/16
-  // lanes of wavefront 0, 16 bytes each) into the slot's 256-byte tail;
-  // K_valid is 16-byte aligned and readable up to the next 16-byte boundary.
-  auto stage_valid = [&](int n, char* dst) __attribute__((always_inline)) {
-    if (a.kvalid != nullptr && wave == 0 && lane < BNS / 16) {
-      const int64_t key0 = static_cast<int64_t>(n < 0 ? 0 : n) * BNS;
-      const int64_t chunk = min(key0 + 16 * lane, (klast / 16) * 16);
-      const char* src = reinterpret_cast<const char*>(a.kvalid) + chunk;
-      __builtin_amdgcn_global_load_lds(src, RCSA_LDS(void, dst + C::BUF), 16, 0, 0);
-    }
-  };
   // validity of the wavefront's HK keys of step n from the caller's bits
   // (uniform scalar loads; keys past K_LEN are cleared)
   // (split in two: the raw words, loaded ahead, and the mask of step n)
@@ -522,8 +484,9 @@ sparse_attn_kernel(AttnArgs a) {
     const uint32_t* w = a.kmask + ((n < 0 ? 0 : n) * BNS + kh * C::HK) / 32;
     return make_uint2(ld_const(w), C::HK == 64 ? ld_const(w + 1) : 0u);
   };
-  // Only the step holding K_LEN can have keys past it: its keep mask for this
-  // wavefront's half is computed once.
+  // The step holding K_LEN has its keep mask for this wavefront's half computed
+  // once; a last block's steps past it (and -1) keep nothing.
+  const uint32_t last_step = static_cast<uint32_t>(klast) / BNS;
   const int tail_step = klen % BNS != 0 ? klen / BNS : -1;
   const uint64_t tail_keep = [&]() -> uint64_t {
     const int left = klen - (klen / BNS * BNS + kh * C::HK);
@@ -531,15 +494,10 @@ sparse_attn_kernel(AttnArgs a) {
   }();
   auto mask_of = [&](int n, uint2 words) __attribute__((always_inline)) -> uint64_t {
     const uint64_t m = words.x | (static_cast<uint64_t>(words.y) << 32);
-    return n < 0 ? 0ull : (n == tail_step ? m & tail_keep : m);
+    return static_cast<uint32_t>(n) > last_step ? 0ull : (n == tail_step ? m & tail_keep : m);
   };
-  auto mask_bits = [&](int n) __attribute__((always_inline)) -> uint64_t {
-    return mask_of(n, mask_words(n));
-  };
-  // Validity bits come from the caller when MASK is set; the 3-slot ring is
-  // launched with MASK whenever the caller passes bits, so without MASK it
-  // always takes the bytes (and drops the bit path at compile time).
-  const bool use_bits = MASK || (!kDmaInPv && a.kmask != nullptr);
+  // MASK: the caller's validity bits; otherwise the staged validity bytes
+  constexpr bool use_bits = MASK;
   // validity of this lane's key in the wavefront's half, from the slot tail
   auto key_valid = [&](int n, const char* tile) __attribute__((always_inline)) -> bool {
     const int key = n * BNS + kh * C::HK + lane;
@@ -686,10 +644,8 @@ sparse_attn_kernel(AttnArgs a) {
       }
     }
     l_run += part;
-    if constexpr (kDmaInPv) {
-      if constexpr (kValidCopy) stage_valid_flat(n_fill, fill);
-      stage_flat(n_fill, fill, fill_tok);
-    }
+    if constexpr (kValidCopy) stage_valid_flat(n_fill, fill);
+    stage_flat(n_fill, fill, fill_tok);
     // ---- O^T += V^T P^T, V^T operand by transposing LDS reads; the reads of
     //      the next 16-key step are in flight during this step's MFMAs ----
     auto v_group = [&](int g, v8bf (&op)[C::NDT]) __attribute__((always_inline)) {
@@ -720,7 +676,7 @@ sparse_attn_kernel(AttnArgs a) {
       for (int dt = 0; dt < C::NDT; ++dt) {
         __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
         if (g + 1 < 2 * C::KT) __builtin_amdgcn_sched_group_barrier(0x100, 2, 0);
-        if (kDmaInPv && g * C::NDT + dt < kOps)
+        if (g * C::NDT + dt < kOps)
           __builtin_amdgcn_sched_group_barrier(0x010, 1, 0);
       }
   };
@@ -734,59 +690,45 @@ sparse_attn_kernel(AttnArgs a) {
   // slot-map entries of the step that fills each slot (GATHER)
   uint32_t tk_m[3][kTokArr] = {};
   int n_pre = -1;  // next step to stage
-  if constexpr (kDmaInPv) {
-    // both prologue steps always copy (step 0 stands in past the list), so
-    // every wavefront has exactly 2 * kOps copies in flight
+  // both prologue steps always copy (step 0 stands in past the list), so
+  // every wavefront has exactly 2 * kOps copies in flight
 #pragma unroll
-    for (int sidx = 0; sidx < STAGES - 1; ++sidx) {
-      n_m[sidx] = sidx < steps ? block_of(sidx) : -1;
-      ks_m[sidx] = fetch_scale(n_m[sidx]);
-    }
-    if constexpr (GATHER) n_pre = STAGES - 1 < steps ? block_of(STAGES - 1) : -1;
-    // gathered: the map reads of the two prologue steps, then their copies,
-    // then the map read of step 2.  The first ring wait counts the copies of
-    // one step plus one step's map reads as the younger operations, so the
-    // map read of step 2 must come after the copies of step 0: the scheduling
-    // fence keeps the compiler from hoisting it (loads issue in order).
-    load_tokens(n_m[0], tk_m[0]);
-    load_tokens(n_m[1], tk_m[1]);
-#pragma unroll
-    for (int sidx = 0; sidx < STAGES - 1; ++sidx) {
-      char* const dst = sidx == 0 ? s_0 : sidx == 1 ? s_1 : s_2;
-      if constexpr (kValidCopy) stage_valid_flat(n_m[sidx], dst);
-      stage_flat(n_m[sidx], dst, tk_m[sidx]);
-      // the copies of step 0 stay older than those of step 1 (the first
-      // ring wait leaves one step's copies in flight)
-      __builtin_amdgcn_sched_barrier(0);
-    }
-    if constexpr (GATHER) {
-      __builtin_amdgcn_sched_barrier(0);
-      load_tokens(n_pre, tk_m[2]);
-      __builtin_amdgcn_sched_barrier(0);
-    }
-    if (use_bits) mk_m[0] = mask_words(n_m[0]);
-    if constexpr (!GATHER) n_pre = STAGES - 1 < steps ? block_of(STAGES - 1) : -1;
-    // the Q loads (and the first two map reads) precede these 2 kOps copies
-    // (and the third map read): with at most that many outstanding, Q has
-    // landed and both prologue stages stay in flight
-    __builtin_amdgcn_s_waitcnt(vmcnt_imm(2 * kOps + kTok));
-  } else {
-#pragma unroll
-    for (int sidx = 0; sidx < STAGES - 1; ++sidx) {
-      if (sidx < steps) {
-        char* const dst = sidx == 0 ? s_0 : sidx == 1 ? s_1 : s_2;
-        n_m[sidx] = block_of(sidx);
-        ks_m[sidx] = fetch_scale(n_m[sidx]);
-        stage_valid(n_m[sidx], dst);
-        stage(n_m[sidx], dst);
-      }
-    }
-    n_pre = STAGES - 1 < steps ? block_of(STAGES - 1) : -1;
+  for (int sidx = 0; sidx < STAGES - 1; ++sidx) {
+    n_m[sidx] = sidx < steps ? block_of(sidx) : -1;
+    ks_m[sidx] = fetch_scale(n_m[sidx]);
   }
-  // 3-slot ring: the list entry of the step after n_pre, as loaded
+  if constexpr (GATHER) n_pre = STAGES - 1 < steps ? block_of(STAGES - 1) : -1;
+  // gathered: the map reads of the two prologue steps, then their copies,
+  // then the map read of step 2.  The first ring wait counts the copies of
+  // one step plus one step's map reads as the younger operations, so the
+  // map read of step 2 must come after the copies of step 0: the scheduling
+  // fence keeps the compiler from hoisting it (loads issue in order).
+  load_tokens(n_m[0], tk_m[0]);
+  load_tokens(n_m[1], tk_m[1]);
+#pragma unroll
+  for (int sidx = 0; sidx < STAGES - 1; ++sidx) {
+    char* const dst = sidx == 0 ? s_0 : sidx == 1 ? s_1 : s_2;
+    if constexpr (kValidCopy) stage_valid_flat(n_m[sidx], dst);
+    stage_flat(n_m[sidx], dst, tk_m[sidx]);
+    // the copies of step 0 stay older than those of step 1 (the first
+    // ring wait leaves one step's copies in flight)
+    __builtin_amdgcn_sched_barrier(0);
+  }
+  if constexpr (GATHER) {
+    __builtin_amdgcn_sched_barrier(0);
+    load_tokens(n_pre, tk_m[2]);
+    __builtin_amdgcn_sched_barrier(0);
+  }
+  if (use_bits) mk_m[0] = mask_words(n_m[0]);
+  if constexpr (!GATHER) n_pre = STAGES - 1 < steps ? block_of(STAGES - 1) : -1;
+  // the Q loads (and the first two map reads) precede these 2 kOps copies
+  // (and the third map read): with at most that many outstanding, Q has
+  // landed and both prologue stages stay in flight
+  __builtin_amdgcn_s_waitcnt(vmcnt_imm(2 * kOps + kTok));
+  // the list entry of the step after n_pre, as loaded
   // (read only when the list is not empty: an empty list may have no entries)
   int32_t pre_raw =
-      (kDmaInPv && steps > 0) ? ld_const(list + (STAGES < steps ? STAGES : 0) / C::SUB) : -1;
+      steps > 0 ? ld_const(list + (STAGES < steps ? STAGES : 0) / C::SUB) : -1;
   auto iteration = [&](auto slot_c, int j) __attribute__((always_inline)) {
     constexpr int J = decltype(slot_c)::value;
     constexpr int F = (J + STAGES - 1) % STAGES;  // slot of block j + STAGES - 1
@@ -798,47 +740,28 @@ sparse_attn_kernel(AttnArgs a) {
     // block j's copies are the oldest in flight; the STAGES-2 younger
     // stages may remain (wavefront 0's extra validity copy is waited too),
     // then every wavefront's copies of block j have landed and slot F is free
-    if constexpr (kDmaInPv) {
-      wait_vm_barrier<kOps + kTok>();  // every step issues kOps copies (+ kTok map reads)
-    } else if constexpr (STAGES == 3) {
-      if (j + 1 < steps) wait_vm_barrier<C::DMA>();
-      else wait_vm_barrier<0>();
-    } else {
-      wait_vm_barrier<0>();
-    }
-    if constexpr (kDmaInPv) {
-      // every iteration copies (a step past the list re-copies step 0 into
-      // the slot it fills, which nobody reads), so every wait counts the
-      // same copies; the K/V copies issue between the PV MFMAs
-      // Scalar loads for later blocks go out after this block's QK MFMAs:
-      // the scale of block j+2, the list entry of block j+3 and the
-      // validity bits of block j+1.
-      // Loaded values are only stored here (their first use is a later
-      // block's), so no wait lands before this block's softmax.
-      constexpr int N1 = (J + 1) % STAGES;  // slot of block j + 1
-      const int nf = n_pre;
-      n_m[F] = nf;
-      n_pre = j + STAGES < steps ? block_step(pre_raw, j + STAGES) : -1;
-      const int nxt = j + STAGES + 1 < steps ? j + STAGES + 1 : 0;  // in-bounds entry
-      compute(tile, n_m[J], ks_m[J], use_bits ? mask_of(n_m[J], mk_m[J]) : 0ull, nf, fill,
-              tk_m[F], [&]() __attribute__((always_inline)) {
-                ks_m[F] = fetch_scale(nf);
-                pre_raw = ld_const(list + nxt / C::SUB);
-                if (use_bits) mk_m[N1] = mask_words(n_m[N1]);
-                // map entries of block j + 3, which will fill this block's slot
-                load_tokens(n_pre, tk_m[J]);
-              });
-    } else {
-      if (j + STAGES - 1 < steps) {
-        n_m[F] = n_pre;
-        ks_m[F] = fetch_scale(n_pre);
-        stage_valid(n_pre, fill);
-        stage(n_pre, fill);
-        n_pre = j + STAGES < steps ? block_of(j + STAGES) : -1;
-      }
-      compute(tile, n_m[J], ks_m[J], use_bits ? mask_bits(n_m[J]) : 0ull, -1, fill, tk_m[F],
-              []() __attribute__((always_inline)) {});
-    }
+    wait_vm_barrier<kOps + kTok>();  // every step issues kOps copies (+ kTok map reads)
+    // every iteration copies (a step past the list re-copies step 0 into
+    // the slot it fills, which nobody reads), so every wait counts the
+    // same copies; the K/V copies issue between the PV MFMAs
+    // Scalar loads for later blocks go out after this block's QK MFMAs:
+    // the scale of block j+2, the list entry of block j+3 and the
+    // validity bits of block j+1.
+    // Loaded values are only stored here (their first use is a later
+    // block's), so no wait lands before this block's softmax.
+    constexpr int N1 = (J + 1) % STAGES;  // slot of block j + 1
+    const int nf = n_pre;
+    n_m[F] = nf;
+    n_pre = j + STAGES < steps ? block_step(pre_raw, j + STAGES) : -1;
+    const int nxt = j + STAGES + 1 < steps ? j + STAGES + 1 : 0;  // in-bounds entry
+    compute(tile, n_m[J], ks_m[J], use_bits ? mask_of(n_m[J], mk_m[J]) : 0ull, nf, fill,
+            tk_m[F], [&]() __attribute__((always_inline)) {
+              ks_m[F] = fetch_scale(nf);
+              pre_raw = ld_const(list + nxt / C::SUB);
+              if (use_bits) mk_m[N1] = mask_words(n_m[N1]);
+              // map entries of block j + 3, which will fill this block's slot
+              load_tokens(n_pre, tk_m[J]);
+            });
   };
   if constexpr (kPadRounds) {
     // Whole rounds of STAGES steps, no exit between them: a step past the list
@@ -860,15 +783,13 @@ sparse_attn_kernel(AttnArgs a) {
       iteration(std::integral_constant<int, 0>{}, j);
       if (j + 1 >= steps) break;
       iteration(std::integral_constant<int, 1>{}, j + 1);
-      if constexpr (STAGES > 2) {
-        if (j + 2 >= steps) break;
-        iteration(std::integral_constant<int, 2>{}, j + 2);
-      }
+      if (j + 2 >= steps) break;
+      iteration(std::integral_constant<int, 2>{}, j + 2);
     }
   }
 
   // the trailing copies (past the list) land before the slots are reused or freed
-  if constexpr (kDmaInPv) __builtin_amdgcn_s_waitcnt(vmcnt_imm(0));
+  __builtin_amdgcn_s_waitcnt(vmcnt_imm(0));
 
   // ---- merge the key halves, normalise, write O (bf16) and the LSE ----
   const float l_tot = pair_sum(l_run);
@@ -999,6 +920,10 @@ int launch_bf16_gather(AttnArgs& a, dim3 grid, hipStream_t s);
 // validity bytes.
 int launch_int8_cu3(AttnArgs& a, dim3 grid, bool gather, bool bits, hipStream_t s);
 int launch_bf16_cu3(AttnArgs& a, dim3 grid, bool gather, hipStream_t s);
+// The block shapes other than D 128 with 128 x 128 blocks (sparse_attn_shapes.hip);
+// many: at least two rounds of query blocks per XCD.
+int launch_attn_shape(AttnArgs& a, bool int8, int64_t D, int64_t BM, int64_t BN, bool many,
+                      dim3 grid, hipStream_t s);
 
 }  // namespace rcsa
 

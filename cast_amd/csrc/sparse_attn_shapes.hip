@@ -1,0 +1,69 @@
+// The attention kernel of sparse_attn_kernel.h for the block shapes other
+// than D 128 with 128 x 128 blocks: head_dim 64 or 64-row / 64-key blocks.
+//
+// Two forms per shape, chosen as for the main shape by the query blocks of an
+// XCD.  With at least two rounds of them, small workgroups of one key half
+// share a compute unit (MANY): each waits for its own copies only, so the
+// others' MFMAs cover the wait.  Below that, workgroups of two key halves and
+// longer ring steps (FEW) walk a list in half as many steps.  us, MANY / FEW /
+// the one 2-slot workgroup per compute unit they replace, 24 heads, 80 x 128
+// keys a row, validity bits:
+//                                1792 query rows       256 query rows
+//   bf16 D 128, 64 x 128         360 / 406 / 608       84 /  85 / 122
+//   bf16 D 128, 64 x 64          349 / 433 / 593       80 /  93 / 113
+//   bf16 D 64, 64 x 64           215 / 203 / 263       54 /  45 /  53
+//   int8 D 128, 64 x 128         298 / 355 / 522       64 /  75 / 102
+//   int8 D 64, 64 x 64           202 / 214 / 261       51 /  47 /  53
+// and at 8 heads x 1024 rows x 32 of 64 key blocks, int8 D 128, 64 x 128:
+// 51 / 41 / 48.  (bf16 D 64 keeps FEW throughout: within 5% at 3584 rows.)
+// Validity bytes are read by callers of the C ABI without bits only: FEW.
+#include "sparse_attn_kernel.h"
+
+namespace rcsa {
+
+template <bool INT8, int D, int BM, int BN, int BNS, int NKH, int WPE>
+static int launch_form(AttnArgs& a, dim3 grid, hipStream_t s) {
+  constexpr int kThreads = BM / 32 * NKH * 64;
+  if (a.kmask != nullptr)
+    sparse_attn_kernel<INT8, D, BM, BN, BNS, NKH, true, false, WPE>
+        <<<grid, dim3(kThreads), 0, s>>>(a);
+  else
+    sparse_attn_kernel<INT8, D, BM, BN, BNS, NKH, false, false, WPE>
+        <<<grid, dim3(kThreads), 0, s>>>(a);
+  return launch_status();
+}
+
+template <bool INT8, int D, int BM, int BN, int BNS, int WPE>
+static int launch_many(AttnArgs& a, dim3 grid, hipStream_t s) {
+  sparse_attn_kernel<INT8, D, BM, BN, BNS, 1, true, false, WPE>
+      <<<grid, dim3(BM / 32 * 64), 0, s>>>(a);
+  return launch_status();
+}
+
+int launch_attn_shape(AttnArgs& a, bool int8, int64_t D, int64_t BM, int64_t BN, bool many,
+                      dim3 grid, hipStream_t s) {
+  many = many && a.kmask != nullptr;
+#define RCSA_SHAPE(D_, BM_, BN_) if (D == D_ && BM == BM_ && BN == BN_)
+  if (int8) {
+    RCSA_SHAPE(128, 128, 64) return many ? launch_many<true, 128, 128, 64, 32, 3>(a, grid, s) : launch_form<true, 128, 128, 64, 64, 2, 0>(a, grid, s);
+    RCSA_SHAPE(128, 64, 128) return many ? launch_many<true, 128, 64, 128, 32, 2>(a, grid, s) : launch_form<true, 128, 64, 128, 64, 2, 0>(a, grid, s);
+    RCSA_SHAPE(128, 64, 64) return many ? launch_many<true, 128, 64, 64, 32, 2>(a, grid, s) : launch_form<true, 128, 64, 64, 64, 2, 0>(a, grid, s);
+    RCSA_SHAPE(64, 128, 128) return many ? launch_many<true, 64, 128, 128, 64, 3>(a, grid, s) : launch_form<true, 64, 128, 128, 128, 2, 0>(a, grid, s);
+    // (a 64-key step has too few K copies for the eight wavefronts of two halves)
+    RCSA_SHAPE(64, 128, 64) return launch_form<true, 64, 128, 64, 64, 1, 3>(a, grid, s);
+    RCSA_SHAPE(64, 64, 128) return many ? launch_many<true, 64, 64, 128, 32, 3>(a, grid, s) : launch_form<true, 64, 64, 128, 64, 2, 0>(a, grid, s);
+    RCSA_SHAPE(64, 64, 64) return many ? launch_many<true, 64, 64, 64, 32, 3>(a, grid, s) : launch_form<true, 64, 64, 64, 64, 2, 0>(a, grid, s);
+  } else {
+    RCSA_SHAPE(128, 128, 64) return many ? launch_many<false, 128, 128, 64, 32, 3>(a, grid, s) : launch_form<false, 128, 128, 64, 64, 2, 0>(a, grid, s);
+    RCSA_SHAPE(128, 64, 128) return many ? launch_many<false, 128, 64, 128, 32, 2>(a, grid, s) : launch_form<false, 128, 64, 128, 64, 2, 0>(a, grid, s);
+    RCSA_SHAPE(128, 64, 64) return many ? launch_many<false, 128, 64, 64, 32, 2>(a, grid, s) : launch_form<false, 128, 64, 64, 64, 2, 0>(a, grid, s);
+    RCSA_SHAPE(64, 128, 128) return launch_form<false, 64, 128, 128, 64, 2, 0>(a, grid, s);
+    RCSA_SHAPE(64, 128, 64) return launch_form<false, 64, 128, 64, 64, 2, 0>(a, grid, s);
+    RCSA_SHAPE(64, 64, 128) return launch_form<false, 64, 64, 128, 64, 2, 0>(a, grid, s);
+    RCSA_SHAPE(64, 64, 64) return launch_form<false, 64, 64, 64, 64, 2, 0>(a, grid, s);
+  }
+#undef RCSA_SHAPE
+  return RCSA_ERR_SHAPE;
+}
+
+}  // namespace rcsa

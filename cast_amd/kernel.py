@@ -66,5 +66,10 @@ def longcat_asymmetric(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor,
     valid = key_valid.reshape(-1).to(torch.uint8).contiguous()
     if q.shape[2] % query_block_size or k.shape[2] % key_block_size:
         raise RuntimeError("asymmetric sparse storage is not block aligned")
+    if key_block_size % 32 == 0 and valid.numel() == k.shape[2] and valid.is_cuda:
+        indices, counts, bits, ordered = _lists_and_bits(k, indices, counts, valid,
+                                                         key_block_size)
+        return ops.sparse_attn_bf16(q, k, v, indices, counts, None, block_m=query_block_size,
+                                    block_n=key_block_size, block_mask=bits, ordered=ordered)
     return ops.sparse_attn_bf16(q, k, v, indices, counts, valid, block_m=query_block_size,
                                 block_n=key_block_size)
