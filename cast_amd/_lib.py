@@ -64,6 +64,7 @@ SIGNATURES: dict[str, list] = {
                               c_float, _P],
     "rcsa_route_check": [_P, _P, _P, _P, _I, _I, _I, _I, _P, _P],
     "rcsa_quantize_rows_int8": [_P, c_int, _I, _I, _I, _P, _P, _P],
+    "rcsa_int8_linear_group": [_P, _P, _I, _P, _P, _P, _P, _P, _P, c_int, _I, _I, _P],
     "rcsa_int8_linear": [_P, _P, _P, _P, _P, _I, _I, _I, _P, _I, _P],
     "rcsa_order_lists_max_blocks": [],
     "rcsa_order_lists": [_P, _P] + [_I] * 6 + [_P] + [_I] * 6 + [_P, _P, _P, _I, _P, _P],

@@ -5,24 +5,23 @@
 // an all-zero row), q = rne(x * 127 / absmax) clamped to [-127, 127].
 //
 // int8_linear_kernel: out[m][n] = bf16(bf16(acc * xs[m] * ws[n]) + bias[n]),
-// acc = sum_k x[m][k] w[n][k] in int32.  A workgroup (8 wavefronts, one per CU)
-// computes a 256 (tokens) x 256 (channels) tile; each wavefront 64 x 128 as
-// 2 x 4 tiles of v_mfma_i32_32x32x32_i8 with the weights as the A operand, so a
-// lane ends up holding one token and runs of 4 consecutive channels; lanes l and
-// l + 32 swap halves (v_permlane32_swap) so that each stores 8 consecutive
-// channels (16 bytes).  Both operands are staged by direct-to-LDS copies through
-// a 2-slot ring of 128-byte K steps (64 KiB per slot), so every row a copy reads
-// is one whole 128-byte line (half as many L2 requests as 64-byte steps);
-// 16-byte chunks of each 128-byte row are XORed by (row / 2) mod 8 so the
-// ds_read_b128 operand reads are conflict free.  When the 256 x 256 tiles would
-// end in a short round, the rows of that round run as 128 x 128 tiles (each
-// wavefront 32 x 64) of the same launch, taken first.  The launch is
-// persistent: one workgroup per compute unit walks its XCD's tiles, and the
-// copy ring runs on from one 256 x 256 tile to the next, so a tile's first
-// copies fly during the previous tile's epilogue (at 38,720 x 3072 x 3072:
-// 0.396-0.407 against 0.415-0.421 ms with one workgroup per tile, interleaved
-// on one box; holding half of each output tile in registers to store it
-// beside the next tile's first MFMAs gained nothing more).
+// acc = sum_k x[m][k] w[n][k] in int32, for up to four projections of one x.  A
+// workgroup of four wavefronts, one per SIMD, computes a tile of 256 (tokens) x
+// 256 (channels) or 128 x 128 with v_mfma_i32_32x32x32_i8, the weights as the A
+// operand, so a lane ends up holding one token and runs of 4 consecutive
+// channels.  A wavefront's quarter of 128 x 128 reads 8 operand tiles from LDS
+// for 16 MFMAs: half the matrix cores' time at 128 bytes a clock (64 x 128
+// quarters of eight wavefronts take three quarters of it and run at 42% of the
+// matrix cores' cycles).  Both operands are staged by direct-to-LDS copies
+// through a ring of 128-byte K steps (one whole line of every row); 16-byte
+// chunks of each 128-byte row are XORed by (row / 2) mod 8 so the ds_read_b128
+// operand reads are conflict free.  The launch is persistent: one workgroup per
+// compute unit walks its XCD's tiles of all projections, and the ring runs on
+// from one tile to the next.  Three projections of 3072 x 3072, one launch,
+// against three launches of the eight-wavefront kernel: 38,720 tokens 1034
+// against 1199 us (2.1 POP/s), 3520 tokens 92 against 155, 880 tokens (128 x 128
+// tiles) 32 against 144 us.  What bounds it: the matrix cores' clock under load
+// (1.9 GHz) and the epilogue, which no MFMA of the same SIMD covers.
 #include <type_traits>
 
 #include "rcsa_common.h"
@@ -32,56 +31,99 @@
 namespace rcsa {
 
 constexpr int kQThreads = 256;       // quantiser: 4 rows per workgroup
-constexpr int kGemmThreads = 512;    // 8 wavefronts: 4 (tokens) x 2 (channels)
+constexpr int kGemmWaves = 4;        // 2 (tokens) x 2 (channels), one per SIMD
+constexpr int kGemmThreads = kGemmWaves * kWave;
 constexpr int kKS = 128;             // bytes of K per ring step (one 128-byte line per row)
 
-template <typename T>
-__device__ __forceinline__ float to_f32(T v) {
-  if constexpr (std::is_same<T, float>::value) return v;
-  else return bf16_to_f32(v);
+typedef unsigned int v4u __attribute__((ext_vector_type(4)));
+
+// Two floats as packed bf16 (round to nearest even), low half = a.
+__device__ __forceinline__ uint32_t cvt_bf16x2(float a, float b) {
+  typedef __bf16 v2bf __attribute__((ext_vector_type(2)));
+  const v2bf v = {static_cast<__bf16>(a), static_cast<__bf16>(b)};
+  return __builtin_bit_cast(uint32_t, v);
 }
 
-template <typename T>
+// Eight floats as int8 (two words).
+__device__ __forceinline__ uint2 quant8(const float (&v)[8], float inv) {
+  uint32_t lo = 0, hi = 0;
+#pragma unroll
+  for (int j = 0; j < 4; ++j) {
+    lo |= (static_cast<uint32_t>(quant_i8(v[j], inv)) & 0xffu) << (8 * j);
+    hi |= (static_cast<uint32_t>(quant_i8(v[j + 4], inv)) & 0xffu) << (8 * j);
+  }
+  return make_uint2(lo, hi);
+}
+
+// NC > 0: rows of at most NC 512-channel chunks stay in registers between the
+// two passes (all loads in flight at once, one read of x); NC == 0: any length,
+// read twice.  HBM-bound: 38,720 x 3072 bf16 takes 69 us (5.2 TB/s), read twice
+// 86 us.
+template <typename T, int NC>
 __global__ void __launch_bounds__(kQThreads)
 quant_rows_kernel(const T* x, int64_t M, int64_t C, int64_t ldx, int8_t* q, float* scale) {
   const int lane = threadIdx.x % kWave;
   const int64_t row = static_cast<int64_t>(blockIdx.x) * (kQThreads / kWave) + threadIdx.x / kWave;
   if (row >= M) return;
   const T* xr = x + row * ldx;
-  float amax = 0.0f;
-  for (int64_t c = lane * 8; c < C; c += kWave * 8) {
-    float v[8];
-    Vec8<T>::load(xr + c, v);
-#pragma unroll
-    for (int j = 0; j < 8; ++j) amax = fmaxf(amax, fabsf(v[j]));
-  }
-  amax = wave_max(amax);
-  const float inv = amax > 0.0f ? 127.0f / amax : 1.0f;
-  if (lane == 0) scale[row] = amax > 0.0f ? amax / 127.0f : 1.0f;
   int8_t* qr = q + row * C;
-  for (int64_t c = lane * 8; c < C; c += kWave * 8) {
-    float v[8];
-    Vec8<T>::load(xr + c, v);
-    uint32_t lo = 0, hi = 0;
+  float amax = 0.0f;
+  if constexpr (NC > 0) {
+    float v[NC][8];
 #pragma unroll
-    for (int j = 0; j < 4; ++j) {
-      lo |= (static_cast<uint32_t>(quant_i8(v[j], inv)) & 0xffu) << (8 * j);
-      hi |= (static_cast<uint32_t>(quant_i8(v[j + 4], inv)) & 0xffu) << (8 * j);
+    for (int i = 0; i < NC; ++i) {
+      const int64_t c = (i * kWave + lane) * 8;
+      if (c < C) {
+        Vec8<T>::load(xr + c, v[i]);
+      } else {
+#pragma unroll
+        for (int j = 0; j < 8; ++j) v[i][j] = 0.0f;
+      }
     }
-    *reinterpret_cast<uint2*>(qr + c) = make_uint2(lo, hi);
+#pragma unroll
+    for (int i = 0; i < NC; ++i)
+#pragma unroll
+      for (int j = 0; j < 8; ++j) amax = fmaxf(amax, fabsf(v[i][j]));
+    amax = wave_max(amax);
+    const float inv = amax > 0.0f ? 127.0f / amax : 1.0f;
+#pragma unroll
+    for (int i = 0; i < NC; ++i) {
+      const int64_t c = (i * kWave + lane) * 8;
+      if (c < C) *reinterpret_cast<uint2*>(qr + c) = quant8(v[i], inv);
+    }
+  } else {
+    for (int64_t c = lane * 8; c < C; c += kWave * 8) {
+      float v[8];
+      Vec8<T>::load(xr + c, v);
+#pragma unroll
+      for (int j = 0; j < 8; ++j) amax = fmaxf(amax, fabsf(v[j]));
+    }
+    amax = wave_max(amax);
+    const float inv = amax > 0.0f ? 127.0f / amax : 1.0f;
+    for (int64_t c = lane * 8; c < C; c += kWave * 8) {
+      float v[8];
+      Vec8<T>::load(xr + c, v);
+      *reinterpret_cast<uint2*>(qr + c) = quant8(v, inv);
+    }
   }
+  if (lane == 0) scale[row] = amax > 0.0f ? amax / 127.0f : 1.0f;
 }
 
+constexpr int kMaxLinear = 4;  // projections of one launch
+
+// The projections of one input: out_g[m][n] for g < n_lin, n < N_g.
 struct LinearArgs {
   const int8_t* x;      // [M, K]
   const float* xs;      // [M]
-  const int8_t* w;      // [N, K]
-  const float* ws;      // [N]
-  const u16* bias;      // [N] bf16 or NULL
-  u16* out;             // [M, ldo] bf16
-  int64_t M, N, K, ldo;
-  // 256 x 256 tiles over rows [0, big_rows), 128 x 128 tiles over [big_rows, M)
-  int64_t big_rows;
+  int64_t M, K;
+  int32_t n_lin;
+  int32_t steps;        // K steps of a tile, padded to the ring's slots with empty ones
+  int64_t tiles[kMaxLinear + 1];  // first tile of each projection; [n_lin]: all tiles
+  const int8_t* w[kMaxLinear];    // [N, K]
+  const float* ws[kMaxLinear];    // [N]
+  const u16* bias[kMaxLinear];    // [N] bf16 or NULL
+  void* out[kMaxLinear];          // [M, ldo], bf16 or the same values as fp32
+  int64_t N[kMaxLinear], ldo[kMaxLinear];
 };
 
 constexpr int kQkvRsrc3 = 0x00020000;  // raw untyped buffer, 32-bit data format
@@ -96,319 +138,350 @@ __device__ __forceinline__ void dma16(const int8_t* base, int bytes, uint32_t vo
 // chunk XOR of a 128-byte row: (row / 2) mod 8
 __device__ __forceinline__ int qkv_swz(int row) { return (row >> 1) & 7; }
 
-// s_waitcnt immediate for vmcnt <= n only (gfx9 encoding)
-constexpr int qkv_vmcnt(int n) {
-  return (n & 0xf) | (0x7 << 4) | (0xf << 8) | (((n >> 4) & 0x3) << 14);
-}
-
+// Wait until at most N copies of this wavefront are outstanding and its LDS
+// reads have returned, then barrier: unlike __syncthreads() the younger copies
+// stay in flight.
 template <int N>
-__device__ __forceinline__ void qkv_wait_barrier() {
+__device__ __forceinline__ void lin_wait_barrier() {
   static_assert(N >= 0 && N < 64, "vmcnt range");
-  asm volatile("s_waitcnt vmcnt(%0)\n\ts_barrier" ::"n"(N) : "memory");
+  __builtin_amdgcn_sched_barrier(0);
+  asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"n"(N) : "memory");
+  __builtin_amdgcn_sched_barrier(0);
 }
 
-// A workgroup tile of 8 wavefronts (4 along tokens x 2 along channels), each
-// TMT x TNT tiles of 32 x 32.
-template <int TMT, int TNT>
+// A workgroup tile of 4 wavefronts (2 along tokens x 2 along channels), each
+// T x T MFMA tiles of 32 x 32, over a ring of SLOTS K steps.
+template <int T_, int SLOTS_>
 struct LinTile {
-  static constexpr int BM = 4 * 32 * TMT, BN = 2 * 32 * TNT;
-  static constexpr int XB = BM * kKS, WB = BN * kKS;          // bytes of a ring step
-  static constexpr int XU = XB / 1024 / 8, WU = WB / 1024 / 8;  // 1 KiB copy units per wavefront
-  static constexpr int OPS = XU + WU;                         // copies per wavefront and step
-  static constexpr int KS = kKS / 32;                         // MFMA k-steps per ring step
-  static_assert(XU == WU && XU >= 1, "both tiles are copied by the same rows");
+  static constexpr int T = T_, SLOTS = SLOTS_;
+  static constexpr int B = 2 * 32 * T;                 // tokens and channels of a tile
+  static constexpr int OB = B * kKS;                   // bytes of one operand's step
+  static constexpr int U = OB / 1024 / kGemmWaves;     // 1 KiB copies per wavefront and operand
+  static constexpr int OPS = 2 * U;                    // copies per wavefront and step
+  static constexpr int KS = kKS / 32;                  // MFMA k-steps per ring step
+  static constexpr int CH = 8;                         // 16-byte chunks of an epilogue row
+  static constexpr int EB = 2 * 32 * CH * 16;          // epilogue bytes per wavefront: 2 x 32 rows
+  static_assert((SLOTS - 2) * OPS < 64, "vmcnt range");
+  static_assert(SLOTS * 2 * OB + kGemmWaves * EB <= 160 * 1024, "LDS of a compute unit");
 };
 
-using BigTile = LinTile<2, 4>;    // 256 x 256, each wavefront 64 x 128
-using SmallTile = LinTile<1, 2>;  // 128 x 128, each wavefront 32 x 64
+using BigTile = LinTile<4, 2>;   // 256 x 256, 64 KiB steps
+using MidTile = LinTile<2, 4>;   // 128 x 128, 32 KiB steps
 
-// The per-lane pieces of a tile shape: copy offsets, operand offsets, the
-// k-step's copies and MFMAs, and the dequantising epilogue.
-template <int TMT, int TNT>
-struct LinLane {
-  using T = LinTile<TMT, TNT>;
-  int wave, wm, wn, hf, li;
-  uint32_t off[T::XU];  // copies: the same rows of both tiles
-  // Operand offsets.  Row 32 i + li of a wavefront's rows has the chunk
-  // swizzle (li / 2) mod 8 for every i (the rows differ above bit 4), so its
-  // 32-row tiles sit 4 KiB apart and one lane offset per k-step serves them
-  // all (the 4 KiB steps become instruction immediates).
-  int xk[T::KS], wk[T::KS];
-
-  __device__ __forceinline__ explicit LinLane(const LinearArgs& a) {
-    const int t = threadIdx.x;
-    const int lane = t % kWave;
-    wave = __builtin_amdgcn_readfirstlane(t / kWave);
-    wm = wave & 3;
-    wn = wave >> 2;
-    hf = lane >> 5;
-    li = lane & 31;
-    // each tile is units of 1 KiB (8 rows of 128 bytes); lane l lands at row
-    // 8 u + l / 8, chunk l % 8 of its unit and loads the chunk that the
-    // swizzle puts there
-#pragma unroll
-    for (int i = 0; i < T::XU; ++i) {
-      const int r = (wave * T::XU + i) * 8 + lane / 8;
-      off[i] = static_cast<uint32_t>(r * a.K + ((lane & 7) ^ qkv_swz(r)) * 16);
-    }
-#pragma unroll
-    for (int ks = 0; ks < T::KS; ++ks) {
-      const int c = ((ks * 2 + hf) ^ qkv_swz(li)) * 16;
-      xk[ks] = (wm * 32 * TMT + li) * kKS + c;
-      wk[ks] = T::XB + (wn * 32 * TNT + li) * kKS + c;
-    }
-  }
-
-  // The copies of k-step s of the operand rows at xb (xbytes readable) and wb
-  // (wbytes readable) into dst.  Ranges of 0 bytes read nothing.
-  __device__ __forceinline__ void stage(const int8_t* xb, int xbytes, const int8_t* wb,
-                                        int wbytes, int s, char* dst) const {
-    const int k0 = s * kKS;
-#pragma unroll
-    for (int i = 0; i < T::XU; ++i)
-      dma16(xb, xbytes, off[i], k0, dst + (wave * T::XU + i) * 1024);
-#pragma unroll
-    for (int i = 0; i < T::WU; ++i)
-      dma16(wb, wbytes, off[i], k0, dst + T::XB + (wave * T::WU + i) * 1024);
-  }
-
-  // One ring step: the copies of a later step into `fill` first, then the
-  // MFMAs of the step in `tile`, each with one operand read of the following
-  // k-steps.
-  __device__ __forceinline__ void step(v16i (&acc)[TNT][TMT], const char* tile,
-                                       const int8_t* fxb, int fxbytes, const int8_t* fwb,
-                                       int fwbytes, int fs, char* fill) const {
-    stage(fxb, fxbytes, fwb, fwbytes, fs, fill);
-#pragma unroll
-    for (int ks = 0; ks < T::KS; ++ks) {
-      v4i xf[TMT], wf[TNT];
-#pragma unroll
-      for (int i = 0; i < TMT; ++i)
-        xf[i] = *reinterpret_cast<const v4i*>(tile + xk[ks] + i * 32 * kKS);
-#pragma unroll
-      for (int i = 0; i < TNT; ++i)
-        wf[i] = *reinterpret_cast<const v4i*>(tile + wk[ks] + i * 32 * kKS);
-#pragma unroll
-      for (int tni = 0; tni < TNT; ++tni)
-#pragma unroll
-        for (int tmi = 0; tmi < TMT; ++tmi)
-          acc[tni][tmi] = __builtin_amdgcn_mfma_i32_32x32x32_i8(wf[tni], xf[tmi], acc[tni][tmi],
-                                                                0, 0, 0);
-    }
-    constexpr int kReads = TMT + TNT, kMfma = TMT * TNT;
-    __builtin_amdgcn_sched_group_barrier(0x020, T::OPS, 0);
-    __builtin_amdgcn_sched_group_barrier(0x100, kReads, 0);
-#pragma unroll
-    for (int i = 0; i < T::KS * kMfma; ++i) {
-      __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
-      if (i < (T::KS - 1) * kReads) __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
-    }
-  }
-
-  // epilogue: lane holds token m = li of each 32-token tile and channels
-  // 8 g + 4 hf + (0..3) of each 32-channel tile; lanes l and l + 32 swap
-  // halves so that each stores 8 consecutive channels (16 bytes)
-  __device__ __forceinline__ void store(const LinearArgs& a, const v16i (&acc)[TNT][TMT],
-                                        int64_t m0, int64_t n0) const {
-#pragma unroll
-    for (int tmi = 0; tmi < TMT; ++tmi) {
-      const int64_t m = m0 + wm * 32 * TMT + tmi * 32 + li;
-      if (m >= a.M) continue;
-      const float xs = a.xs[m];
-      u16* orow = a.out + m * a.ldo;
-#pragma unroll
-      for (int tni = 0; tni < TNT; ++tni)
-#pragma unroll
-        for (int p = 0; p < 2; ++p) {
-          uint32_t pk[2][2];
-#pragma unroll
-          for (int gg = 0; gg < 2; ++gg) {
-            const int g = 2 * p + gg;
-            const int64_t n = n0 + wn * 32 * TNT + tni * 32 + 8 * g + 4 * hf;
-            const float4 ws = *reinterpret_cast<const float4*>(a.ws + n);
-            float y[4] = {static_cast<float>(acc[tni][tmi][4 * g + 0]) * xs * ws.x,
-                          static_cast<float>(acc[tni][tmi][4 * g + 1]) * xs * ws.y,
-                          static_cast<float>(acc[tni][tmi][4 * g + 2]) * xs * ws.z,
-                          static_cast<float>(acc[tni][tmi][4 * g + 3]) * xs * ws.w};
-            if (a.bias != nullptr) {
-              const uint2 bb = *reinterpret_cast<const uint2*>(a.bias + n);
-              const float bv[4] = {__uint_as_float(bb.x << 16),
-                                   __uint_as_float(bb.x & 0xffff0000u),
-                                   __uint_as_float(bb.y << 16),
-                                   __uint_as_float(bb.y & 0xffff0000u)};
-#pragma unroll
-              for (int e = 0; e < 4; ++e) y[e] = bf16_to_f32(f32_to_bf16(y[e])) + bv[e];
-            }
-            pk[gg][0] = pack_bf16x2(y[0], y[1]);
-            pk[gg][1] = pack_bf16x2(y[2], y[3]);
-          }
-          // lane l (half 0) keeps channels 8(2p) + 0..3 and takes + 4..7 from
-          // lane l + 32, which keeps 8(2p + 1) + 4..7 and takes + 0..3
-          uint32_t st[4];
-#pragma unroll
-          for (int w = 0; w < 2; ++w) {
-            const auto r = __builtin_amdgcn_permlane32_swap(pk[0][w], pk[1][w], false, false);
-            st[w] = r[0];
-            st[2 + w] = r[1];
-          }
-          const int64_t n = n0 + wn * 32 * TNT + tni * 32 + 8 * (2 * p + hf);
-          *reinterpret_cast<uint4*>(orow + n) = make_uint4(st[0], st[1], st[2], st[3]);
-        }
-    }
-  }
-};
-
-template <int TMT, int TNT>
-__device__ __forceinline__ void zero_acc(v16i (&acc)[TNT][TMT]) {
-#pragma unroll
-  for (int i = 0; i < TNT; ++i)
-#pragma unroll
-    for (int j = 0; j < TMT; ++j)
-#pragma unroll
-      for (int r = 0; r < 16; ++r) acc[i][j][r] = 0;
-}
-
-// Operand rows of a tile and the bytes a copy may read (the rows past M of a
-// partial last tile read as zeros).
+// Where a tile's operands are and where its outputs go.
 struct TileSrc {
   const int8_t* xb;
   const int8_t* wb;
   int xbytes, wbytes;
+  int32_t g, m0, n0;
 };
-template <int TMT, int TNT>
-__device__ __forceinline__ TileSrc tile_src(const LinearArgs& a, int64_t m0, int64_t n0) {
-  using T = LinTile<TMT, TNT>;
-  const int64_t rows_x = a.M - m0 < T::BM ? a.M - m0 : T::BM;
-  return {a.x + m0 * a.K, a.w + n0 * a.K, static_cast<int>(rows_x * a.K),
-          static_cast<int>(T::BN * a.K)};
+
+// Tile `work` of the launch.  Consecutive tiles walk groups of kGroupM token
+// blocks for one channel block, then the next, so the 32 workgroups of an XCD
+// share 4 token blocks and 8 weight blocks in its L2.
+template <class L>
+__device__ __forceinline__ TileSrc tile_src(const LinearArgs& a, uint32_t work) {
+  constexpr uint32_t kGroupM = 4;
+  int32_t g = 0;
+#pragma unroll
+  for (int i = 1; i < kMaxLinear; ++i)
+    if (i < a.n_lin && work >= static_cast<uint32_t>(a.tiles[i])) g = i;
+  work -= static_cast<uint32_t>(a.tiles[g]);
+  const uint32_t n_m = static_cast<uint32_t>((a.M + L::B - 1) / L::B);
+  const uint32_t n_n = static_cast<uint32_t>(a.N[g]) / L::B;
+  const uint32_t group = work / (kGroupM * n_n), in_group = work % (kGroupM * n_n);
+  const uint32_t group_m = n_m - group * kGroupM < kGroupM ? n_m - group * kGroupM : kGroupM;
+  const int32_t m0 = static_cast<int32_t>((group * kGroupM + in_group % group_m) * L::B);
+  const int32_t n0 = static_cast<int32_t>(in_group / group_m * L::B);
+  const int64_t rows = a.M - m0 < L::B ? a.M - m0 : L::B;  // rows past M read as zeros
+  return {a.x + m0 * a.K, a.w[g] + n0 * a.K, static_cast<int>(rows * a.K),
+          static_cast<int>(L::B * a.K), g, m0, n0};
 }
 
-// One 128 x 128 tile: a 2-slot ring of k-steps (step j in slot j % 2; the
-// copies of step j + 1 go out at the start of step j, after every wavefront
-// has finished step j - 1 and step j has landed), then the epilogue.
-__device__ __forceinline__ void small_tile(const LinearArgs& a, int64_t m0, int64_t n0,
-                                           char* s_0, char* s_1) {
-  const LinLane<1, 2> L(a);
-  const TileSrc src = tile_src<1, 2>(a, m0, n0);
-  const int steps = static_cast<int>(a.K / kKS);
-  v16i acc[2][1];
-  zero_acc<1, 2>(acc);
-  L.stage(src.xb, src.xbytes, src.wb, src.wbytes, 0, s_0);
-  // past the last step the copies are empty ranges: nothing is read
-  auto fill_of = [&](int s) { return s < steps ? src : TileSrc{src.xb, src.wb, 0, 0}; };
-  for (int j = 0; j + 1 < steps; j += 2) {
-    qkv_wait_barrier<0>();
-    const TileSrc f1 = fill_of(j + 1);
-    L.step(acc, s_0, f1.xb, f1.xbytes, f1.wb, f1.wbytes, j + 1, s_1);
-    qkv_wait_barrier<0>();
-    const TileSrc f2 = fill_of(j + 2);
-    L.step(acc, s_1, f2.xb, f2.xbytes, f2.wb, f2.wbytes, j + 2, s_0);
+// One persistent workgroup per compute unit: workgroup j of XCD x takes the
+// XCD's tiles j, j + per_wg, ...  The copy ring runs on from tile to tile, so a
+// tile's first steps land during the previous tile's last MFMAs and epilogue.
+template <class L, bool OUT32>
+__global__ void __launch_bounds__(kGemmThreads) __attribute__((amdgpu_waves_per_eu(1, 1)))
+int8_linear_kernel(LinearArgs a, int32_t per_wg, int32_t per_xcd) {
+  constexpr int T = L::T, SLOTS = L::SLOTS, KS = L::KS;
+  // (slots in arrays of their own: the compiler then knows that reads of one do
+  // not alias the copies in flight into the others)
+  __shared__ __attribute__((aligned(1024))) char s_0[2 * L::OB];
+  __shared__ __attribute__((aligned(1024))) char s_1[2 * L::OB];
+  __shared__ __attribute__((aligned(1024))) char s_2[SLOTS > 2 ? 2 * L::OB : 16];
+  __shared__ __attribute__((aligned(1024))) char s_3[SLOTS > 2 ? 2 * L::OB : 16];
+  __shared__ __attribute__((aligned(1024))) char s_e[kGemmWaves * L::EB];
+  const int32_t first = static_cast<int32_t>(blockIdx.x % kNumXcd) * per_xcd;
+  const int32_t all = static_cast<int32_t>(a.tiles[a.n_lin]);
+  const int32_t end = first + per_xcd < all ? first + per_xcd : all;
+  int32_t item = first + static_cast<int32_t>(blockIdx.x / kNumXcd);
+  if (item >= end) return;
+
+  const int lane = threadIdx.x % kWave;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
+  const int wm = wave & 1, wn = wave >> 1, hf = lane >> 5, li = lane & 31;
+  // each operand's step is units of 1 KiB (8 rows of 128 bytes); lane l lands at
+  // row 8 u + l / 8, chunk l % 8 of its unit and loads the chunk that the
+  // swizzle puts there (the same rows of both operands)
+  uint32_t off[L::U];
+#pragma unroll
+  for (int i = 0; i < L::U; ++i) {
+    const int r = (wave * L::U + i) * 8 + lane / 8;
+    off[i] = static_cast<uint32_t>(r * a.K + ((lane & 7) ^ qkv_swz(r)) * 16);
   }
-  if (steps & 1) {  // the last step of an odd count, in slot 0
-    qkv_wait_barrier<0>();
-    L.step(acc, s_0, src.xb, 0, src.wb, 0, steps, s_1);
+  // Row 32 i + li of a wavefront's rows has the chunk swizzle (li / 2) mod 8 for
+  // every i, so its 32-row tiles sit 4 KiB apart and one lane offset per k-step
+  // serves them all (the 4 KiB steps become instruction immediates).
+  int xk[KS], wk[KS];
+#pragma unroll
+  for (int ks = 0; ks < KS; ++ks) {
+    const int c = ((ks * 2 + hf) ^ qkv_swz(li)) * 16;
+    xk[ks] = (wm * 32 * T + li) * kKS + c;
+    wk[ks] = L::OB + (wn * 32 * T + li) * kKS + c;
   }
-  __builtin_amdgcn_s_waitcnt(qkv_vmcnt(0));
-  L.store(a, acc, m0, n0);
-}
+  const int real_steps = static_cast<int>(a.K / kKS), steps = a.steps;
 
-// XCD-local big tile `work` -> its origin.  Consecutive work items of an XCD
-// walk groups of kGroupM token blocks for one channel block, then the next,
-// so the 32 workgroups of an XCD share 4 token blocks and 8 weight blocks in
-// its L2 (at 38,720 x 3072 x 3072, interleaved on one box: 0.398-0.403 ms with
-// 4 blocks per group; 2, 6 and 8: 0.407-0.414, 0.399-0.410 and 0.404-0.409 ms).
-__device__ __forceinline__ bool big_tile_of(const LinearArgs& a, int64_t work, int64_t* m0,
-                                            int64_t* n0) {
-  constexpr int64_t kGroupM = 4;
-  const int64_t n_m = (a.big_rows + BigTile::BM - 1) / BigTile::BM;
-  const int64_t tiles_n = a.N / BigTile::BN;
-  if (work >= n_m * tiles_n) return false;
-  const int64_t group = work / (kGroupM * tiles_n), in_group = work % (kGroupM * tiles_n);
-  const int64_t group_m = n_m - group * kGroupM < kGroupM ? n_m - group * kGroupM : kGroupM;
-  *m0 = (group * kGroupM + in_group % group_m) * BigTile::BM;
-  *n0 = (in_group / group_m) * BigTile::BN;
-  return true;
-}
+  // the copies of k-step s of a tile (none of the bytes of a step past K: zeros)
+  auto stage = [&](const TileSrc& t, int s, char* dst) __attribute__((always_inline)) {
+    const int xbytes = s < real_steps ? t.xbytes : 0, wbytes = s < real_steps ? t.wbytes : 0;
+    const int k0 = s * kKS;
+#pragma unroll
+    for (int i = 0; i < L::U; ++i)
+      dma16(t.xb, xbytes, off[i], k0, dst + (wave * L::U + i) * 1024);
+#pragma unroll
+    for (int i = 0; i < L::U; ++i)
+      dma16(t.wb, wbytes, off[i], k0, dst + L::OB + (wave * L::U + i) * 1024);
+  };
+  v4i xf[2][T], wf[2][T];
+  auto read = [&](const char* slot, auto ks_c, auto set_c) __attribute__((always_inline)) {
+    constexpr int ks = decltype(ks_c)::value, set = decltype(set_c)::value;
+#pragma unroll
+    for (int i = 0; i < T; ++i)
+      xf[set][i] = *reinterpret_cast<const v4i*>(slot + xk[ks] + i * 32 * kKS);
+#pragma unroll
+    for (int i = 0; i < T; ++i)
+      wf[set][i] = *reinterpret_cast<const v4i*>(slot + wk[ks] + i * 32 * kKS);
+  };
+  v16i acc[T][T];  // [channel tile][token tile]
+  auto mfma = [&](auto set_c) __attribute__((always_inline)) {
+    constexpr int set = decltype(set_c)::value;
+#pragma unroll
+    for (int n = 0; n < T; ++n)
+#pragma unroll
+      for (int m = 0; m < T; ++m)
+        acc[n][m] = __builtin_amdgcn_mfma_i32_32x32x32_i8(wf[set][n], xf[set][m], acc[n][m],
+                                                          0, 0, 0);
+  };
+  using std::integral_constant;
+  // Step s in slot `cur`: each k-step's operands are read during the MFMAs of
+  // the one before.  Before the last k-step every wavefront has read the slot
+  // and step s + 1 has landed (one barrier): the slot is refilled with step
+  // s + SLOTS of the stream and the next slot's first operands are read beside
+  // the last MFMAs.
+  auto step = [&](char* cur, const char* nxt, const TileSrc& ft,
+                  int fs) __attribute__((always_inline)) {
+    read(cur, integral_constant<int, 1>{}, integral_constant<int, 1>{});
+    mfma(integral_constant<int, 0>{});
+    read(cur, integral_constant<int, 2>{}, integral_constant<int, 0>{});
+    mfma(integral_constant<int, 1>{});
+    read(cur, integral_constant<int, 3>{}, integral_constant<int, 1>{});
+    mfma(integral_constant<int, 0>{});
+    // (operand reads first, then spread the rest of each group over the MFMAs)
+#pragma unroll
+    for (int q = 0; q < 3; ++q) {
+#pragma unroll
+      for (int i = 0; i < 2 * T; ++i) {
+        __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
+        __builtin_amdgcn_sched_group_barrier(0x008, T * T / (2 * T), 0);
+      }
+    }
+    lin_wait_barrier<(SLOTS - 2) * L::OPS>();
+    stage(ft, fs, cur);
+    read(nxt, integral_constant<int, 0>{}, integral_constant<int, 0>{});
+    mfma(integral_constant<int, 1>{});
+#pragma unroll
+    for (int i = 0; i < 2 * T; ++i) {
+      __builtin_amdgcn_sched_group_barrier(0x008, T * T / (2 * T), 0);
+      __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
+      __builtin_amdgcn_sched_group_barrier(0x020, L::OPS / (2 * T), 0);
+    }
+    __builtin_amdgcn_sched_barrier(0);
+  };
 
-// The 256 x 256 tiles items first, first + stride, ... of an XCD's per_xcd.
-// The ring runs on from tile to tile: with an even k-step count, the last
-// step of a tile fills the other slot with the next tile's first step, so
-// those copies fly during the epilogue (with an odd count the next tile
-// starts its ring after a barrier).
-__device__ __forceinline__ void big_tiles(const LinearArgs& a, int64_t xcd, int64_t first,
-                                          int64_t stride, int64_t per_xcd, char* s_0,
-                                          char* s_1) {
-  int64_t item = first, m0 = 0, n0 = 0;
-  if (item >= per_xcd || !big_tile_of(a, xcd * per_xcd + item, &m0, &n0)) return;
-  const LinLane<2, 4> L(a);
-  const int steps = static_cast<int>(a.K / kKS);
-  const bool chain = (steps & 1) == 0;
-  TileSrc src = tile_src<2, 4>(a, m0, n0);
-  L.stage(src.xb, src.xbytes, src.wb, src.wbytes, 0, s_0);
-  v16i acc[4][2];
+  // Epilogue: a lane holds token li of each 32-token tile and channels
+  // 8 g + 4 hf + (0..3) of each 32-channel tile; lanes l and l + 32 swap halves
+  // (8 consecutive channels each), and 32 tokens x 64 channels at a time go
+  // through the wavefront's own LDS rows so that stores write whole lines.
+  auto store = [&](const TileSrc& t) __attribute__((always_inline)) {
+    char* const eb = s_e + wave * L::EB;
+    const u16* const bias = a.bias[t.g];
+    const u16* const bias_or_ws =
+        bias != nullptr ? bias : reinterpret_cast<const u16*>(a.ws[t.g]);
+    uint32_t keep = bias != nullptr ? 0xffffffffu : 0u;
+    asm volatile("" : "+v"(keep));  // (masks, not sixteen branches)
+    const uint32_t none = ~keep & 0x80008000u;
+    const int64_t nw = t.n0 + wn * 32 * T, mw = t.m0 + wm * 32 * T;
+    float xs[T];
+#pragma unroll
+    for (int m = 0; m < T; ++m) {
+      const int64_t r = mw + m * 32 + li;
+      xs[m] = a.xs[r < a.M ? r : a.M - 1];
+    }
+    // stores through a buffer that ends after the tile's last row: rows past M
+    // are dropped
+    constexpr uint32_t kOutBytes = OUT32 ? 4 : 2;
+    const uint32_t row_bytes = static_cast<uint32_t>(a.ldo[t.g]) * kOutBytes;
+    const int64_t left = a.M - t.m0;
+    const uint32_t rows_left = static_cast<uint32_t>(left < L::B ? left : L::B);
+    const __amdgpu_buffer_rsrc_t out = __builtin_amdgcn_make_buffer_rsrc(
+        static_cast<char*>(a.out[t.g]) + static_cast<int64_t>(t.m0) * row_bytes, 0, static_cast<int>(rows_left * row_bytes), kQkvRsrc3);
+    const uint32_t lane_out = (lane / L::CH) * row_bytes + (lane % L::CH) * 8u * kOutBytes;
+    const int col = static_cast<int>(nw * kOutBytes);
+#pragma unroll
+    for (int np = 0; np < T / 2; ++np) {  // 64 channels: whole 128-byte lines
+      float4 ws[2][4];
+      uint2 bb[2][4];
+#pragma unroll
+      for (int n = 0; n < 2; ++n)
+#pragma unroll
+        for (int g = 0; g < 4; ++g) {
+          const int64_t c = nw + (2 * np + n) * 32 + 8 * g + 4 * hf;
+          ws[n][g] = *reinterpret_cast<const float4*>(a.ws[t.g] + c);
+          // (no bias: -0, which adds nothing to any value; the load then reads
+          // the scales, which are there and long enough)
+          const uint2 b = *reinterpret_cast<const uint2*>(bias_or_ws + c);
+          bb[n][g] = make_uint2((b.x & keep) | none, (b.y & keep) | none);
+        }
+      __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+      for (int m = 0; m < T; ++m) {
+        char* const rows = eb + (m & 1) * (32 * L::CH * 16);
+        // (the accumulators leave their AGPRs here, not all before the epilogue)
+        asm volatile("" : "+a"(acc[2 * np][m]), "+a"(acc[2 * np + 1][m]));
+#pragma unroll
+        for (int n = 0; n < 2; ++n)
+#pragma unroll
+          for (int p = 0; p < 2; ++p) {
+            uint32_t pk[2][2];
+#pragma unroll
+            for (int gg = 0; gg < 2; ++gg) {
+              const int g = 2 * p + gg;
+              const float wv[4] = {ws[n][g].x, ws[n][g].y, ws[n][g].z, ws[n][g].w};
+              float y[4];
+#pragma unroll
+              for (int e = 0; e < 4; ++e)
+                y[e] = static_cast<float>(acc[2 * np + n][m][4 * g + e]) * xs[m] * wv[e];
+              pk[gg][0] = cvt_bf16x2(y[0], y[1]);
+              pk[gg][1] = cvt_bf16x2(y[2], y[3]);
+              const uint32_t bw[2] = {bb[n][g].x, bb[n][g].y};
+#pragma unroll
+              for (int w = 0; w < 2; ++w)
+                pk[gg][w] = cvt_bf16x2(
+                    __uint_as_float(pk[gg][w] << 16) + __uint_as_float(bw[w] << 16),
+                    __uint_as_float(pk[gg][w] & 0xffff0000u) +
+                        __uint_as_float(bw[w] & 0xffff0000u));
+            }
+            // lane l (half 0) keeps channels 8(2p) + 0..3 and takes + 4..7 from
+            // lane l + 32, which keeps 8(2p + 1) + 4..7 and takes + 0..3
+            v4u st;
+#pragma unroll
+            for (int w = 0; w < 2; ++w) {
+              const auto r = __builtin_amdgcn_permlane32_swap(pk[0][w], pk[1][w], false, false);
+              st[w] = r[0];
+              st[2 + w] = r[1];
+            }
+            const int c = n * 4 + 2 * p + hf;
+            *reinterpret_cast<v4u*>(rows + (li * L::CH + (c ^ (li & (L::CH - 1)))) * 16) = st;
+          }
+        // (the rows are this wavefront's own: its LDS operations stay in order)
+#pragma unroll
+        for (int i = 0; i < 32 * L::CH / kWave; ++i) {
+          const int r = i * (kWave / L::CH) + lane / L::CH, c = lane % L::CH;
+          const v4u v = *reinterpret_cast<const v4u*>(
+              rows + (r * L::CH + (c ^ (r & (L::CH - 1)))) * 16);
+          const uint32_t row = wm * 32 * T + m * 32 + i * (kWave / L::CH);
+          const int voff = static_cast<int>(row * row_bytes + lane_out);
+          const int soff = col + np * 64 * static_cast<int>(kOutBytes);
+          if constexpr (OUT32) {
+            const v4u lo = {v[0] << 16, v[0] & 0xffff0000u, v[1] << 16, v[1] & 0xffff0000u};
+            const v4u hi = {v[2] << 16, v[2] & 0xffff0000u, v[3] << 16, v[3] & 0xffff0000u};
+            __builtin_amdgcn_raw_buffer_store_b128(lo, out, voff, soff, 0);
+            __builtin_amdgcn_raw_buffer_store_b128(hi, out, voff + 16, soff, 0);
+          } else {
+            __builtin_amdgcn_raw_buffer_store_b128(v, out, voff, soff, 0);
+          }
+        }
+        __builtin_amdgcn_sched_barrier(0);
+      }
+    }
+  };
+
+  TileSrc cur = tile_src<L>(a, static_cast<uint32_t>(item));
+#pragma unroll
+  for (int i = 0; i < SLOTS; ++i) {
+    stage(cur, i, i == 0 ? s_0 : i == 1 ? s_1 : i == 2 ? s_2 : s_3);
+    __builtin_amdgcn_sched_barrier(0);  // the steps' copies stay in order
+  }
+  lin_wait_barrier<(SLOTS - 1) * L::OPS>();
+  read(s_0, integral_constant<int, 0>{}, integral_constant<int, 0>{});
   while (true) {
-    zero_acc<2, 4>(acc);
-    const int64_t next = item + stride;
-    int64_t nm0 = 0, nn0 = 0;
-    const bool has_next = next < per_xcd && big_tile_of(a, xcd * per_xcd + next, &nm0, &nn0);
-    TileSrc nsrc = tile_src<2, 4>(a, nm0, nn0);
-    if (!(has_next && chain)) nsrc.xbytes = nsrc.wbytes = 0;  // the last fill reads nothing
-    for (int j = 0; j + 1 < steps; j += 2) {
-      qkv_wait_barrier<0>();
-      L.step(acc, s_0, src.xb, src.xbytes, src.wb, src.wbytes, j + 1, s_1);
-      qkv_wait_barrier<0>();
-      // one step call with selected operands (a branch between two calls
-      // makes the compiler spill)
-      const bool last = j + 2 >= steps;
-      L.step(acc, s_1, last ? nsrc.xb : src.xb, last ? nsrc.xbytes : src.xbytes,
-             last ? nsrc.wb : src.wb, last ? nsrc.wbytes : src.wbytes, last ? 0 : j + 2, s_0);
-    }
-    if (!chain) {  // the last step of an odd count, in slot 0
-      qkv_wait_barrier<0>();
-      L.step(acc, s_0, src.xb, 0, src.wb, 0, steps, s_1);
-    }
-    L.store(a, acc, m0, n0);
+#pragma unroll
+    for (int n = 0; n < T; ++n)
+#pragma unroll
+      for (int m = 0; m < T; ++m)
+#pragma unroll
+        for (int r = 0; r < 16; ++r) acc[n][m][r] = 0;
+    const int32_t next = item + per_wg;
+    const bool has_next = next < end;
+    TileSrc nt = has_next ? tile_src<L>(a, static_cast<uint32_t>(next)) : cur;
+    if (!has_next) nt.xbytes = nt.wbytes = 0;  // the last fills read nothing
+    int s = 0;
+    do {  // (steps >= SLOTS)
+      const bool last = s + SLOTS >= steps;  // refill with the next tile's first steps
+      TileSrc ft = cur;
+      ft.xb = last ? nt.xb : cur.xb;
+      ft.wb = last ? nt.wb : cur.wb;
+      ft.xbytes = last ? nt.xbytes : cur.xbytes;
+      ft.wbytes = last ? nt.wbytes : cur.wbytes;
+      const int fs = last ? 0 : s + SLOTS;
+      if constexpr (SLOTS == 2) {
+        step(s_0, s_1, ft, fs);
+        step(s_1, s_0, ft, fs + 1);
+      } else {
+        step(s_0, s_1, ft, fs);
+        step(s_1, s_2, ft, fs + 1);
+        step(s_2, s_3, ft, fs + 2);
+        step(s_3, s_0, ft, fs + 3);
+      }
+      s += SLOTS;
+    } while (s < steps);
+    store(cur);
     if (!has_next) break;
     item = next;
-    m0 = nm0;
-    n0 = nn0;
-    src = tile_src<2, 4>(a, m0, n0);
-    if (!chain) {  // every wavefront is past its last step before slot 0 refills
-      __builtin_amdgcn_s_waitcnt(qkv_vmcnt(0));
-      __syncthreads();
-      L.stage(src.xb, src.xbytes, src.wb, src.wbytes, 0, s_0);
-    }
+    cur = nt;
   }
-  __builtin_amdgcn_s_waitcnt(qkv_vmcnt(0));
-}
-
-// One workgroup per compute unit (the LDS ring admits one), `per_wg` of them
-// on each XCD: workgroup j of XCD x takes the XCD's 128 x 128 tiles j,
-// j + per_wg, ... (the rows past big_rows), then its 256 x 256 tiles the
-// same way.  The compute units that take a small tile start their big tiles
-// a quarter tile later than the others, so the two groups' output stores
-// fall beside the other group's MFMAs instead of all at once.
-__global__ void __launch_bounds__(kGemmThreads) __attribute__((amdgpu_waves_per_eu(2, 2)))
-int8_linear_kernel(LinearArgs a, int64_t per_wg, int64_t per_xcd_small, int64_t per_xcd_big) {
-  __shared__ __attribute__((aligned(1024))) char s_0[BigTile::XB + BigTile::WB];
-  __shared__ __attribute__((aligned(1024))) char s_1[BigTile::XB + BigTile::WB];
-  const int64_t xcd = blockIdx.x % kNumXcd, j = blockIdx.x / kNumXcd;
-  const int64_t tiles_n = a.N / SmallTile::BN;
-  const int64_t n_small =
-      (a.M - a.big_rows + SmallTile::BM - 1) / SmallTile::BM * tiles_n;
-  for (int64_t i = j; i < per_xcd_small; i += per_wg) {
-    const int64_t tile = xcd * per_xcd_small + i;
-    if (tile >= n_small) break;
-    small_tile(a, a.big_rows + tile / tiles_n * SmallTile::BM, tile % tiles_n * SmallTile::BN,
-               s_0, s_1);
-    __syncthreads();  // every wavefront is done with the slots
-  }
-  big_tiles(a, xcd, j, per_wg, per_xcd_big, s_0, s_1);
+  // the trailing copies (empty ranges) land before the slots are freed
+  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
 }
 
 }  // namespace rcsa
 
 using namespace rcsa;
+
+template <typename T>
+static void launch_quant_rows(const void* x, int64_t M, int64_t C, int64_t ldx, int8_t* q,
+                              float* scale, hipStream_t stream) {
+  const int64_t rows_per = kQThreads / kWave;
+  const dim3 grid(static_cast<unsigned>((M + rows_per - 1) / rows_per)), block(kQThreads);
+  const T* xt = static_cast<const T*>(x);
+  const int64_t chunks = (C + 511) / 512;
+  if (chunks <= 2) quant_rows_kernel<T, 2><<<grid, block, 0, stream>>>(xt, M, C, ldx, q, scale);
+  else if (chunks <= 4) quant_rows_kernel<T, 4><<<grid, block, 0, stream>>>(xt, M, C, ldx, q, scale);
+  else if (chunks <= 6) quant_rows_kernel<T, 6><<<grid, block, 0, stream>>>(xt, M, C, ldx, q, scale);
+  else if (chunks <= 10) quant_rows_kernel<T, 10><<<grid, block, 0, stream>>>(xt, M, C, ldx, q, scale);
+  else quant_rows_kernel<T, 0><<<grid, block, 0, stream>>>(xt, M, C, ldx, q, scale);
+}
 
 extern "C" int rcsa_quantize_rows_int8(const void* x, int dtype, int64_t M, int64_t C, int64_t ldx,
                                        int8_t* q, float* scale, hipStream_t stream) {
@@ -416,56 +489,94 @@ extern "C" int rcsa_quantize_rows_int8(const void* x, int dtype, int64_t M, int6
   if (M <= 0 || C <= 0 || C % 8 || ldx < C || ldx % 8) return RCSA_ERR_SHAPE;
   if ((reinterpret_cast<uintptr_t>(x) & 15u) || (reinterpret_cast<uintptr_t>(q) & 7u))
     return RCSA_ERR_ALIGN;
-  const int64_t rows_per = kQThreads / kWave;
-  const dim3 grid(static_cast<unsigned>((M + rows_per - 1) / rows_per));
-  if (dtype == RCSA_BF16)
-    quant_rows_kernel<u16><<<grid, dim3(kQThreads), 0, stream>>>(static_cast<const u16*>(x), M, C,
-                                                                  ldx, q, scale);
-  else if (dtype == RCSA_F32)
-    quant_rows_kernel<float><<<grid, dim3(kQThreads), 0, stream>>>(static_cast<const float*>(x), M,
-                                                                    C, ldx, q, scale);
-  else
-    return RCSA_ERR_DTYPE;
+  if (dtype == RCSA_BF16) launch_quant_rows<u16>(x, M, C, ldx, q, scale, stream);
+  else if (dtype == RCSA_F32) launch_quant_rows<float>(x, M, C, ldx, q, scale, stream);
+  else return RCSA_ERR_DTYPE;
   return launch_status();
+}
+
+// Compute units of the current device (256 when it cannot be read).
+static int64_t device_cus() {
+  int dev = 0, cus = 0;
+  if (hipGetDevice(&dev) != hipSuccess ||
+      hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess ||
+      cus < kNumXcd)
+    return 256;
+  return cus;
+}
+
+template <class L>
+static int64_t count_tiles(LinearArgs& a) {
+  a.tiles[0] = 0;
+  for (int g = 0; g < a.n_lin; ++g)
+    a.tiles[g + 1] = a.tiles[g] + (a.M + L::B - 1) / L::B * (a.N[g] / L::B);
+  return a.tiles[a.n_lin];
+}
+
+template <class L>
+static int launch_linear(LinearArgs& a, int64_t cus, bool out_f32, hipStream_t stream) {
+  const int64_t tiles = count_tiles<L>(a);
+  if (tiles >= (int64_t{1} << 30)) return RCSA_ERR_SHAPE;
+  a.steps = static_cast<int32_t>((a.K / kKS + L::SLOTS - 1) / L::SLOTS * L::SLOTS);
+  // one workgroup per compute unit, the same number on every XCD
+  const int64_t per_xcd = (tiles + kNumXcd - 1) / kNumXcd;
+  const int64_t per_wg = per_xcd < cus / kNumXcd ? per_xcd : cus / kNumXcd;
+  const dim3 grid(static_cast<unsigned>(per_wg * kNumXcd)), block(kGemmThreads);
+  const int32_t wg = static_cast<int32_t>(per_wg), px = static_cast<int32_t>(per_xcd);
+  if (out_f32) int8_linear_kernel<L, true><<<grid, block, 0, stream>>>(a, wg, px);
+  else int8_linear_kernel<L, false><<<grid, block, 0, stream>>>(a, wg, px);
+  return launch_status();
+}
+
+extern "C" int rcsa_int8_linear_group(const int8_t* x, const float* x_scale, int64_t n_linear,
+                                      const int8_t* const* w, const float* const* w_scale,
+                                      const void* const* bias, const int64_t* N,
+                                      void* const* out, const int64_t* ldo, int out_f32,
+                                      int64_t M, int64_t K, hipStream_t stream) {
+  if (!x || !x_scale || !w || !w_scale || !bias || !N || !out || !ldo) return RCSA_ERR_NULL;
+  if (n_linear <= 0 || n_linear > kMaxLinear || M <= 0 || M >= (int64_t{1} << 31) - 256 ||
+      K <= 0 || K % kKS)
+    return RCSA_ERR_SHAPE;
+  // the copies address a tile with 32-bit offsets
+  if (static_cast<int64_t>(BigTile::B) * K >= (int64_t{1} << 31)) return RCSA_ERR_SHAPE;
+  if (reinterpret_cast<uintptr_t>(x) & 15u) return RCSA_ERR_ALIGN;
+  LinearArgs a{};
+  a.x = x;
+  a.xs = x_scale;
+  a.M = M;
+  a.K = K;
+  a.n_lin = static_cast<int32_t>(n_linear);
+  for (int g = 0; g < a.n_lin; ++g) {
+    if (!w[g] || !w_scale[g] || !out[g]) return RCSA_ERR_NULL;
+    // (the stores address a tile's rows with 32-bit offsets)
+    if (N[g] <= 0 || N[g] % BigTile::B || ldo[g] < N[g] || ldo[g] % 4 ||
+        ldo[g] >= (int64_t{1} << 30) / BigTile::B)
+      return RCSA_ERR_SHAPE;
+    if ((reinterpret_cast<uintptr_t>(w[g]) & 15u) ||
+        (reinterpret_cast<uintptr_t>(w_scale[g]) & 15u) ||
+        (reinterpret_cast<uintptr_t>(out[g]) & 7u) || (reinterpret_cast<uintptr_t>(bias[g]) & 7u))
+      return RCSA_ERR_ALIGN;
+    a.w[g] = w[g];
+    a.ws[g] = w_scale[g];
+    a.bias[g] = static_cast<const u16*>(bias[g]);
+    a.out[g] = out[g];
+    a.N[g] = N[g];
+    a.ldo[g] = ldo[g];
+  }
+  // The tile size that needs less time for its whole rounds: a round of 128 x 128
+  // tiles takes 5/16 of a round of 256 x 256 tiles (14 and 44 us at K 3072; three
+  // projections of 880 tokens: 2 rounds, 32 us, against 1 round, 44 us; of 1760
+  // tokens: 4 rounds, 59 us, against 1 round, 51 us).
+  const int64_t cus = device_cus();
+  const int64_t big = (count_tiles<BigTile>(a) + cus - 1) / cus * 16;
+  const int64_t mid = (count_tiles<MidTile>(a) + cus - 1) / cus * 5;
+  return big <= mid ? launch_linear<BigTile>(a, cus, out_f32 != 0, stream)
+                    : launch_linear<MidTile>(a, cus, out_f32 != 0, stream);
 }
 
 extern "C" int rcsa_int8_linear(const int8_t* x, const float* x_scale, const int8_t* w,
                                 const float* w_scale, const void* bias, int64_t M, int64_t N,
                                 int64_t K, void* out, int64_t ldo, hipStream_t stream) {
-  if (!x || !x_scale || !w || !w_scale || !out) return RCSA_ERR_NULL;
-  if (M <= 0 || N <= 0 || K <= 0 || N % BigTile::BN || K % kKS || ldo < N || ldo % 4)
-    return RCSA_ERR_SHAPE;
-  // the copies address a tile with 32-bit offsets
-  if (static_cast<int64_t>(BigTile::BM) * K >= (int64_t{1} << 31)) return RCSA_ERR_SHAPE;
-  if ((reinterpret_cast<uintptr_t>(x) & 15u) || (reinterpret_cast<uintptr_t>(w) & 15u) ||
-      (reinterpret_cast<uintptr_t>(w_scale) & 15u) || (reinterpret_cast<uintptr_t>(out) & 7u) ||
-      (reinterpret_cast<uintptr_t>(bias) & 7u))
-    return RCSA_ERR_ALIGN;
-  // 256 x 256 tiles, except that a short last round (fewer tiles than half the
-  // compute units) is re-cut: the rows its tiles would cover go to 128 x 128
-  // tiles, a quarter of the work each, taken first (which also offsets the
-  // rounds of the compute units that take one)
-  const int64_t big_n = N / BigTile::BN;
-  const int64_t all_big = ((M + BigTile::BM - 1) / BigTile::BM) * big_n;
-  int64_t big_rows = M;
-  int dev = 0, cus = 0;
-  if (hipGetDevice(&dev) == hipSuccess &&
-      hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) == hipSuccess &&
-      cus > 0) {
-    const int64_t rem = all_big % cus;
-    const int64_t rows = (all_big - rem) / big_n * BigTile::BM;  // whole row blocks of full rounds
-    if (rem != 0 && 2 * rem < cus && rows > 0 && rows < M) big_rows = rows;
-  }
-  const int64_t big_tiles = ((big_rows + BigTile::BM - 1) / BigTile::BM) * big_n;
-  const int64_t small_tiles =
-      big_rows < M ? ((M - big_rows + SmallTile::BM - 1) / SmallTile::BM) * (N / SmallTile::BN) : 0;
-  if (big_tiles >= (int64_t{1} << 30) || small_tiles >= (int64_t{1} << 30)) return RCSA_ERR_SHAPE;
-  LinearArgs a{x, x_scale, w, w_scale, static_cast<const u16*>(bias), static_cast<u16*>(out),
-               M, N, K, ldo, big_rows};
-  // one workgroup per compute unit, the same number on every XCD
-  const int64_t per_wg = cus >= kNumXcd ? cus / kNumXcd : 32;
-  const dim3 grid(static_cast<unsigned>(per_wg * kNumXcd));
-  int8_linear_kernel<<<grid, dim3(kGemmThreads), 0, stream>>>(
-      a, per_wg, (small_tiles + kNumXcd - 1) / kNumXcd, (big_tiles + kNumXcd - 1) / kNumXcd);
-  return launch_status();
+  return rcsa_int8_linear_group(x, x_scale, 1, &w, &w_scale, &bias, &N, &out, &ldo, 0, M, K,
+                                stream);
 }

@@ -38,6 +38,7 @@ struct Api {
   decltype(&rcsa_sparse_attn_int8_split) sparse_attn_int8_split = nullptr;
   decltype(&rcsa_quantize_rows_int8) quantize_rows_int8 = nullptr;
   decltype(&rcsa_int8_linear) int8_linear = nullptr;
+  decltype(&rcsa_int8_linear_group) int8_linear_group = nullptr;
 };
 
 std::mutex g_mu;
@@ -63,6 +64,7 @@ void bind_library(const std::string& path) {
   bind_one(h, "rcsa_sparse_attn_int8_split", api.sparse_attn_int8_split);
   bind_one(h, "rcsa_quantize_rows_int8", api.quantize_rows_int8);
   bind_one(h, "rcsa_int8_linear", api.int8_linear);
+  bind_one(h, "rcsa_int8_linear_group", api.int8_linear_group);
   g_api = api;
   g_bound = true;
 }
@@ -506,6 +508,61 @@ void int8_linear(const at::Tensor& x_i8, const at::Tensor& x_scale, const at::Te
                                     l.stream));
 }
 
+// projections of one x [M, K]: w[g] [N_g, K], out[g] [M, N_g] (all bf16 or all fp32)
+void int8_linear_group(const at::Tensor& x_i8, const at::Tensor& x_scale, at::TensorList w,
+                       at::TensorList w_scale, const c10::List<c10::optional<at::Tensor>>& bias,
+                       at::TensorList out) {
+  const char* op = "int8_linear_group";
+  const Api& a = api(op);
+  const size_t n = w.size();
+  TORCH_CHECK(n > 0 && n <= 4 && w_scale.size() == n && bias.size() == n && out.size() == n, op,
+              ": one to four weights, with as many scales, biases and outputs");
+  int dev = -1;
+  on_device(op, dev, x_i8, "x");
+  on_device(op, dev, x_scale, "x_scale");
+  TORCH_CHECK(x_i8.dim() == 2 && x_i8.is_contiguous(), op, ": x must be a contiguous matrix");
+  want(op, x_i8, at::kChar, "x");
+  want(op, x_scale, at::kFloat, "x_scale");
+  const int64_t M = x_i8.size(0), K = x_i8.size(1);
+  want_numel(op, x_scale, M, "x_scale");
+  const at::ScalarType dt = out[0].scalar_type();
+  TORCH_CHECK(dt == at::kBFloat16 || dt == at::kFloat, op, ": out must be bfloat16 or float32");
+  const int8_t* wp[4];
+  const float* sp[4];
+  const void* bp[4];
+  void* outp[4];
+  int64_t N[4], ldo[4];
+  for (size_t g = 0; g < n; ++g) {
+    on_device(op, dev, w[g], "w");
+    on_device(op, dev, w_scale[g], "w_scale");
+    on_device(op, dev, out[g], "out");
+    const c10::optional<at::Tensor> b = bias.get(g);
+    on_device(op, dev, b, "bias");
+    want(op, w[g], at::kChar, "w");
+    want(op, w_scale[g], at::kFloat, "w_scale");
+    want(op, out[g], dt, "out");
+    TORCH_CHECK(w[g].dim() == 2 && w[g].is_contiguous() && w[g].size(1) == K, op,
+                ": w must be contiguous [N, K] matrices");
+    N[g] = w[g].size(0);
+    want_numel(op, w_scale[g], N[g], "w_scale");
+    if (b.has_value()) {
+      want(op, *b, at::kBFloat16, "bias");
+      want_numel(op, *b, N[g], "bias");
+    }
+    TORCH_CHECK(out[g].dim() == 2 && out[g].size(0) == M && out[g].size(1) == N[g] &&
+                    out[g].stride(1) == 1, op, ": out must be [M, N] with unit column stride");
+    wp[g] = ptr<const int8_t>(w[g]);
+    sp[g] = ptr<const float>(w_scale[g]);
+    bp[g] = ptr<const void>(b);
+    outp[g] = out[g].data_ptr();
+    ldo[g] = out[g].stride(0);
+  }
+  const Launch l(device_of(op, dev));
+  check_status(a, op, a.int8_linear_group(ptr<const int8_t>(x_i8), ptr<const float>(x_scale),
+                                          static_cast<int64_t>(n), wp, sp, bp, N, outp, ldo,
+                                          dt == at::kFloat, M, K, l.stream));
+}
+
 }  // namespace
 
 TORCH_LIBRARY(rcsa, m) {
@@ -544,4 +601,8 @@ TORCH_LIBRARY(rcsa, m) {
       "int8_linear(Tensor x_i8, Tensor x_scale, Tensor w_i8, Tensor w_scale, Tensor? bias, "
       "Tensor(a!) out) -> ()",
       &int8_linear);
+  m.def(
+      "int8_linear_group(Tensor x_i8, Tensor x_scale, Tensor[] w, Tensor[] w_scale, "
+      "Tensor?[] bias, Tensor(a!)[] out) -> ()",
+      &int8_linear_group);
 }

@@ -995,21 +995,55 @@ def int8_linear(x_i8: torch.Tensor, x_scale: torch.Tensor, w_i8: torch.Tensor,
     _require_cuda(fn, x_i8, x_scale, w_i8, w_scale)
     if x_i8.dtype != torch.int8 or w_i8.dtype != torch.int8:
         raise TypeError(f"{fn}: x and w must be int8")
-    x_i8, w_i8 = x_i8.contiguous(), w_i8.contiguous()
+    x_i8 = x_i8.contiguous()
     M, K = x_i8.shape
-    N, K2 = w_i8.shape
-    if K2 != K:
-        raise ValueError(f"{fn}: x [M, {K}] and w [N, {K2}] disagree")
-    xs = x_scale.reshape(-1).float().contiguous()
-    ws = w_scale.reshape(-1).float().contiguous()
-    if xs.numel() != M or ws.numel() != N:
-        raise ValueError(f"{fn}: need {M} token scales and {N} channel scales")
-    b = bias.reshape(-1).to(torch.bfloat16).contiguous() if bias is not None else None
-    if b is not None and b.numel() != N:
-        raise ValueError(f"{fn}: bias must have {N} entries")
+    xs = _token_scales(x_scale, M, fn)
+    w_i8, ws, b = _projection(w_i8, w_scale, bias, K, fn)
+    N = w_i8.shape[0]
     if out is None:
         out = torch.empty(M, N, device=x_i8.device, dtype=torch.bfloat16)
     if out.dtype != torch.bfloat16 or out.shape != (M, N) or out.stride(1) != 1:
         raise ValueError(f"{fn}: out must be bfloat16 [{M}, {N}] with contiguous rows")
     _lib.torch_ops().int8_linear(x_i8, xs, w_i8, ws, b, out)
     return out
+
+
+def _token_scales(x_scale: torch.Tensor, M: int, fn: str) -> torch.Tensor:
+    xs = x_scale.reshape(-1).float().contiguous()
+    if xs.numel() != M:
+        raise ValueError(f"{fn}: need {M} token scales")
+    return xs
+
+
+def _projection(w_i8, w_scale, bias, K: int, fn: str):
+    """A projection's weights, scales and bias as the kernel reads them."""
+    w_i8 = w_i8.contiguous()
+    N, K2 = w_i8.shape
+    if K2 != K:
+        raise ValueError(f"{fn}: x [M, {K}] and w [N, {K2}] disagree")
+    ws = w_scale.reshape(-1).float().contiguous()
+    if ws.numel() != N:
+        raise ValueError(f"{fn}: need {N} channel scales")
+    b = bias.reshape(-1).to(torch.bfloat16).contiguous() if bias is not None else None
+    if b is not None and b.numel() != N:
+        raise ValueError(f"{fn}: bias must have {N} entries")
+    return w_i8, ws, b
+
+
+def int8_linear_group(x_i8: torch.Tensor, x_scale: torch.Tensor, projections, *,
+                      out_dtype=torch.bfloat16):
+    """``int8_linear`` of several ``(w_i8, w_scale, bias)`` (one to four) over one x in
+    one launch (``rcsa_int8_linear_group``); ``out_dtype`` float32 widens the bf16
+    values in the same pass.  Returns their outputs ``[M, N]``."""
+    fn = "int8_linear_group"
+    _require_cuda(fn, x_i8, x_scale, *(t for p in projections for t in p[:2]))
+    if x_i8.dtype != torch.int8 or any(p[0].dtype != torch.int8 for p in projections):
+        raise TypeError(f"{fn}: x and w must be int8")
+    x_i8 = x_i8.contiguous()
+    M, K = x_i8.shape
+    xs = _token_scales(x_scale, M, fn)
+    ready = [_projection(*p, K, fn) for p in projections]
+    outs = [torch.empty(M, w.shape[0], device=x_i8.device, dtype=out_dtype) for w, _, _ in ready]
+    _lib.torch_ops().int8_linear_group(x_i8, xs, [p[0] for p in ready], [p[1] for p in ready],
+                                       [p[2] for p in ready], outs)
+    return outs

@@ -6,7 +6,8 @@ self-attention block quantise their common input once and reuse it.  The
 modules are the upstream Matrix ``Int8Linear`` layers (``in_features``,
 ``out_features``, ``weight_int8`` [out, in], ``weight_scales`` [out],
 ``bias``); the quantiser and the GEMMs are ``rcsa_quantize_rows_int8`` and
-``rcsa_int8_linear`` (int8 MFMA with the dequantising epilogue) instead of the
+``rcsa_int8_linear_group`` (int8 MFMA with the dequantising epilogue, the three
+projections in one launch) instead of the
 upstream Triton kernels.  Each projection returns bf16(acc * x_scale * w_scale),
 plus the bias in bf16, cast to the input's dtype, as the reference does.
 """
@@ -20,13 +21,6 @@ import torch
 from . import ops
 
 _REQUIRED = ("in_features", "out_features", "weight_int8", "weight_scales", "bias")
-
-
-def _project(module: Any, x_i8: torch.Tensor, x_scale: torch.Tensor, x_shape: torch.Size,
-             output_dtype: torch.dtype) -> torch.Tensor:
-    out = ops.int8_linear(x_i8, x_scale, module.weight_int8, module.weight_scales,
-                          bias=module.bias)
-    return out.view(*x_shape[:-1], int(module.out_features)).to(output_dtype)
 
 
 def shared_int8_qkv(q_module: Any, k_module: Any, v_module: Any, x: torch.Tensor):
@@ -46,7 +40,13 @@ def shared_int8_qkv(q_module: Any, k_module: Any, v_module: Any, x: torch.Tensor
     if any(m.weight_int8.dtype != torch.int8 for m in modules):
         raise RuntimeError("shared Matrix QKV weights must be int8")
     x_i8, x_scale = ops.quantize_rows_int8(x)
-    return tuple(_project(m, x_i8, x_scale, x.shape, x.dtype) for m in modules)
+    # the kernel widens its bf16 values itself for an fp32 input
+    wide = torch.float32 if x.dtype == torch.float32 else torch.bfloat16
+    outs = ops.int8_linear_group(
+        x_i8, x_scale, [(m.weight_int8, m.weight_scales, m.bias) for m in modules],
+        out_dtype=wide)
+    return tuple(o.view(*x.shape[:-1], int(m.out_features)).to(x.dtype)
+                 for m, o in zip(modules, outs))
 
 
 class SharedInt8QKVForwardCoordinator:

@@ -619,12 +619,22 @@ int rcsa_order_lists(const int32_t* block_indices, const int32_t* block_indices_
  * The launch is persistent (one workgroup per compute unit, each with a fixed
  * share of the tiles): it expects the device to itself, and beside other
  * kernels it stays correct but runs as slowly as its latest workgroup.
+ *
+ * rcsa_int8_linear_group: n_linear (1 to 4) such projections of one x in one
+ * launch; w, w_scale, bias (entries may be NULL), N, out and ldo are host arrays
+ * of n_linear entries, read before the call returns.  With out_f32 the outputs
+ * are fp32 (ldo in elements): the bf16 values, widened.
  */
 int rcsa_quantize_rows_int8(const void* x, int dtype, int64_t M, int64_t C, int64_t ldx,
                             int8_t* q, float* scale, hipStream_t stream);
 int rcsa_int8_linear(const int8_t* x, const float* x_scale, const int8_t* w, const float* w_scale,
                      const void* bias, int64_t M, int64_t N, int64_t K, void* out, int64_t ldo,
                      hipStream_t stream);
+int rcsa_int8_linear_group(const int8_t* x, const float* x_scale, int64_t n_linear,
+                           const int8_t* const* w, const float* const* w_scale,
+                           const void* const* bias, const int64_t* N, void* const* out,
+                           const int64_t* ldo, int out_f32, int64_t M, int64_t K,
+                           hipStream_t stream);
 
 #ifdef __cplusplus
 }
