@@ -494,6 +494,7 @@ sparse_attn_kernel(AttnArgs a) {
   }();
   auto mask_of = [&](int n, uint2 words) __attribute__((always_inline)) -> uint64_t {
     const uint64_t m = words.x | (static_cast<uint64_t>(words.y) << 32);
+    if constexpr (GATHER) return n < 0 ? 0ull : m;  // (whole key blocks: no tail)
     return static_cast<uint32_t>(n) > last_step ? 0ull : (n == tail_step ? m & tail_keep : m);
   };
   // MASK: the caller's validity bits; otherwise the staged validity bytes
