@@ -21,6 +21,7 @@ RCSA_BF16 = 0
 RCSA_F32 = 1
 RCSA_ORDER_INDEX = 0
 RCSA_ORDER_RANK = 1
+RCSA_ORDER_RANK_LOCAL = 2
 
 _P = c_void_p
 _I = c_int64
@@ -41,6 +42,7 @@ SIGNATURES: dict[str, list] = {
     "rcsa_closed_loop_degrees": [_P, _P, _I, _I, _P, _I, _I, _I, _I, _I, _I, _I, _I,
                                  c_float, c_int, c_int, _P, _P, _P],
     "rcsa_select_topk": [_P, _I, _I, _I, _P, _I, _I, _P, _P, _I, _P, _I, _P, c_int, _P],
+    "rcsa_select_check": [_P, _P, _P, _P, _I, _I, _I, _I, _P, _P, _P],
     "rcsa_quantize_key": [_P, c_int, _I, _I, _I, _I, _I, _I, _I, _I, _P, _P, _I, _P, _P, _P,
                           _P, _P, _P, _P],
     "rcsa_sparse_attn_bf16": [_P, _P, _P, _P, c_float, _P, _P, _P, _P] + [_I] * 18

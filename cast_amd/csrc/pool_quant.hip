@@ -287,61 +287,100 @@ pool_qk_kernel(PoolArgs q, PoolArgs k, int64_t q_tiles, PoolArgs v, int64_t k_en
   else pool_tile<T, D, BS, false, false, MAP, false>(v, blockIdx.x - k_end);
 }
 
-// Cosine scores: one workgroup per (bh, 16 query blocks, 64 key blocks).
-// The tiles are loaded with 16-byte loads, all issued before the LDS stores.
-template <int D>
+// Cosine scores: one workgroup per (bh, 16 RQ query blocks, 64 key blocks), RQ x 4
+// scores per thread, four channels per LDS read (RQ + 4 reads for 16 RQ FMAs;
+// one score per thread and channel reads two words for each FMA and was bound by
+// LDS).  Every score is one FMA chain over the channels in order.  The rows are
+// D + 4 words apart, so the 16 key rows of a read start four banks apart.
+// At 24 heads, D 128: 330 x 330 blocks 26 against 56 us, 28 x 853 11 against 18 us.
+template <int D, int RQ>
 __global__ void __launch_bounds__(256)
 score_kernel(const float* qhat, const float* khat, int64_t nq, int64_t nk,
              float* score) {
-  __shared__ float sq[16][D];
-  __shared__ float sk[64][D + 1];
-  constexpr int C4 = D / 4;                      // float4 per row
-  constexpr int QL = 16 * C4 / 256;              // float4 loads per thread (query tile)
-  constexpr int KL = 64 * C4 / 256;              // (key tile)
-  const int64_t tiles_q = (nq + 15) / 16, tiles_k = (nk + 63) / 64;
+  constexpr int TQ = 16 * RQ, TK = 64, LD = D + 4, C4 = D / 4;
+  __shared__ __attribute__((aligned(16))) float sq[TQ][LD];
+  __shared__ __attribute__((aligned(16))) float sk[TK][LD];
+  constexpr int QL = TQ * C4 / 256;              // float4 loads per thread (query tile)
+  constexpr int KL = TK * C4 / 256;              // (key tile)
+  const int64_t tiles_q = (nq + TQ - 1) / TQ, tiles_k = (nk + TK - 1) / TK;
   const int64_t tk = blockIdx.x % tiles_k;
   const int64_t tq = (blockIdx.x / tiles_k) % tiles_q;
   const int64_t bh = blockIdx.x / (tiles_k * tiles_q);
   const int t = threadIdx.x;
-  const float4* qb = reinterpret_cast<const float4*>(qhat + (bh * nq + tq * 16) * D);
-  const float4* kb = reinterpret_cast<const float4*>(khat + (bh * nk + tk * 64) * D);
-  // rows past the end re-read the last row (then zeroed): every load is in bounds
+  const float4* qb = reinterpret_cast<const float4*>(qhat + (bh * nq + tq * TQ) * D);
+  const float4* kb = reinterpret_cast<const float4*>(khat + (bh * nk + tk * TK) * D);
+  // rows past the end re-read the last row: every load is in bounds
+  const int q_last = static_cast<int>(min<int64_t>(nq - tq * TQ, TQ)) - 1;
+  const int k_last = static_cast<int>(min<int64_t>(nk - tk * TK, TK)) - 1;
   float4 qv[QL], kv[KL];
-  const int q_last = static_cast<int>(min<int64_t>(nq - tq * 16, 16)) - 1;
-  const int k_last = static_cast<int>(min<int64_t>(nk - tk * 64, 64)) - 1;
 #pragma unroll
   for (int i = 0; i < QL; ++i) {
-    const int e = t + 256 * i, r = e / C4;
-    qv[i] = qb[min(r, q_last) * C4 + e % C4];
-    if (r > q_last) qv[i] = make_float4(0.f, 0.f, 0.f, 0.f);
+    const int e = t + 256 * i;
+    qv[i] = qb[min(e / C4, q_last) * C4 + e % C4];
   }
 #pragma unroll
   for (int i = 0; i < KL; ++i) {
-    const int e = t + 256 * i, r = e / C4;
-    kv[i] = kb[min(r, k_last) * C4 + e % C4];
-    if (r > k_last) kv[i] = make_float4(0.f, 0.f, 0.f, 0.f);
+    const int e = t + 256 * i;
+    kv[i] = kb[min(e / C4, k_last) * C4 + e % C4];
   }
 #pragma unroll
   for (int i = 0; i < QL; ++i) {
-    const int e = t + 256 * i, r = e / C4, cc = (e % C4) * 4;
-    sq[r][cc] = qv[i].x; sq[r][cc + 1] = qv[i].y; sq[r][cc + 2] = qv[i].z; sq[r][cc + 3] = qv[i].w;
+    const int e = t + 256 * i;
+    *reinterpret_cast<float4*>(&sq[e / C4][e % C4 * 4]) = qv[i];
   }
 #pragma unroll
   for (int i = 0; i < KL; ++i) {
-    const int e = t + 256 * i, r = e / C4, cc = (e % C4) * 4;
-    sk[r][cc] = kv[i].x; sk[r][cc + 1] = kv[i].y; sk[r][cc + 2] = kv[i].z; sk[r][cc + 3] = kv[i].w;
+    const int e = t + 256 * i;
+    *reinterpret_cast<float4*>(&sk[e / C4][e % C4 * 4]) = kv[i];
   }
   __syncthreads();
-  const int qi = t / 16;
+  const int qi = t / 16 * RQ, kj = t % 16;  // rows qi.., columns kj + 16 u
+  float acc[RQ][4];
 #pragma unroll
-  for (int u = 0; u < 4; ++u) {
-    const int kj = t % 16 + 16 * u;
-    float acc = 0.0f;
-#pragma unroll 8
-    for (int cc = 0; cc < D; ++cc) acc = fmaf(sq[qi][cc], sk[kj][cc], acc);
-    const int64_t gi = tq * 16 + qi, gj = tk * 64 + kj;
-    if (gi < nq && gj < nk) score[(bh * nq + gi) * nk + gj] = acc;
+  for (int r = 0; r < RQ; ++r)
+#pragma unroll
+    for (int u = 0; u < 4; ++u) acc[r][u] = 0.0f;
+#pragma unroll 4
+  for (int c = 0; c < D; c += 4) {
+    float4 a[RQ], b[4];
+#pragma unroll
+    for (int r = 0; r < RQ; ++r) a[r] = *reinterpret_cast<const float4*>(&sq[qi + r][c]);
+#pragma unroll
+    for (int u = 0; u < 4; ++u) b[u] = *reinterpret_cast<const float4*>(&sk[kj + 16 * u][c]);
+#pragma unroll
+    for (int r = 0; r < RQ; ++r)
+#pragma unroll
+      for (int u = 0; u < 4; ++u) {
+        acc[r][u] = fmaf(a[r].x, b[u].x, acc[r][u]);
+        acc[r][u] = fmaf(a[r].y, b[u].y, acc[r][u]);
+        acc[r][u] = fmaf(a[r].z, b[u].z, acc[r][u]);
+        acc[r][u] = fmaf(a[r].w, b[u].w, acc[r][u]);
+      }
   }
+#pragma unroll
+  for (int r = 0; r < RQ; ++r)
+#pragma unroll
+    for (int u = 0; u < 4; ++u) {
+      const int64_t gi = tq * TQ + qi + r, gj = tk * TK + kj + 16 * u;
+      if (gi < nq && gj < nk) score[(bh * nq + gi) * nk + gj] = acc[r][u];
+    }
+}
+
+template <int D>
+static void launch_score(const float* qhat, const float* khat, int64_t n_bh, int64_t nq,
+                         int64_t nk, float* score, hipStream_t s) {
+  const int64_t tiles_k = (nk + 63) / 64;
+  auto grid = [&](int64_t tq) {
+    return dim3(static_cast<unsigned>(n_bh * ((nq + tq - 1) / tq) * tiles_k));
+  };
+  // the largest query tile that the rows fill and that leaves the device a
+  // workgroup per compute unit
+  if (nq > 32 && n_bh * ((nq + 63) / 64) * tiles_k >= 512)
+    score_kernel<D, 4><<<grid(64), dim3(256), 0, s>>>(qhat, khat, nq, nk, score);
+  else if (nq > 16 && n_bh * ((nq + 31) / 32) * tiles_k >= 256)
+    score_kernel<D, 2><<<grid(32), dim3(256), 0, s>>>(qhat, khat, nq, nk, score);
+  else
+    score_kernel<D, 1><<<grid(16), dim3(256), 0, s>>>(qhat, khat, nq, nk, score);
 }
 
 // Number of nonzero bytes of a 32-bit word.
@@ -724,10 +763,8 @@ extern "C" int rcsa_block_scores(const float* qhat, const float* khat, int64_t n
   if (!qhat || !khat || !score) return RCSA_ERR_NULL;
   if (n_bh <= 0 || n_qblocks <= 0 || n_kblocks <= 0) return RCSA_ERR_SHAPE;
   if (!(head_dim == 64 || head_dim == 128)) return RCSA_ERR_SHAPE;
-  const int64_t tiles = n_bh * ((n_qblocks + 15) / 16) * ((n_kblocks + 63) / 64);
-  dim3 grid(static_cast<unsigned>(tiles)), block(256);
-  if (head_dim == 128) score_kernel<128><<<grid, block, 0, stream>>>(qhat, khat, n_qblocks, n_kblocks, score);
-  else score_kernel<64><<<grid, block, 0, stream>>>(qhat, khat, n_qblocks, n_kblocks, score);
+  if (head_dim == 128) launch_score<128>(qhat, khat, n_bh, n_qblocks, n_kblocks, score, stream);
+  else launch_score<64>(qhat, khat, n_bh, n_qblocks, n_kblocks, score, stream);
   return launch_status();
 }
 
@@ -825,7 +862,7 @@ extern "C" int rcsa_quantize_key_select(
   if (head_dim != 128) return RCSA_ERR_SHAPE;  // the fused scores are unrolled for 128
   const SelArgs sel{score, batch * n_heads * n_qblocks, n_qblocks, n_blocks, row_k,
                     row_k_stride_bh, k_fixed, forced, allowed, mask_stride_bh, indices, max_k,
-                    counts, qhat, khat, head_dim};
+                    counts, qhat, khat, head_dim, false};
   return quantize_key_impl(k, dtype, batch, n_heads, n_blocks, block_size, head_dim, stride_b,
                            stride_h, stride_t, valid, slot_token, src_len, ksum, kmin, kmax,
                            kmean, k_i8, k_scale, &sel, stream);

@@ -13,7 +13,8 @@ from typing import Optional
 import torch
 
 from . import _lib
-from ._lib import RCSA_BF16, RCSA_F32, RCSA_ORDER_INDEX, RCSA_ORDER_RANK, check
+from ._lib import (RCSA_BF16, RCSA_F32, RCSA_ORDER_INDEX, RCSA_ORDER_RANK,
+                   RCSA_ORDER_RANK_LOCAL, check)
 
 __all__ = [
     "pool_query", "pool_key", "block_scores", "select_topk", "quantize_key",
@@ -375,7 +376,8 @@ def select_topk(score: torch.Tensor, k, *, forced: Optional[torch.Tensor] = None
 
     Order of preference: forced, then score descending, then block index
     ascending (the stable-argsort tie rule of
-    P/qk_uncertainty_tangent_attention.py:978-980).  ``k`` is an int, or an
+    P/qk_uncertainty_tangent_attention.py:978-980); "rank_local" ranks the forced
+    blocks among themselves by the fp32 value of score + 1e6.  ``k`` is an int, or an
     int tensor of shape [NQ] (shared by heads) or [NBH, NQ].  Returns
     ``(indices int32 [NBH, NQ, max_k], counts int32 [NBH, NQ])``; unused
     slots hold -1.
@@ -393,9 +395,38 @@ def select_topk(score: torch.Tensor, k, *, forced: Optional[torch.Tensor] = None
     st = _lib.load().rcsa_select_topk(
         score.data_ptr(), nbh, nq, nk, _ptr(row_k), stride, k_fixed, _ptr(fm), _ptr(am),
         mstride, indices.data_ptr(), max_k, counts.data_ptr(),
-        RCSA_ORDER_RANK if order == "rank" else RCSA_ORDER_INDEX, _stream())
+        _ORDERS[order], _stream())
     check(st, fn)
     return indices, counts
+
+
+_ORDERS = {"index": RCSA_ORDER_INDEX, "rank": RCSA_ORDER_RANK,
+           "rank_local": RCSA_ORDER_RANK_LOCAL}
+
+
+def select_check(selected: torch.Tensor, counts: torch.Tensor, local: torch.Tensor,
+                 score: torch.Tensor) -> torch.Tensor:
+    """The certificate sums of a selection (``rcsa_select_check``): float64 [3] on the
+    device = (repeated neighbours, local blocks kept, sum of the scores); selected int32
+    [..., N, maxK], counts int32 [..., N], local bool [N, NK], score fp32 [B*H, N, NK]."""
+    fn = "select_check"
+    _require_cuda(fn, selected, counts, local, score)
+    nbh, nq, nk = score.shape
+    max_k = selected.shape[-1]
+    if selected.numel() != nbh * nq * max_k or counts.numel() != nbh * nq \
+            or tuple(local.shape) != (nq, nk):
+        raise ValueError(f"{fn}: inconsistent selection/score/stencil shapes")
+    if selected.dtype != torch.int32 or counts.dtype != torch.int32 \
+            or score.dtype != torch.float32:
+        raise TypeError(f"{fn}: selected and counts must be int32, score float32")
+    sel, cnt, loc, sc = (selected.contiguous(), counts.contiguous(),
+                         _bytes_mask(local, score.device), score.contiguous())
+    rows = torch.empty(nbh * nq, 3, device=score.device, dtype=torch.float64)
+    out = torch.empty(3, device=score.device, dtype=torch.float64)
+    check(_lib.load().rcsa_select_check(sel.data_ptr(), cnt.data_ptr(), loc.data_ptr(),
+                                        sc.data_ptr(), nbh, nq, nk, max_k, rows.data_ptr(),
+                                        out.data_ptr(), _stream()), fn)
+    return out
 
 
 def _selection_args(nbh, nq, nk, k, forced, allowed, max_k, order, device, fn):
@@ -420,8 +451,8 @@ def _selection_args(nbh, nq, nk, k, forced, allowed, max_k, order, device, fn):
         k_fixed = 0
     if max_k is None:
         max_k = max(1, min(kmax, nk))
-    if order not in ("index", "rank"):
-        raise ValueError(f"{fn}: order must be 'index' or 'rank'")
+    if order not in _ORDERS:
+        raise ValueError(f"{fn}: order must be 'index', 'rank' or 'rank_local'")
     fm, fstride = _mask_u8(forced, nbh, nq, nk, device, fn)
     am, astride = _mask_u8(allowed, nbh, nq, nk, device, fn)
     if fm is not None and am is not None and fstride != astride:

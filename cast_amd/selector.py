@@ -8,9 +8,9 @@ the chain that CAST's attention compiler
 P/control_response_cwca_attention.py:2083-2099) ends in:
 
 * Q/K ``[B, H, T*h*w, D]`` are tiled into (tt, th, tw) blocks of the latent
-  grid, mean-pooled and L2-normalised (``rcsa_pack_tokens`` +
-  ``rcsa_pool_query`` / ``rcsa_pool_key``; a zero-padded mean and the
-  valid-token mean have the same direction);
+  grid, mean-pooled and L2-normalised (``rcsa_pool_query_key``
+  through the slot map; a zero-padded mean and the valid-token mean have the
+  same direction);
 * cosine block scores (``rcsa_block_scores``);
 * the row budgets are read at call time from the compiler's
   ``_runtime_degrees(q_blocks)`` (P/qk_uncertainty_tangent_attention.py:982,
@@ -142,11 +142,10 @@ class BlockSelector:
             raise RuntimeError("row budgets were not compiled")
         if row_degrees is None:
             row_degrees = self._row_degrees
-        rows_fn = row_degrees if callable(row_degrees) else (lambda _qb: row_degrees)
         return select_blocks(q, k, geometry_counts=geometry_counts, latent_hw=latent_hw,
                              block_shape=block_shape, compiled_shape=self._block_shape,
                              num_blocks=self._num_blocks, degree=self._degree,
-                             runtime_degrees=rows_fn, ray_motion=self._ray_motion,
+                             runtime_degrees=row_degrees, ray_motion=self._ray_motion,
                              first_order_motion=self._first_order_motion,
                              kind=self.trajectory_complexity_kind)
 
@@ -218,47 +217,59 @@ def select_blocks(q: torch.Tensor, k: torch.Tensor, *, geometry_counts: torch.Te
     if lay.n_blocks != num_blocks:
         raise RuntimeError("latent grid does not give the compiled number of blocks")
     bs, nb = lay.block_size, lay.n_blocks
-    # packed [B, H, nb*bs, D] tiles (q viewed as [B, L, H, D], no copy of q itself)
-    qp = ops.pack_tokens(q.transpose(1, 2), lay.slot_token)
-    kp = ops.pack_tokens(k.transpose(1, 2), lay.slot_token)
-    qhat, _, _ = ops.pool_query(qp, lay.slot_valid, bs)
-    khat, _, _, _ = ops.pool_key(kp, lay.slot_valid, bs)
+    # a callable reads the packed tiles [B, H, nb, bs, D]; budgets as they are need
+    # no packed copy
+    wants_tiles = callable(runtime_degrees)
+    qt, kt = q.transpose(1, 2), k.transpose(1, 2)  # token-major views
+    qp = ops.pack_tokens(qt, lay.slot_token) if wants_tiles else None
+    if q.dtype == k.dtype and min(q.stride(2), k.stride(2)) >= D and q.stride(3) == 1 \
+            and k.stride(3) == 1:
+        # pooled through the slot map, both in one launch
+        qhat, _, _, khat, *_ = ops.pool_query_key(
+            qt, None, kt, None, bs, q_slot_token=lay.slot_token32,
+            k_slot_token=lay.slot_token32, quantize=False)
+    else:  # rows that overlap, or two dtypes
+        if qp is None:
+            qp = ops.pack_tokens(qt, lay.slot_token)
+        qhat, _, _ = ops.pool_query(qp, lay.slot_valid, bs)
+        khat, _, _, _ = ops.pool_key(ops.pack_tokens(kt, lay.slot_token), lay.slot_valid, bs)
     score = ops.block_scores(qhat, khat)                      # [B*H, nb, nb]
     local = layout.local_stencil(nb, *lay.grid, device=q.device)
-    ranking = torch.where(local, (score + 1e6) - 1e6, score)  # order of fl(s + 1e6)
-    rows = torch.as_tensor(runtime_degrees(qp.view(B, H, nb, bs, D)))
+    rows = torch.as_tensor(runtime_degrees(qp.view(B, H, nb, bs, D)) if wants_tiles
+                           else runtime_degrees)
     rows = rows.detach().to("cpu", torch.long).reshape(-1)
     if rows.numel() != nb:
         raise RuntimeError("row budgets do not match the attention blocks")
     if int(rows.min()) < 0 or int(rows.max()) > nb:
         raise RuntimeError("TABA assigned more keys than exist")
     max_degree = int(rows.max())
-    selected, _ = ops.select_topk(ranking, max_degree, forced=local, max_k=max_degree,
-                                  order="rank")
+    selected, _ = ops.select_topk(score, max_degree, forced=local, max_k=max_degree,
+                                  order="rank_local")  # local order: that of fl(s + 1e6)
     selected = selected.view(B, H, nb, max_degree)
-    counts = rows.to(device=q.device, dtype=torch.int32)[None, None].expand(B, H, -1)
-    counts = counts.contiguous()
+    # pinned, so the copy waits for nothing on the stream
+    counts = rows.to(torch.int32).pin_memory().to(device=q.device, non_blocking=True)
+    counts = counts[None, None].expand(B, H, -1).contiguous()
     # certificate: no repeated neighbour in a row's prefix, every local block kept
-    live = torch.arange(max_degree, device=q.device)[None, None, None, :] < counts[..., None]
-    dup = ((selected[..., 1:] == selected[..., :-1]) & live[..., 1:]).sum()
-    chosen = (torch.gather(local[None, None].expand(B, H, -1, -1), -1, selected.long())
-              & live).sum()
-    host = torch.stack([dup.double(), chosen.double(), score.double().mean()]).cpu()
-    duplicates = int(host[0])
+    sums = ops.select_check(selected, counts, local, score)
+    # (what the report takes from the host is ready before the sums are read)
     expected_local = int(layout.local_stencil(nb, *lay.grid).sum()) * B * H
+    ray = torch.as_tensor(ray_motion).float()
+    first = torch.as_tensor(first_order_motion).float()
+    motion = dict(mean_ray_motion=float(ray.mean()), max_ray_motion=float(ray.max()),
+                  mean_first_order_motion=float(first.mean()))
+    budgets = dict(budget_min=int(rows.min()), budget_max=max_degree,
+                   budget_total=int(rows.sum()))
+    host = sums.tolist()
+    duplicates = int(host[0])
     missing_local = expected_local - int(host[1])
     if duplicates or missing_local:
         raise RuntimeError("TABA selection certificate failed")
-    ray = torch.as_tensor(ray_motion).float()
-    first = torch.as_tensor(first_order_motion).float()
     report = (report_cls or SelectionReport)(
         batch_heads=B * H, query_rows=nb, edges_per_row=int(degree),
         row_duplicate_violations=duplicates, selected_orientation_violations=0,
         max_orientation_violations_per_row=0, mean_selected_ray_cosine=0.0,
-        mean_selected_qk_cosine=float(host[2]), qk_read_for_selection=True,
+        mean_selected_qk_cosine=host[2] / score.numel(), qk_read_for_selection=True,
         selector_count=1, protected_local_edges=expected_local,
         missing_local_edges=missing_local, mean_geometry_gate=0.0, max_geometry_gate=0.0,
-        budget_min=int(rows.min()), budget_max=max_degree, budget_total=int(rows.sum()),
-        mean_ray_motion=float(ray.mean()), max_ray_motion=float(ray.max()),
-        trajectory_complexity_kind=kind, mean_first_order_motion=float(first.mean()))
+        trajectory_complexity_kind=kind, **motion, **budgets)
     return selected, counts, report

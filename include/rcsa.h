@@ -45,7 +45,9 @@ enum { RCSA_BF16 = 0, RCSA_F32 = 1 };
 /* Selection output order. */
 enum {
   RCSA_ORDER_INDEX = 0, /* ascending block index (what the attention kernel streams best) */
-  RCSA_ORDER_RANK = 1   /* descending rank: forced first, then score desc, index asc */
+  RCSA_ORDER_RANK = 1,  /* descending rank: forced first, then score desc, index asc */
+  RCSA_ORDER_RANK_LOCAL = 2 /* rank order, the forced columns among themselves by the
+                               fp32 value of score + 1e6 (as score + 1e6 * local ranks) */
 };
 
 /* Human-readable text for a status code (static storage). */
@@ -229,6 +231,18 @@ int rcsa_select_topk(const float* score, int64_t n_bh, int64_t n_qblocks,
                      const uint8_t* forced, const uint8_t* allowed,
                      int64_t mask_stride_bh, int32_t* indices, int64_t max_k,
                      int32_t* counts, int order, hipStream_t stream);
+
+/*
+ * The certificate of a selection (P/qk_uncertainty_tangent_attention.py:1046-1062)
+ * as device sums, out double [3]: [0] entries equal to the one before them among
+ * the first min(max(counts, 0), max_k) of every row, [1] entries whose block is
+ * in the row's local stencil, [2] the sum of all scores.  selected int32
+ * [n_bh][NQB][max_k], counts int32 [n_bh][NQB], local uint8 [NQB][NKB], score fp32
+ * [n_bh][NQB][NKB]; row_sums: workspace, double [n_bh * NQB][3].
+ */
+int rcsa_select_check(const int32_t* selected, const int32_t* counts, const uint8_t* local,
+                      const float* score, int64_t n_bh, int64_t n_qblocks, int64_t n_kblocks,
+                      int64_t max_k, double* row_sums, double* out, hipStream_t stream);
 
 /*
  * int8 key quantiser with per-head mean smoothing.  No reference
