@@ -50,25 +50,6 @@ class _DeviceStats:
                 "std": float(v.std(unbiased=False))}
 
 
-def _time_cells(values: torch.Tensor, local, compact_group: int, source_group: int,
-                offset: int) -> torch.Tensor:
-    """``_compact_time_cells`` (P/control_response_cwca_attention.py:1123-1163) on the
-    values' device with the frames on the host: frame f >= offset reads tile
-    (f - offset) // source_group, earlier frames read 0, and each run of
-    compact_group frames is averaged.  No host read-back."""
-    rows = []
-    for lo in range(0, len(local), compact_group):
-        group = local[lo:lo + compact_group]
-        tiles = [(f - offset) // source_group for f in group if f >= offset]
-        if tiles:
-            idx = torch.tensor(tiles, dtype=torch.long).pin_memory().to(values.device,
-                                                                       non_blocking=True)
-            rows.append(values.index_select(0, idx).sum(0) / float(len(group)))
-        else:
-            rows.append(torch.zeros(values.shape[1], device=values.device, dtype=values.dtype))
-    return torch.stack(rows)
-
-
 class DeviceClosedLoopBudget:
     """Mixin: put it before ``MatrixClosedLoopCWCAAttentionCompiler`` in the bases."""
 
@@ -106,9 +87,6 @@ class DeviceClosedLoopBudget:
             raise RuntimeError("compact Closed-Loop degree layout differs from packed rows")
         dev = curvature.device if curvature.is_cuda else torch.device("cuda")
         curv = curvature.to(device=dev, dtype=torch.float32)
-        eps = torch.finfo(torch.float32).eps
-        normalized = curv / curv.mean(dim=0, keepdim=True).clamp_min(eps)
-        compact_curvature = _time_cells(normalized, local, group, source_group, offset)
         response = None
         response_weight = 0.0
         feedback = self.feedback_form
@@ -130,19 +108,21 @@ class DeviceClosedLoopBudget:
             source = (f"compact_{feedback}_curvature_control_response_"
                       f"lambda_{self.response_weight:g}")
             previous = layer_index - 1
-            response_stats = _DeviceStats(
-                _time_cells(response, local, group, source_group, offset))
-        degrees, status = ops.closed_loop_degrees(
+        layer = ops.closed_loop_layer(
             curv, local, current_temporal_offset=offset, source_group=source_group,
             compact_group=group, mean_degree=int(mean_degree), base_degree=int(base_degree),
             total_blocks=int(total_blocks), memory_blocks=int(memory_blocks),
             response=response, response_weight=response_weight, feedback_form=feedback,
-            fixed_query_budget=fixed, check_status=False)
+            fixed_query_budget=fixed, fn="closed_loop_degrees")
+        if response is not None:
+            response_stats = _DeviceStats(layer.response_cells)
         pending = getattr(self, "_rcsa_pending_status", None)
         if pending is None:
             pending = self._rcsa_pending_status = []
-        pending.append(status)
-        current = degrees[int(memory_blocks):].view(cells, spatial).long()
+        pending.append(layer.status)
+        # (the layer's degrees, memory rows included, ride along for the caller)
+        current = layer.degrees64[int(memory_blocks):].view(cells, spatial)
+        current.rcsa_layer = layer
         worldline = cells * int(mean_degree)
         current_edges = cells * spatial * int(mean_degree)
         metadata = {
@@ -157,7 +137,7 @@ class DeviceClosedLoopBudget:
             "compact_time_cells": cells,
             "spatial_worldlines": spatial,
             "response": response_stats,
-            "curvature": _DeviceStats(compact_curvature),
+            "curvature": _DeviceStats(layer.curvature_cells),
             "current_worldline_budget": worldline,
             "current_edge_budget": current_edges,
             "global_edge_budget": int(memory_blocks) * int(mean_degree) + current_edges,
@@ -171,8 +151,11 @@ class DeviceClosedLoopBudget:
                               local_support_preserved: bool, native_qk_topk: bool) -> None:
         record = dict(metadata)
         d = degrees.detach()
+        layer = getattr(degrees, "rcsa_layer", None)
+        k_min, k_max, k_mean = ((d.min(), d.max(), d.float().mean()) if layer is None
+                                else (*layer.min_max.unbind(), layer.mean))
         record.update({
-            "k_min": d.min(), "k_max": d.max(), "k_mean": d.float().mean(),
+            "k_min": k_min, "k_max": k_max, "k_mean": k_mean,
             "budget_exact": metadata["global_edge_budget"] == metadata["reference_edge_budget"],
             "local_support_preserved": bool(local_support_preserved),
             "native_qk_topk": bool(native_qk_topk),

@@ -181,6 +181,12 @@ struct ClosedLoopArgs {
   int use_response, fixed_budget;
   int32_t* degrees;        // [total_blocks]
   int32_t* status;         // [1]
+  // what the layer's records keep (nullable)
+  int64_t* degrees64;      // [total_blocks]
+  float* curvature_cells;  // [cells][spatial]
+  float* response_cells;   // [cells][spatial], with a response
+  int64_t* min_max;        // [2] of the degrees
+  float* mean;             // [1]
 };
 
 // One workgroup.  Thread t owns spatial worldlines t, t + 256, ...: the
@@ -233,8 +239,10 @@ __global__ void __launch_bounds__(kBudgetThreads) closed_loop_kernel(ClosedLoopA
       const float cnt = static_cast<float>(f1 - f0);
       const float curv = cs / cnt;
       float signal = curv;
+      if (a.curvature_cells) a.curvature_cells[c * S + sp] = curv;
       if (a.use_response) {
         const float resp = rs / cnt;
+        if (a.response_cells) a.response_cells[c * S + sp] = resp;
         if (a.feedback == 0) {
           signal = curv + a.response_weight * resp;
         } else {
@@ -319,7 +327,33 @@ __global__ void __launch_bounds__(kBudgetThreads) closed_loop_kernel(ClosedLoopA
       }
     missing -= n_room < missing ? n_room : missing;
   }
-  for (int i = lo; i < hi; ++i) a.degrees[i] = s_deg[i];
+  int least = INT32_MAX, most = INT32_MIN, sum_part = 0;
+  for (int i = lo; i < hi; ++i) {
+    const int d = s_deg[i];
+    a.degrees[i] = d;
+    if (a.degrees64) a.degrees64[i] = d;
+    least = d < least ? d : least;
+    most = d > most ? d : most;
+    sum_part += d;
+  }
+  if (a.min_max || a.mean) {
+    int sum = 0;
+    block_exclusive_scan(sum_part, s_i, &sum);
+    __shared__ int s_min, s_max;
+    if (t == 0) {
+      s_min = INT32_MAX;
+      s_max = INT32_MIN;
+    }
+    __syncthreads();
+    atomicMin(&s_min, least);
+    atomicMax(&s_max, most);
+    __syncthreads();
+    if (t == 0 && a.min_max) {
+      a.min_max[0] = s_min;
+      a.min_max[1] = s_max;
+    }
+    if (t == 0 && a.mean) a.mean[0] = static_cast<float>(sum) / static_cast<float>(n_blocks);
+  }
   __syncthreads();
   if (t == 0) a.status[0] = s_status;
 }
@@ -348,12 +382,14 @@ extern "C" int rcsa_row_budgets(const float* weights, int64_t n_sections, int64_
   return launch_status();
 }
 
-extern "C" int rcsa_closed_loop_degrees(
+extern "C" int rcsa_closed_loop_layer(
     const float* curvature, const float* response, int64_t t_src, int64_t spatial,
     const int32_t* frames, int64_t n_frames, int64_t current_temporal_offset,
     int64_t source_group, int64_t compact_group, int64_t mean_degree, int64_t base_degree,
     int64_t total_blocks, int64_t memory_blocks, float response_weight, int feedback_form,
-    int fixed_query_budget, int32_t* degrees, int32_t* status, hipStream_t stream) {
+    int fixed_query_budget, int32_t* degrees, int32_t* status, int64_t* degrees64,
+    float* curvature_cells, float* response_cells, int64_t* min_max, float* mean,
+    hipStream_t stream) {
   if (!curvature || !frames || !degrees || !status) return RCSA_ERR_NULL;
   if (t_src <= 0 || spatial <= 0 || spatial > kClMaxSpatial || n_frames <= 0 ||
       n_frames > kClMaxFrames || source_group <= 0 || compact_group <= 0 ||
@@ -386,6 +422,24 @@ extern "C" int rcsa_closed_loop_degrees(
   a.fixed_budget = fixed_query_budget != 0;
   a.degrees = degrees;
   a.status = status;
+  a.degrees64 = degrees64;
+  a.curvature_cells = curvature_cells;
+  a.response_cells = response_cells;
+  a.min_max = min_max;
+  a.mean = mean;
   closed_loop_kernel<<<dim3(1), dim3(kBudgetThreads), 0, stream>>>(a);
   return launch_status();
+}
+
+extern "C" int rcsa_closed_loop_degrees(
+    const float* curvature, const float* response, int64_t t_src, int64_t spatial,
+    const int32_t* frames, int64_t n_frames, int64_t current_temporal_offset,
+    int64_t source_group, int64_t compact_group, int64_t mean_degree, int64_t base_degree,
+    int64_t total_blocks, int64_t memory_blocks, float response_weight, int feedback_form,
+    int fixed_query_budget, int32_t* degrees, int32_t* status, hipStream_t stream) {
+  return rcsa_closed_loop_layer(curvature, response, t_src, spatial, frames, n_frames,
+                                current_temporal_offset, source_group, compact_group, mean_degree,
+                                base_degree, total_blocks, memory_blocks, response_weight,
+                                feedback_form, fixed_query_budget, degrees, status, nullptr,
+                                nullptr, nullptr, nullptr, nullptr, stream);
 }

@@ -8,7 +8,7 @@ from __future__ import annotations
 
 import ctypes
 import math
-from typing import Optional
+from typing import NamedTuple, Optional
 
 import torch
 
@@ -302,7 +302,42 @@ def closed_loop_degrees(curvature: torch.Tensor, frames, *, current_temporal_off
     device status word is read back once and a breach raises ``RuntimeError``
     with the reference's message; otherwise ``(degrees, status)`` is returned
     and nothing is read back."""
-    fn = "closed_loop_degrees"
+    res = closed_loop_layer(
+        curvature, frames, current_temporal_offset=current_temporal_offset,
+        source_group=source_group, compact_group=compact_group, mean_degree=mean_degree,
+        base_degree=base_degree, total_blocks=total_blocks, memory_blocks=memory_blocks,
+        response=response, response_weight=response_weight, feedback_form=feedback_form,
+        fixed_query_budget=fixed_query_budget, records=False, fn="closed_loop_degrees")
+    degrees, status = res.degrees, res.status
+    if not check_status:
+        return degrees, status
+    code = int(status.item())
+    for bit, msg in _CL_ERRORS:
+        if code & bit:
+            raise RuntimeError(msg)
+    return degrees
+
+
+class ClosedLoopLayer(NamedTuple):
+    """A compact layer's degrees and what its records keep, all on the device."""
+    degrees: torch.Tensor                       # int32 [total_blocks]
+    status: torch.Tensor                        # int32 [1]
+    degrees64: Optional[torch.Tensor]           # int64 [total_blocks]
+    curvature_cells: Optional[torch.Tensor]     # fp32 [cells, S]
+    response_cells: Optional[torch.Tensor]      # fp32 [cells, S]
+    min_max: Optional[torch.Tensor]             # int64 [2]
+    mean: Optional[torch.Tensor]                # fp32 []
+
+
+def closed_loop_layer(curvature: torch.Tensor, frames, *, current_temporal_offset: int,
+                      source_group: int, compact_group: int, mean_degree: int,
+                      base_degree: int, total_blocks: int, memory_blocks: int,
+                      response: Optional[torch.Tensor] = None, response_weight: float = 0.0,
+                      feedback_form: str = "additive", fixed_query_budget: bool = False,
+                      records: bool = True, fn: str = "closed_loop_layer") -> ClosedLoopLayer:
+    """:func:`closed_loop_degrees` without the status check, and (``records``) the int64
+    degrees, the time cells and the degrees' statistics from the same launch
+    (``rcsa_closed_loop_layer``); nothing is read back."""
     _require_cuda(fn, curvature)
     dev = curvature.device
     if curvature.dtype != torch.float32 or curvature.ndim != 2:
@@ -321,20 +356,23 @@ def closed_loop_degrees(curvature: torch.Tensor, frames, *, current_temporal_off
     degrees = torch.empty(int(total_blocks), device=dev, dtype=torch.int32)
     status = torch.empty(1, device=dev, dtype=torch.int32)
     t_src, spatial = curvature.shape
-    st = _lib.load().rcsa_closed_loop_degrees(
+    deg64 = curv_cells = resp_cells = min_max = mean = None
+    if records:
+        cells = -(-fr.numel() // int(compact_group))
+        deg64 = torch.empty(int(total_blocks), device=dev, dtype=torch.int64)
+        curv_cells = torch.empty(cells, spatial, device=dev, dtype=torch.float32)
+        if response is not None and response_weight != 0.0:
+            resp_cells = torch.empty_like(curv_cells)
+        min_max = torch.empty(2, device=dev, dtype=torch.int64)
+        mean = torch.empty((), device=dev, dtype=torch.float32)
+    check(_lib.load().rcsa_closed_loop_layer(
         curvature.data_ptr(), _ptr(response), t_src, spatial, fr.data_ptr(), fr.numel(),
         int(current_temporal_offset), int(source_group), int(compact_group), int(mean_degree),
         int(base_degree), int(total_blocks), int(memory_blocks), float(response_weight),
         _CL_FEEDBACK[feedback_form], int(bool(fixed_query_budget)), degrees.data_ptr(),
-        status.data_ptr(), _stream())
-    check(st, fn)
-    if not check_status:
-        return degrees, status
-    code = int(status.item())
-    for bit, msg in _CL_ERRORS:
-        if code & bit:
-            raise RuntimeError(msg)
-    return degrees
+        status.data_ptr(), _ptr(deg64), _ptr(curv_cells), _ptr(resp_cells), _ptr(min_max),
+        _ptr(mean), _stream()), fn)
+    return ClosedLoopLayer(degrees, status, deg64, curv_cells, resp_cells, min_max, mean)
 
 
 def block_scores(qhat: torch.Tensor, khat: torch.Tensor) -> torch.Tensor:

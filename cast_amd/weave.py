@@ -231,7 +231,7 @@ def compact_cwca_attention(weave, module: Any, q: torch.Tensor, k: torch.Tensor,
     current_blocks = blocks - memory_blocks
     active_current_values = tuple(int(x) for x in layout.active_frame_values
                                   if int(x) >= int(layout.memory_temporal))
-    degrees = torch.full((blocks,), mean_degree, device=dev, dtype=torch.long)
+    degrees = row_k = layer = None
     width = mean_degree  # a bound of every row's degree, known on the host
     metadata = None
     host_degrees = provider is None
@@ -248,14 +248,25 @@ def compact_cwca_attention(weave, module: Any, q: torch.Tensor, k: torch.Tensor,
                 total_blocks=blocks, memory_blocks=memory_blocks)
             if int(current.numel()) != current_blocks:
                 raise RuntimeError("compact Closed-Loop degree layout differs from packed rows")
-            degrees[memory_blocks:] = current.reshape(-1).to(device=dev, dtype=torch.long)
+            layer = getattr(current, "rcsa_layer", None)
+            if layer is not None and layer.degrees.device == dev:
+                # the whole layer's rows, memory ones at mean_degree, from one launch
+                degrees, row_k = layer.degrees64, layer.degrees
+                degrees.rcsa_layer = layer
+            else:
+                layer = None
+                degrees = torch.full((blocks,), mean_degree, device=dev, dtype=torch.long)
+                degrees[memory_blocks:] = current.reshape(-1).to(device=dev, dtype=torch.long)
             # every row keeps base, and a worldline's cells share cells * mean edges
             width = max(mean_degree, min(blocks, base + cells * (mean_degree - base)))
         else:
+            degrees = torch.full((blocks,), mean_degree, device=dev, dtype=torch.long)
             active_local = torch.tensor(active_current_values, dtype=torch.long) - \
                 int(layout.memory_temporal)
             _curvature_degrees(weave, degrees, layout, blocks, memory_blocks, spatial, tt,
                                mean_degree, base, active_local, current_frames)
+    if degrees is None:
+        degrees = torch.full((blocks,), mean_degree, device=dev, dtype=torch.long)
     if host_degrees:
         _saturate(degrees, blocks, mean_degree)
         width = int(degrees.max().item())
@@ -313,13 +324,16 @@ def compact_cwca_attention(weave, module: Any, q: torch.Tensor, k: torch.Tensor,
         kq = (q_i8, q_scale, k_i8, k_scale)
 
     # ---- top-k at each row's degree, local blocks first (:5829-5832) ----
-    row_k = degrees.to(torch.int32)
+    if row_k is None:
+        row_k = degrees.to(torch.int32)
     # only the router reads the rank order; the attention takes ascending lists
     ordered = route != "refine"
     indices, _ = ops.select_topk(score, row_k, forced=local, max_k=width,
                                  order="index" if ordered else "rank")
     selected = indices.view(B, H, blocks, width)
-    counts = row_k[None, None].expand(B, H, -1).contiguous()
+    counts = row_k[None, None].expand(B, H, -1)
+    if not ordered:  # the router's own kernels read it whole
+        counts = counts.contiguous()
 
     routing_record: Optional[dict] = None
     if route == "bypass":
@@ -380,8 +394,8 @@ def compact_cwca_attention(weave, module: Any, q: torch.Tensor, k: torch.Tensor,
         "compact_blocks": blocks,
         "requested_density": weave.sparse_density,
         "mean_degree": mean_f,
-        "minimum_degree": degrees.min(),
-        "maximum_degree": degrees.max(),
+        "minimum_degree": degrees.min() if layer is None else layer.min_max[0],
+        "maximum_degree": degrees.max() if layer is None else layer.min_max[1],
         "edge_budget": edges,
         "effective_density": edges / float(blocks * blocks),
         "empty_blocks": 0,

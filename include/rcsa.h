@@ -181,6 +181,19 @@ int rcsa_closed_loop_degrees(const float* curvature, const float* response, int6
                              int64_t total_blocks, int64_t memory_blocks, float response_weight,
                              int feedback_form, int fixed_query_budget, int32_t* degrees,
                              int32_t* status, hipStream_t stream);
+/* The same with what a layer's records keep, from the same launch, each nullable:
+ * degrees64 [total_blocks] (the degrees as int64), curvature_cells and response_cells
+ * [cells][spatial] (the compact time cells of the normalised curvature and, with a
+ * response that counts, of the response), min_max [2] and mean [1] of the degrees. */
+int rcsa_closed_loop_layer(const float* curvature, const float* response, int64_t t_src,
+                           int64_t spatial, const int32_t* frames, int64_t n_frames,
+                           int64_t current_temporal_offset, int64_t source_group,
+                           int64_t compact_group, int64_t mean_degree, int64_t base_degree,
+                           int64_t total_blocks, int64_t memory_blocks, float response_weight,
+                           int feedback_form, int fixed_query_budget, int32_t* degrees,
+                           int32_t* status, int64_t* degrees64, float* curvature_cells,
+                           float* response_cells, int64_t* min_max, float* mean,
+                           hipStream_t stream);
 
 /*
  * Per-row key-block budgets on the device, so no budget is read back to the

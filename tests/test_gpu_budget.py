@@ -156,3 +156,34 @@ def test_closed_loop_status_words():
         ops.closed_loop_degrees(c, frames, **bad)
     with pytest.raises(RuntimeError, match="exhausted key capacity"):
         orc.closed_loop_degrees(curv, frames, **bad)
+
+
+@pytest.mark.parametrize("frames,spatial,feedback", [(1, 30, "additive"), (17, 30, "centered_inverse"),
+                                                     (9, 257, "centered_multiplicative")])
+def test_closed_loop_layer_records(dev, frames, spatial, feedback):
+    """The records of the layer's launch: its degrees as int64, their least, largest and
+    mean, and the time cells (fp32 sums of at most four terms: 2^-21 relative)."""
+    from cast_amd import ops
+    g = torch.Generator().manual_seed(frames)
+    group, tiles, offset, memory = 4, 8, 2, 60
+    cells = -(-frames // group)
+    curv = torch.rand(tiles, spatial, generator=g) + 0.05
+    resp = torch.rand(tiles, spatial, generator=g) * 2
+    total = memory + cells * spatial
+    kw = dict(current_temporal_offset=offset, source_group=4, compact_group=group,
+              mean_degree=20, base_degree=16, total_blocks=total, memory_blocks=memory,
+              response=resp.to(dev), response_weight=0.5, feedback_form=feedback)
+    lay = ops.closed_loop_layer(curv.to(dev), list(range(frames)), **kw)
+    deg = ops.closed_loop_degrees(curv.to(dev), list(range(frames)), **kw)
+    assert torch.equal(lay.degrees, deg) and torch.equal(lay.degrees64, deg.long())
+    assert lay.min_max.tolist() == [int(deg.min()), int(deg.max())]
+    assert abs(float(lay.mean) - float(deg.double().mean())) <= 1e-5
+    norm = curv.double() / curv.double().mean(0)
+    for got, src in ((lay.curvature_cells, norm), (lay.response_cells, resp.double())):
+        want = torch.zeros(cells, spatial, dtype=torch.float64)
+        for c in range(cells):
+            part = range(c * group, min(frames, (c + 1) * group))
+            for f in part:
+                if f >= offset:
+                    want[c] += src[(f - offset) // 4] / len(part)
+        torch.testing.assert_close(got.cpu().double(), want, rtol=2.0 ** -20, atol=1e-9)
