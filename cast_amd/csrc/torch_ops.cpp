@@ -8,8 +8,8 @@
 // (status N)") on a non-zero status, as the reference's wrappers raise on a
 // bad layout.  Every tensor is checked to span the elements the call's dims
 // and strides reach, so no argument combination makes a kernel read or write
-// past the tensors it was given.  Nothing here allocates device memory or
-// synchronises.
+// past the tensors it was given.  Nothing here synchronises, and nothing but
+// layer_call, which allocates its outputs, allocates device memory.
 //
 // The C ABI is bound at load time (rcsa::bind_library) from the library the
 // Python side loaded, so one librcsa.so serves both the ctypes binding and
@@ -21,6 +21,7 @@
 #include <string>
 #include <vector>
 
+#include <ATen/ATen.h>
 #include <c10/hip/HIPGuard.h>
 #include <c10/hip/HIPStream.h>
 #include <hip/hip_runtime_api.h>
@@ -39,6 +40,11 @@ struct Api {
   decltype(&rcsa_quantize_rows_int8) quantize_rows_int8 = nullptr;
   decltype(&rcsa_int8_linear) int8_linear = nullptr;
   decltype(&rcsa_int8_linear_group) int8_linear_group = nullptr;
+  decltype(&rcsa_block_scores) block_scores = nullptr;
+  decltype(&rcsa_select_topk) select_topk = nullptr;
+  decltype(&rcsa_quantize_key) quantize_key = nullptr;
+  decltype(&rcsa_attn_split_plan) attn_split_plan = nullptr;
+  decltype(&rcsa_attn_workspace_bytes) attn_workspace_bytes = nullptr;
 };
 
 std::mutex g_mu;
@@ -65,6 +71,11 @@ void bind_library(const std::string& path) {
   bind_one(h, "rcsa_quantize_rows_int8", api.quantize_rows_int8);
   bind_one(h, "rcsa_int8_linear", api.int8_linear);
   bind_one(h, "rcsa_int8_linear_group", api.int8_linear_group);
+  bind_one(h, "rcsa_block_scores", api.block_scores);
+  bind_one(h, "rcsa_select_topk", api.select_topk);
+  bind_one(h, "rcsa_quantize_key", api.quantize_key);
+  bind_one(h, "rcsa_attn_split_plan", api.attn_split_plan);
+  bind_one(h, "rcsa_attn_workspace_bytes", api.attn_workspace_bytes);
   g_api = api;
   g_bound = true;
 }
@@ -563,6 +574,159 @@ void int8_linear_group(const at::Tensor& x_i8, const at::Tensor& x_scale, at::Te
                                           dt == at::kFloat, M, K, l.stream));
 }
 
+// The layer call of cast_amd/pipeline.py (rcsa_attention) in one op: its launches
+// in stream order on one stream, its outputs allocated here.  A call of a few
+// blocks is bound by the host work between its launches (4 heads x 4 query blocks
+// x 12 key blocks, fp32, int8 Q/K: 54 us a call against 176 us from Python).
+// q, k, v: packed [B, H, L, D], or with both slot maps token-major [B, L, H, D].
+// Returns out, indices, counts, score, qhat, khat, k_mask, then with int8 q_i8,
+// q_scale, k_i8, k_scale, kmean, then with return_lse the LSE.
+std::vector<at::Tensor> layer_call(
+    const at::Tensor& q, const at::Tensor& k, const at::Tensor& v,
+    const c10::optional<at::Tensor>& q_valid, const c10::optional<at::Tensor>& k_valid,
+    int64_t bs, const c10::optional<at::Tensor>& row_k, int64_t row_k_stride_bh, int64_t k_fixed,
+    int64_t max_k, const c10::optional<at::Tensor>& forced,
+    const c10::optional<at::Tensor>& allowed, int64_t mask_stride_bh, bool int8, double sm_scale,
+    bool return_lse, int64_t n_split, const c10::optional<at::Tensor>& q_slot,
+    const c10::optional<at::Tensor>& k_slot) {
+  const char* op = "rcsa_attention";
+  const Api& a = api(op);
+  int dev = -1;
+  for (const auto* t : {&q, &k, &v}) on_device(op, dev, *t, "q, k or v");
+  for (const auto* t : {&q_valid, &k_valid, &row_k, &forced, &allowed, &q_slot, &k_slot})
+    on_device(op, dev, *t, "a mask, budget or slot map");
+  const bool map = q_slot.has_value();
+  TORCH_CHECK(map == k_slot.has_value(), op, ": give both slot maps or neither");
+  for (const auto* t : {&q, &k, &v})
+    TORCH_CHECK(t->dim() == 4 && t->stride(3) == 1, op,
+                ": q, k and v must be 4-D with a contiguous last dim");
+  TORCH_CHECK(v.sizes() == k.sizes(), op, ": k and v must have one shape");
+  const int th = map ? 2 : 1, tl = map ? 1 : 2;  // the head and token dims
+  const int64_t B = q.size(0), H = q.size(th), D = q.size(3);
+  TORCH_CHECK(k.size(0) == B && k.size(th) == H && k.size(3) == D, op,
+              ": q and k differ in B, H or D");
+  TORCH_CHECK(bs > 0, op, ": block_size must be positive");
+  const int64_t Lq = map ? q_slot->numel() : q.size(2), Lk = map ? k_slot->numel() : k.size(2);
+  TORCH_CHECK(Lq > 0 && Lk > 0 && Lq % bs == 0 && Lk % bs == 0, op,
+              ": whole blocks of queries and keys");
+  TORCH_CHECK(!map || (D == 128 && bs == 128 && v.scalar_type() == at::kBFloat16), op,
+              ": gathered sources need D 128, 128-token blocks and bf16 values");
+  const int64_t nq = Lq / bs, nk = Lk / bs, nbh = B * H;
+  const at::ScalarType dt = q.scalar_type();
+  TORCH_CHECK((dt == at::kBFloat16 || dt == at::kFloat) && k.scalar_type() == dt, op,
+              ": q and k must share bfloat16 or float32");
+  const int code = dt == at::kBFloat16 ? RCSA_BF16 : RCSA_F32;
+  want_bytes(op, q_valid, "q_valid");
+  want_bytes(op, k_valid, "k_valid");
+  want_bytes(op, forced, "forced");
+  want_bytes(op, allowed, "allowed");
+  want(op, row_k, at::kInt, "row_k");
+  want(op, q_slot, at::kInt, "q_slot");
+  want(op, k_slot, at::kInt, "k_slot");
+  TORCH_CHECK(max_k > 0 && mask_stride_bh >= 0 && row_k_stride_bh >= 0, op,
+              ": max_k must be positive, strides not negative");
+  want_numel(op, q_valid, Lq, "q_valid");
+  want_numel(op, k_valid, Lk, "k_valid");
+  want_numel(op, forced, (nbh - 1) * mask_stride_bh + nq * nk, "forced");
+  want_numel(op, allowed, (nbh - 1) * mask_stride_bh + nq * nk, "allowed");
+  want_numel(op, row_k, (nbh - 1) * row_k_stride_bh + nq, "row_k");
+  const Launch l(device_of(op, dev));
+  const auto f32 = q.options().dtype(at::kFloat), i32 = q.options().dtype(at::kInt),
+             i8 = q.options().dtype(at::kChar), b16 = q.options().dtype(at::kBFloat16);
+  const at::Tensor qhat = at::empty({nbh, nq, D}, f32), khat = at::empty({nbh, nk, D}, f32);
+  const at::Tensor mask = at::empty({nk, bs / 32}, i32);
+  at::Tensor q_i8, q_scale, k_i8, k_scale, kmean, stats;
+  if (int8) {
+    q_i8 = at::empty({B, H, Lq, D}, i8);
+    q_scale = at::empty({nbh, nq}, f32);
+    k_i8 = at::empty({B, H, Lk, D}, i8);
+    k_scale = at::empty({nbh, nk}, f32);
+    kmean = at::empty({nbh, D}, f32);
+    stats = at::empty({3, nbh, nk, D}, f32);  // sum, min, max of every key block
+  }
+  float* const ksum = int8 ? ptr<float>(stats) : nullptr;
+  float* const kmin = int8 ? ksum + nbh * nk * D : nullptr;
+  float* const kmax = int8 ? kmin + nbh * nk * D : nullptr;
+  const int32_t* qm = ptr<const int32_t>(q_slot);
+  const int32_t* km = ptr<const int32_t>(k_slot);
+  const int64_t q_src = map ? q.size(1) : 0, k_src = map ? k.size(1) : 0;
+  const uint8_t* kv = ptr<const uint8_t>(k_valid);
+  check_status(a, "pool_query_key", a.pool_query_key(
+      q.data_ptr(), k.data_ptr(), code, B, H, nq, nk, bs, D, q.stride(0), q.stride(th),
+      q.stride(tl), k.stride(0), k.stride(th), k.stride(tl), ptr<const uint8_t>(q_valid), kv, qm,
+      q_src, km, k_src, ptr<float>(qhat), int8 ? ptr<int8_t>(q_i8) : nullptr,
+      int8 ? ptr<float>(q_scale) : nullptr, ptr<float>(khat), ksum, kmin, kmax,
+      ptr<uint32_t>(mask), l.stream));
+  const at::Tensor score = at::empty({nbh, nq, nk}, f32);
+  const at::Tensor indices = at::empty({B, H, nq, max_k}, i32), counts = at::empty({B, H, nq}, i32);
+  const int32_t* rk = ptr<const int32_t>(row_k);
+  const uint8_t *fm = ptr<const uint8_t>(forced), *am = ptr<const uint8_t>(allowed);
+  if (int8 && code == RCSA_BF16 && D == 128 && bs == 128 && nk <= 1024) {
+    check_status(a, "quantize_key_select", a.quantize_key_select(
+        k.data_ptr(), code, B, H, nk, bs, D, k.stride(0), k.stride(th), k.stride(tl), kv, km,
+        k_src, ksum, kmin, kmax, ptr<float>(kmean), ptr<int8_t>(k_i8), ptr<float>(k_scale),
+        ptr<float>(qhat), ptr<float>(khat), nq, ptr<float>(score), rk, row_k_stride_bh, k_fixed,
+        fm, am, mask_stride_bh, ptr<int32_t>(indices), max_k, ptr<int32_t>(counts), l.stream));
+  } else {
+    check_status(a, "block_scores", a.block_scores(ptr<float>(qhat), ptr<float>(khat), nbh, nq, nk,
+                                                   D, ptr<float>(score), l.stream));
+    check_status(a, "select_topk", a.select_topk(
+        ptr<float>(score), nbh, nq, nk, rk, row_k_stride_bh, k_fixed, fm, am, mask_stride_bh,
+        ptr<int32_t>(indices), max_k, ptr<int32_t>(counts), RCSA_ORDER_INDEX, l.stream));
+    if (int8)
+      check_status(a, "quantize_key", a.quantize_key(
+          k.data_ptr(), code, B, H, nk, bs, D, k.stride(0), k.stride(th), k.stride(tl), kv, km,
+          k_src, ksum, kmin, kmax, ptr<float>(kmean), ptr<int8_t>(k_i8), ptr<float>(k_scale),
+          l.stream));
+  }
+  const at::Tensor vb = v.scalar_type() == at::kBFloat16 ? v : v.to(at::kBFloat16);
+  TORCH_CHECK(vb.stride(3) == 1, op, ": v must keep a contiguous last dim");
+  const int64_t o_rows = map ? q.size(1) : Lq;
+  const at::Tensor out = map ? at::empty({B, o_rows, H, D}, b16) : at::empty({B, H, Lq, D}, b16);
+  at::Tensor lse;
+  if (return_lse) lse = at::empty({B, H, o_rows}, f32);
+  float* const lsep = return_lse ? ptr<float>(lse) : nullptr;
+  int64_t ns = n_split;
+  const char* attn = int8 ? "sparse_attn_int8" : "sparse_attn_bf16";
+  if (ns < 1) check_status(a, attn, a.attn_split_plan(B, H, Lq, bs, max_k, &ns));
+  at::Tensor ws;
+  int64_t ws_bytes = 0;
+  if (ns > 1) {
+    ws_bytes = a.attn_workspace_bytes(B, H, Lq, D, ns);
+    TORCH_CHECK(ws_bytes >= 0, attn, ": no workspace for ", ns, " shares");
+    ws = at::empty({ws_bytes}, q.options().dtype(at::kByte));
+  }
+  void* const wsp = ns > 1 ? ws.data_ptr() : nullptr;
+  const float scale = static_cast<float>(sm_scale);
+  if (int8) {
+    check_status(a, attn, a.sparse_attn_int8_split(
+        ptr<int8_t>(q_i8), ptr<float>(q_scale), nq, ptr<int8_t>(k_i8), ptr<float>(k_scale), nk,
+        vb.data_ptr(), nullptr, ptr<uint32_t>(mask), scale, lsep, out.data_ptr(),
+        ptr<int32_t>(indices), ptr<int32_t>(counts), q_i8.stride(0), q_i8.stride(1), D,
+        k_i8.stride(0), k_i8.stride(1), D, vb.stride(0), vb.stride(th), vb.stride(tl),
+        out.stride(0), out.stride(th), out.stride(tl), indices.stride(0), indices.stride(1), max_k,
+        counts.stride(0), counts.stride(1), 1, B, H, Lq, Lk, D, bs, bs, max_k, ns, wsp, ws_bytes,
+        qm, map ? o_rows : 0, km, k_src, l.stream));
+  } else {
+    const at::Tensor qb = code == RCSA_BF16 ? q : q.to(at::kBFloat16);
+    const at::Tensor kb = code == RCSA_BF16 ? k : k.to(at::kBFloat16);
+    TORCH_CHECK(qb.stride(3) == 1 && kb.stride(3) == 1, op,
+                ": q and k must keep a contiguous last dim");
+    check_status(a, attn, a.sparse_attn_bf16_split(
+        qb.data_ptr(), kb.data_ptr(), vb.data_ptr(), nullptr, ptr<uint32_t>(mask), scale, lsep,
+        out.data_ptr(), ptr<int32_t>(indices), ptr<int32_t>(counts), qb.stride(0), qb.stride(th),
+        qb.stride(tl), kb.stride(0), kb.stride(th), kb.stride(tl), vb.stride(0), vb.stride(th),
+        vb.stride(tl), out.stride(0), out.stride(th), out.stride(tl), indices.stride(0),
+        indices.stride(1), max_k, counts.stride(0), counts.stride(1), 1, B, H, Lq, Lk, D, bs, bs,
+        max_k, ns, wsp, ws_bytes, qm, map ? q_src : 0, km, map ? k_src : 0, nullptr, 0,
+        l.stream));
+  }
+  std::vector<at::Tensor> res{out, indices, counts, score, qhat, khat, mask};
+  if (int8) res.insert(res.end(), {q_i8, q_scale, k_i8, k_scale, kmean});
+  if (return_lse) res.push_back(lse);
+  return res;
+}
+
 }  // namespace
 
 TORCH_LIBRARY(rcsa, m) {
@@ -605,4 +769,10 @@ TORCH_LIBRARY(rcsa, m) {
       "int8_linear_group(Tensor x_i8, Tensor x_scale, Tensor[] w, Tensor[] w_scale, "
       "Tensor?[] bias, Tensor(a!)[] out) -> ()",
       &int8_linear_group);
+  m.def(
+      "layer_call(Tensor q, Tensor k, Tensor v, Tensor? q_valid, Tensor? k_valid, int block_size, "
+      "Tensor? row_k, int row_k_stride_bh, int k_fixed, int max_k, Tensor? forced, "
+      "Tensor? allowed, int mask_stride_bh, bool int8, float sm_scale, bool return_lse, "
+      "int n_split, Tensor? q_slot, Tensor? k_slot) -> Tensor[]",
+      &layer_call);
 }

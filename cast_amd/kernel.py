@@ -63,7 +63,9 @@ def longcat_asymmetric(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor,
     v = v.to(torch.bfloat16).contiguous()
     indices = indices.to(torch.int32).contiguous()
     counts = counts.to(torch.int32).contiguous()
-    valid = key_valid.reshape(-1).to(torch.uint8).contiguous()
+    valid = key_valid.reshape(-1)  # (a bool's bytes are its uint8 values)
+    valid = (valid.contiguous().view(torch.uint8) if valid.dtype == torch.bool
+             else valid.to(torch.uint8).contiguous())
     if q.shape[2] % query_block_size or k.shape[2] % key_block_size:
         raise RuntimeError("asymmetric sparse storage is not block aligned")
     if key_block_size % 32 == 0 and valid.numel() == k.shape[2] and valid.is_cuda:

@@ -19,7 +19,7 @@ from typing import Optional
 
 import torch
 
-from . import ops
+from . import _lib, ops
 
 _SIDE_STREAMS: dict = {}
 
@@ -106,6 +106,12 @@ def rcsa_attention(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor,
         B, H, Lq, D = q.shape
         Lk = k.shape[2]
     bs = block_size
+    if overlap and fuse_select and order == "index" and _one_op(q, k, v, bs, Lq, Lk, int8, gathered,
+                                                                v_token is not None, n_split):
+        return _layer_call(q, k, v, q_valid, k_valid, bs, Lq, Lk, k_select, forced, allowed, int8,
+                           max_k, sm_scale, return_lse, n_split,
+                           q_slot_token if gathered else None,
+                           k_slot_token if gathered else None)
     main = torch.cuda.current_stream(q.device) if q.is_cuda else None
     # the bf16 path has no key pass left to overlap with
     side = _side_stream(q.device) if (overlap and int8 and q.is_cuda) else None
@@ -180,6 +186,47 @@ def rcsa_attention(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor,
     out, lse = res if return_lse else (res, None)
     return RCSAResult(out, idx4, cnt3, score, qhat, khat, lse, q_i8, q_scale, k_i8, k_scale,
                       kmean, k_mask)
+
+
+def _one_op(q, k, v, bs, Lq, Lk, int8, gathered, ring_gather, n_split) -> bool:
+    """Whether the call runs as the native op: well-formed operands (the general path
+    words the errors of the others), and no selection worth a stream of its own, i.e.
+    one inside the key quantiser's launch, no quantiser (bf16), or one of a few
+    thousand key tiles, whose pass is shorter than the two cross-stream waits."""
+    if not (q.is_cuda and k.device == q.device and v.device == q.device
+            and q.ndim == k.ndim == v.ndim == 4 and v.shape == k.shape
+            and q.dtype == k.dtype and q.dtype in (torch.bfloat16, torch.float32)
+            and v.dtype in (torch.bfloat16, torch.float32, torch.float16)
+            and q.stride(3) == k.stride(3) == v.stride(3) == 1):
+        return False
+    heads = 2 if gathered else 1
+    D = q.shape[3]
+    if (k.shape[0], k.shape[heads], k.shape[3]) != (q.shape[0], q.shape[heads], D) \
+            or D not in (64, 128) or bs not in (64, 128) or min(Lq, Lk) <= 0 \
+            or Lq % bs or Lk % bs or (gathered and not ring_gather) \
+            or (n_split is not None and int(n_split) < 1):
+        return False
+    if not int8 or (q.dtype == torch.bfloat16 and D == 128 and bs == 128 and Lk // bs <= 1024):
+        return True
+    return q.shape[0] * q.shape[heads] * (Lk // bs) <= 4096
+
+
+def _layer_call(q, k, v, q_valid, k_valid, bs, Lq, Lk, k_select, forced, allowed, int8, max_k,
+                sm_scale, return_lse, n_split, q_slot, k_slot) -> RCSAResult:
+    fn = "rcsa_attention"
+    dev = q.device
+    B, H, D = q.shape[0], q.shape[1 if q_slot is None else 2], q.shape[3]
+    row_k, stride, k_fixed, max_k, fm, am, mstride = ops._selection_args(
+        B * H, Lq // bs, Lk // bs, k_select, forced, allowed, max_k, "index", dev, "select_topk")
+    res = _lib.torch_ops().layer_call(
+        q, k, v, ops._valid_u8(q_valid, Lq, dev, fn), ops._valid_u8(k_valid, Lk, dev, fn), bs,
+        row_k, stride, k_fixed, max_k, fm, am, mstride, int8,
+        1.0 / math.sqrt(D) if sm_scale is None else float(sm_scale), return_lse,
+        -1 if n_split is None else int(n_split), q_slot, k_slot)
+    out, indices, counts, score, qhat, khat, k_mask = res[:7]
+    q_i8, q_scale, k_i8, k_scale, kmean = res[7:12] if int8 else (None,) * 5
+    return RCSAResult(out, indices, counts, score, qhat, khat, res[-1] if return_lse else None,
+                      q_i8, q_scale, k_i8, k_scale, kmean, k_mask)
 
 
 def relay_attention(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, layout, selected,
