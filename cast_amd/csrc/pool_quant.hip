@@ -294,18 +294,17 @@ pool_qk_kernel(PoolArgs q, PoolArgs k, int64_t q_tiles, PoolArgs v, int64_t k_en
 // D + 4 words apart, so the 16 key rows of a read start four banks apart.
 // At 24 heads, D 128: 330 x 330 blocks 26 against 56 us, 28 x 853 11 against 18 us.
 template <int D, int RQ>
-__global__ void __launch_bounds__(256)
-score_kernel(const float* qhat, const float* khat, int64_t nq, int64_t nk,
-             float* score) {
+__device__ __forceinline__ void score_tile(const float* qhat, const float* khat, int64_t nq,
+                                           int64_t nk, float* score, int64_t tile) {
   constexpr int TQ = 16 * RQ, TK = 64, LD = D + 4, C4 = D / 4;
   __shared__ __attribute__((aligned(16))) float sq[TQ][LD];
   __shared__ __attribute__((aligned(16))) float sk[TK][LD];
   constexpr int QL = TQ * C4 / 256;              // float4 loads per thread (query tile)
   constexpr int KL = TK * C4 / 256;              // (key tile)
   const int64_t tiles_q = (nq + TQ - 1) / TQ, tiles_k = (nk + TK - 1) / TK;
-  const int64_t tk = blockIdx.x % tiles_k;
-  const int64_t tq = (blockIdx.x / tiles_k) % tiles_q;
-  const int64_t bh = blockIdx.x / (tiles_k * tiles_q);
+  const int64_t tk = tile % tiles_k;
+  const int64_t tq = (tile / tiles_k) % tiles_q;
+  const int64_t bh = tile / (tiles_k * tiles_q);
   const int t = threadIdx.x;
   const float4* qb = reinterpret_cast<const float4*>(qhat + (bh * nq + tq * TQ) * D);
   const float4* kb = reinterpret_cast<const float4*>(khat + (bh * nk + tk * TK) * D);
@@ -366,6 +365,12 @@ score_kernel(const float* qhat, const float* khat, int64_t nq, int64_t nk,
     }
 }
 
+template <int D, int RQ>
+__global__ void __launch_bounds__(256)
+score_kernel(const float* qhat, const float* khat, int64_t nq, int64_t nk, float* score) {
+  score_tile<D, RQ>(qhat, khat, nq, nk, score, blockIdx.x);
+}
+
 template <int D>
 static void launch_score(const float* qhat, const float* khat, int64_t n_bh, int64_t nq,
                          int64_t nk, float* score, hipStream_t s) {
@@ -393,15 +398,16 @@ __device__ __forceinline__ int nonzero_bytes(uint32_t w) {
 // four independent partial sums, then an LDS reduction.  The valid-token
 // count is taken with 16-byte loads.
 template <int D>
-__global__ void __launch_bounds__(256)
-kmean_kernel(const float* ksum, const uint8_t* valid, const int32_t* slot_tok,
-             int64_t src_len, int64_t n_blocks, int64_t n_tokens, float* kmean) {
+__device__ __forceinline__ void kmean_tile(const float* ksum, const uint8_t* valid,
+                                           const int32_t* slot_tok, int64_t src_len,
+                                           int64_t n_blocks, int64_t n_tokens, float* kmean,
+                                           int64_t tile) {
   constexpr int CG = 16;          // channels per workgroup
   constexpr int BL = 256 / CG;    // block lanes
   __shared__ float part[BL][CG + 1];
   __shared__ float s_red[4];
-  const int64_t bh = blockIdx.x / (D / CG);
-  const int c0 = static_cast<int>(blockIdx.x % (D / CG)) * CG;
+  const int64_t bh = tile / (D / CG);
+  const int c0 = static_cast<int>(tile % (D / CG)) * CG;
   const int t = threadIdx.x, c = t % CG, bl = t / CG;
   const float* src = ksum + bh * n_blocks * D + c0 + c;
   float acc[4] = {0.0f, 0.0f, 0.0f, 0.0f};
@@ -488,6 +494,27 @@ kmean_kernel(const float* ksum, const uint8_t* valid, const int32_t* slot_tok,
   }
 }
 
+template <int D>
+__global__ void __launch_bounds__(256)
+kmean_kernel(const float* ksum, const uint8_t* valid, const int32_t* slot_tok, int64_t src_len,
+             int64_t n_blocks, int64_t n_tokens, float* kmean) {
+  kmean_tile<D>(ksum, valid, slot_tok, src_len, n_blocks, n_tokens, kmean, blockIdx.x);
+}
+
+// The key mean and the block scores in one launch (both need the pooling pass
+// only, and either alone leaves most compute units idle): the first n_score
+// workgroups take score tiles.
+template <int D, int RQ>
+__global__ void __launch_bounds__(256)
+kmean_score_kernel(const float* ksum, const uint8_t* valid, const int32_t* slot_tok,
+                   int64_t src_len, int64_t n_blocks, int64_t n_tokens, float* kmean,
+                   const float* qhat, const float* khat, int64_t nq, float* score,
+                   int64_t n_score) {
+  if (blockIdx.x < n_score) score_tile<D, RQ>(qhat, khat, nq, n_blocks, score, blockIdx.x);
+  else kmean_tile<D>(ksum, valid, slot_tok, src_len, n_blocks, n_tokens, kmean,
+                     blockIdx.x - n_score);
+}
+
 // Smoothed per-block key quantiser: one workgroup per (bh, block).  The tile
 // loads are issued first; the scale (from the block's min/max and the head
 // mean) is computed while they are in flight.
@@ -561,17 +588,19 @@ quant_key_kernel(PoolArgs a, const float* kmean, int8_t* k_i8, float* k_scale) {
   quant_tile<T, D, BS, MAP>(a, kmean, k_i8, k_scale, blockIdx.x);
 }
 
-// The key quantiser and the block scores + top-k selection in one launch: the
-// first n_sel workgroups each score and select kSelWaves rows (latency-bound
-// work that then runs inside the HBM-bound key pass), the rest quantise key
-// tiles.  No reference counterpart; replaces a side stream and its two
-// cross-stream waits.
+// The key quantiser and the top-k selection in one launch: the first n_sel
+// workgroups each select kSelWaves rows (latency-bound work that then runs
+// inside the HBM-bound key pass), the rest quantise key tiles.  No reference
+// counterpart; replaces a side stream and its two cross-stream waits.  (The
+// scores come from the key mean's launch: computed here, a column per lane, they
+// held their compute units: quantising 289 key blocks of 24 heads beside 7 rows a
+// head took 63 us instead of 53, 330 blocks beside 30 rows 77 instead of 61.)
 template <typename T, int D, int BS, bool MAP, int PER>
 __global__ void __launch_bounds__(kPoolThreads)
 quant_select_kernel(PoolArgs a, const float* kmean, int8_t* k_i8, float* k_scale, SelArgs sel,
                     int64_t n_sel) {
   static_assert(kSelWaves * kWave == kPoolThreads, "one block shape");
-  if (blockIdx.x < n_sel) select_rows<PER, false, true>(sel, blockIdx.x, nullptr);
+  if (blockIdx.x < n_sel) select_rows<PER, false>(sel, blockIdx.x, nullptr);
   else quant_tile<T, D, BS, MAP>(a, kmean, k_i8, k_scale, blockIdx.x - n_sel);
 }
 
@@ -775,7 +804,7 @@ static int quantize_key_impl(const void* k, int dtype, int64_t batch, int64_t n_
                              const uint8_t* valid, const int32_t* slot_token, int64_t src_len,
                              const float* ksum, const float* kmin, const float* kmax,
                              float* kmean, int8_t* k_i8, float* k_scale, const SelArgs* sel,
-                             hipStream_t stream) {
+                             const float* qhat, const float* khat, hipStream_t stream) {
   if (!k || !ksum || !kmin || !kmax || !kmean || !k_i8 || !k_scale) return RCSA_ERR_NULL;
   // the fused launch exists for the layer call's shape only
   if (sel && !(dtype == RCSA_BF16 && head_dim == 128 && block_size == 128 && n_blocks <= 1024))
@@ -787,12 +816,28 @@ static int quantize_key_impl(const void* k, int dtype, int64_t batch, int64_t n_
   if (!aligned16(k) || (reinterpret_cast<uintptr_t>(k_i8) & 7u)) return RCSA_ERR_ALIGN;
   const int64_t nbh = batch * n_heads;
   const int64_t n_tokens = n_blocks * block_size;
-  if (head_dim == 128)
+  if (sel) {
+    const int64_t nq = sel->n_q, tiles_k = (n_blocks + 63) / 64;
+    const bool rows32 = nq > 16 && nbh * ((nq + 31) / 32) * tiles_k >= 64;
+    const int64_t tq = rows32 ? 32 : 16;
+    const int64_t n_score = nbh * ((nq + tq - 1) / tq) * tiles_k;
+    const dim3 grid(static_cast<unsigned>(n_score + nbh * 8));
+    float* score = const_cast<float*>(sel->score);
+    if (rows32)
+      kmean_score_kernel<128, 2><<<grid, dim3(256), 0, stream>>>(
+          ksum, valid, slot_token, src_len, n_blocks, n_tokens, kmean, qhat, khat, nq, score,
+          n_score);
+    else
+      kmean_score_kernel<128, 1><<<grid, dim3(256), 0, stream>>>(
+          ksum, valid, slot_token, src_len, n_blocks, n_tokens, kmean, qhat, khat, nq, score,
+          n_score);
+  } else if (head_dim == 128) {
     kmean_kernel<128><<<dim3(nbh * 8), dim3(256), 0, stream>>>(ksum, valid, slot_token, src_len,
                                                                n_blocks, n_tokens, kmean);
-  else
+  } else {
     kmean_kernel<64><<<dim3(nbh * 4), dim3(256), 0, stream>>>(ksum, valid, slot_token, src_len,
                                                               n_blocks, n_tokens, kmean);
+  }
   st = launch_status();
   if (st) return st;
   PoolArgs a{k, n_heads, n_blocks, stride_b, stride_h, stride_t, valid, nullptr,
@@ -804,7 +849,9 @@ static int quantize_key_impl(const void* k, int dtype, int64_t batch, int64_t n_
     dim3 grid(static_cast<unsigned>(n_sel + nbh * n_blocks));
 #define RCSA_QS(MAP, PER) \
   quant_select_kernel<u16, 128, 128, MAP, PER><<<grid, block, 0, stream>>>(a, kmean, k_i8, k_scale, *sel, n_sel)
-    if (n_blocks <= 512) {
+    if (n_blocks <= 384) {
+      if (slot_token) RCSA_QS(true, 6); else RCSA_QS(false, 6);
+    } else if (n_blocks <= 512) {
       if (slot_token) RCSA_QS(true, 8); else RCSA_QS(false, 8);
     } else {
       if (slot_token) RCSA_QS(true, 16); else RCSA_QS(false, 16);
@@ -843,7 +890,7 @@ extern "C" int rcsa_quantize_key(const void* k, int dtype, int64_t batch,
                                  float* k_scale, hipStream_t stream) {
   return quantize_key_impl(k, dtype, batch, n_heads, n_blocks, block_size, head_dim, stride_b,
                            stride_h, stride_t, valid, slot_token, src_len, ksum, kmin, kmax,
-                           kmean, k_i8, k_scale, nullptr, stream);
+                           kmean, k_i8, k_scale, nullptr, nullptr, nullptr, stream);
 }
 
 extern "C" int rcsa_quantize_key_select(
@@ -862,8 +909,8 @@ extern "C" int rcsa_quantize_key_select(
   if (head_dim != 128) return RCSA_ERR_SHAPE;  // the fused scores are unrolled for 128
   const SelArgs sel{score, batch * n_heads * n_qblocks, n_qblocks, n_blocks, row_k,
                     row_k_stride_bh, k_fixed, forced, allowed, mask_stride_bh, indices, max_k,
-                    counts, qhat, khat, head_dim, false};
+                    counts, false};
   return quantize_key_impl(k, dtype, batch, n_heads, n_blocks, block_size, head_dim, stride_b,
                            stride_h, stride_t, valid, slot_token, src_len, ksum, kmin, kmax,
-                           kmean, k_i8, k_scale, &sel, stream);
+                           kmean, k_i8, k_scale, &sel, qhat, khat, stream);
 }

@@ -31,11 +31,6 @@ struct SelArgs {
   int32_t* indices;
   int64_t max_k;
   int32_t* counts;
-  // fused scoring (SCORE kernels): score(row, j) = qhat[row] . khat[bh, j],
-  // summed over the head_dim channels in order, written to score when set
-  const float* qhat;
-  const float* khat;
-  int64_t head_dim;
   // forced columns rank among themselves by fl(score + 1e6) (RCSA_ORDER_RANK_LOCAL)
   bool coarse_forced;
 };
@@ -43,30 +38,11 @@ struct SelArgs {
 constexpr int kSelWaves = 4;
 
 // Value of column j of a row (0 when it is not allowed), and whether it is forced.
-template <bool SCORE>
 __device__ __forceinline__ uint32_t column_value(const SelArgs& a, int64_t row, int64_t bh,
                                                  int64_t i, int64_t j, bool& forced) {
   forced = false;
   if (j >= a.n_k) return 0u;
-  float s;
-  if constexpr (SCORE) {  // the cosine score, in rcsa_block_scores' summation order
-    constexpr int kD = 128;  // the fused launch's head_dim: the loads unroll and overlap
-    const float4* q = reinterpret_cast<const float4*>(a.qhat + row * kD);
-    const float4* k = reinterpret_cast<const float4*>(a.khat + (bh * a.n_k + j) * kD);
-    float acc = 0.0f;
-#pragma unroll
-    for (int c = 0; c < kD / 4; ++c) {
-      const float4 qv = q[c], kv = k[c];
-      acc = fmaf(qv.x, kv.x, acc);
-      acc = fmaf(qv.y, kv.y, acc);
-      acc = fmaf(qv.z, kv.z, acc);
-      acc = fmaf(qv.w, kv.w, acc);
-    }
-    if (a.score) const_cast<float*>(a.score)[row * a.n_k + j] = acc;
-    s = acc;
-  } else {
-    s = a.score[row * a.n_k + j];
-  }
+  float s = a.score[row * a.n_k + j];
   const int64_t moff = bh * a.mask_stride_bh + i * a.n_k + j;
   if (a.allowed && a.allowed[moff] == 0) return 0u;
   forced = a.forced && a.forced[moff] != 0;
@@ -109,10 +85,8 @@ __device__ __forceinline__ void write_ranked(const uint32_t* v, const uint16_t* 
 
 // PER > 0: values held in registers (PER per lane, n_k <= 64 * PER).
 // PER == 0: values recomputed from memory on every pass (any n_k <= 65536).
-// SCORE: the scores are computed here (PER > 0 only: each once).
-template <int PER, bool RANK, bool SCORE>
+template <int PER, bool RANK>
 __device__ __forceinline__ void select_rows(const SelArgs& a, int64_t block, char* s_rank) {
-  static_assert(!SCORE || PER > 0, "fused scores need the values in registers");
   static_assert(PER <= 32, "one forced bit per pass");
   const int lane = threadIdx.x % kWave, wave = threadIdx.x / kWave;
   const int64_t row = block * kSelWaves + wave;
@@ -126,7 +100,7 @@ __device__ __forceinline__ void select_rows(const SelArgs& a, int64_t block, cha
 #pragma unroll PER > 0 ? PER : 1
   for (int p = 0; p < passes; ++p) {
     bool f;
-    const uint32_t v = column_value<SCORE>(a, row, bh, i, lane + int64_t{kWave} * p, f);
+    const uint32_t v = column_value(a, row, bh, i, lane + int64_t{kWave} * p, f);
     f = f && v != 0;
     if (PER > 0) {
       vals[p] = v;
@@ -149,8 +123,7 @@ __device__ __forceinline__ void select_rows(const SelArgs& a, int64_t block, cha
         f = (fbits >> p) & 1u;
         return vals[p];
       } else {
-        const uint32_t v =
-            column_value<SCORE>(a, row, bh, i, lane + int64_t{kWave} * p, f);
+        const uint32_t v = column_value(a, row, bh, i, lane + int64_t{kWave} * p, f);
         f = f && v != 0;
         return v;
       }

@@ -8,7 +8,7 @@ template <int PER, bool RANK>
 __global__ void __launch_bounds__(kSelWaves * kWave)
 select_kernel(SelArgs a) {
   extern __shared__ __attribute__((aligned(16))) char s_rank[];  // RANK: kSelWaves rank lists
-  select_rows<PER, RANK, false>(a, blockIdx.x, s_rank);
+  select_rows<PER, RANK>(a, blockIdx.x, s_rank);
 }
 
 // The selection's certificate: per row the repeated neighbours of its list
@@ -111,7 +111,7 @@ extern "C" int rcsa_select_topk(const float* score, int64_t n_bh, int64_t n_qblo
   if (mask_stride_bh < 0 || row_k_stride_bh < 0) return RCSA_ERR_STRIDE;
   SelArgs a{score, n_bh * n_qblocks, n_qblocks, n_kblocks, row_k, row_k_stride_bh,
             k_fixed, forced, allowed, mask_stride_bh, indices, max_k, counts,
-            nullptr, nullptr, 0, order == RCSA_ORDER_RANK_LOCAL};
+            order == RCSA_ORDER_RANK_LOCAL};
   if (order != RCSA_ORDER_INDEX) launch_select<true>(a, stream);
   else launch_select<false>(a, stream);
   return launch_status();

@@ -280,8 +280,8 @@ int rcsa_quantize_key(const void* k, int dtype, int64_t batch, int64_t n_heads,
 
 /*
  * rcsa_quantize_key, rcsa_block_scores and rcsa_select_topk (index order) in
- * two launches instead of four: the key mean, then one launch whose first
- * workgroups score and select the rows (one wavefront per row) while the rest
+ * two launches instead of four: the key mean and the scores, then one launch whose
+ * first workgroups select the rows (one wavefront per row) while the rest
  * quantise the key tiles.  Outputs are those of the separate calls bit for
  * bit (each score is summed over the channels in rcsa_block_scores' order).
  * No reference counterpart: the int8 layer call's form, replacing a side
