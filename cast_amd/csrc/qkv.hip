@@ -336,8 +336,8 @@ int8_linear_kernel(LinearArgs a, int32_t per_wg, int32_t per_xcd) {
     const uint32_t rows_left = static_cast<uint32_t>(left < L::B ? left : L::B);
     const __amdgpu_buffer_rsrc_t out = __builtin_amdgcn_make_buffer_rsrc(
         static_cast<char*>(a.out[t.g]) + static_cast<int64_t>(t.m0) * row_bytes, 0, static_cast<int>(rows_left * row_bytes), kQkvRsrc3);
-    const uint32_t lane_out = (lane / L::CH) * row_bytes + (lane % L::CH) * 8u * kOutBytes;
-    const int col = static_cast<int>(nw * kOutBytes);
+    const uint32_t lane_out = (lane / L::CH) * row_bytes + (lane % L::CH) * 8u * kOutBytes +
+                              static_cast<uint32_t>(nw) * kOutBytes;
 #pragma unroll
     for (int np = 0; np < T / 2; ++np) {  // 64 channels: whole 128-byte lines
       float4 ws[2][4];
@@ -401,15 +401,17 @@ int8_linear_kernel(LinearArgs a, int32_t per_wg, int32_t per_xcd) {
           const v4u v = *reinterpret_cast<const v4u*>(
               rows + (r * L::CH + (c ^ (r & (L::CH - 1)))) * 16);
           const uint32_t row = wm * 32 * T + m * 32 + i * (kWave / L::CH);
-          const int voff = static_cast<int>(row * row_bytes + lane_out);
-          const int soff = col + np * 64 * static_cast<int>(kOutBytes);
+          // (no scalar offset: with one, the compiler lets the next instruction
+          // overwrite the registers that a 16-byte store is still reading)
+          const int voff = static_cast<int>(row * row_bytes + lane_out) +
+                           np * 64 * static_cast<int>(kOutBytes);
           if constexpr (OUT32) {
             const v4u lo = {v[0] << 16, v[0] & 0xffff0000u, v[1] << 16, v[1] & 0xffff0000u};
             const v4u hi = {v[2] << 16, v[2] & 0xffff0000u, v[3] << 16, v[3] & 0xffff0000u};
-            __builtin_amdgcn_raw_buffer_store_b128(lo, out, voff, soff, 0);
-            __builtin_amdgcn_raw_buffer_store_b128(hi, out, voff + 16, soff, 0);
+            __builtin_amdgcn_raw_buffer_store_b128(lo, out, voff, 0, 0);
+            __builtin_amdgcn_raw_buffer_store_b128(hi, out, voff + 16, 0, 0);
           } else {
-            __builtin_amdgcn_raw_buffer_store_b128(v, out, voff, soff, 0);
+            __builtin_amdgcn_raw_buffer_store_b128(v, out, voff, 0, 0);
           }
         }
         __builtin_amdgcn_sched_barrier(0);
