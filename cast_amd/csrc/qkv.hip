@@ -15,12 +15,12 @@
 // matrix cores' cycles).  Both operands are staged by direct-to-LDS copies
 // through a ring of 128-byte K steps (one whole line of every row); 16-byte
 // chunks of each 128-byte row are XORed by (row / 2) mod 8 so the ds_read_b128
-// operand reads are conflict free.  The launch is persistent: one workgroup per
-// compute unit walks its XCD's tiles of all projections, and the ring runs on
-// from one tile to the next.  Three projections of 3072 x 3072, one launch,
+// operand reads are conflict free.  The launch is persistent: a compute unit's
+// workgroups walk its XCD's tiles of all projections, and the ring runs on from
+// one tile to the next.  Three projections of 3072 x 3072, one launch,
 // against three launches of the eight-wavefront kernel: 38,720 tokens 1034
 // against 1199 us (2.1 POP/s), 3520 tokens 92 against 155, 880 tokens (128 x 128
-// tiles) 32 against 144 us.  What bounds it: the matrix cores' clock under load
+// tiles) 31 against 144 us.  What bounds it: the matrix cores' clock under load
 // (1.9 GHz) and the epilogue, which no MFMA of the same SIMD covers.
 #include <type_traits>
 
@@ -151,22 +151,28 @@ __device__ __forceinline__ void lin_wait_barrier() {
 
 // A workgroup tile of 4 wavefronts (2 along tokens x 2 along channels), each
 // T x T MFMA tiles of 32 x 32, over a ring of SLOTS K steps.
-template <int T_, int SLOTS_>
+// WGS workgroups share a compute unit.
+template <int T_, int SLOTS_, int WGS_>
 struct LinTile {
-  static constexpr int T = T_, SLOTS = SLOTS_;
+  static constexpr int T = T_, SLOTS = SLOTS_, WGS = WGS_;
   static constexpr int B = 2 * 32 * T;                 // tokens and channels of a tile
   static constexpr int OB = B * kKS;                   // bytes of one operand's step
   static constexpr int U = OB / 1024 / kGemmWaves;     // 1 KiB copies per wavefront and operand
   static constexpr int OPS = 2 * U;                    // copies per wavefront and step
   static constexpr int KS = kKS / 32;                  // MFMA k-steps per ring step
   static constexpr int CH = 8;                         // 16-byte chunks of an epilogue row
-  static constexpr int EB = 2 * 32 * CH * 16;          // epilogue bytes per wavefront: 2 x 32 rows
+  static constexpr int ROWS = 32 * CH * 16;            // 32 epilogue rows of a wavefront
+  static constexpr int EN = WGS == 1 ? 2 : 1;          // in one or two buffers
+  static constexpr int EB = EN * ROWS;
   static_assert((SLOTS - 2) * OPS < 64, "vmcnt range");
-  static_assert(SLOTS * 2 * OB + kGemmWaves * EB <= 160 * 1024, "LDS of a compute unit");
+  static_assert(WGS * (SLOTS * 2 * OB + kGemmWaves * EB) <= 160 * 1024, "LDS of a compute unit");
 };
 
-using BigTile = LinTile<4, 2>;   // 256 x 256, 64 KiB steps
-using MidTile = LinTile<2, 4>;   // 128 x 128, 32 KiB steps
+using BigTile = LinTile<4, 2, 1>;  // 256 x 256, 64 KiB steps
+// 128 x 128, 32 KiB steps: two workgroups fill each other's waits (three
+// projections of 880 tokens 31.4 us against 33.1 with one of four slots, 2640
+// tokens 81 against 87)
+using MidTile = LinTile<2, 2, 2>;
 
 // Where a tile's operands are and where its outputs go.
 struct TileSrc {
@@ -198,19 +204,18 @@ __device__ __forceinline__ TileSrc tile_src(const LinearArgs& a, uint32_t work) 
           static_cast<int>(L::B * a.K), g, m0, n0};
 }
 
-// One persistent workgroup per compute unit: workgroup j of XCD x takes the
+// L::WGS persistent workgroups per compute unit: workgroup j of XCD x takes the
 // XCD's tiles j, j + per_wg, ...  The copy ring runs on from tile to tile, so a
 // tile's first steps land during the previous tile's last MFMAs and epilogue.
 template <class L, bool OUT32>
-__global__ void __launch_bounds__(kGemmThreads) __attribute__((amdgpu_waves_per_eu(1, 1)))
+__global__ void __launch_bounds__(kGemmThreads) __attribute__((amdgpu_waves_per_eu(L::WGS, L::WGS)))
 int8_linear_kernel(LinearArgs a, int32_t per_wg, int32_t per_xcd) {
   constexpr int T = L::T, SLOTS = L::SLOTS, KS = L::KS;
+  static_assert(SLOTS == 2, "the unrolled ring");
   // (slots in arrays of their own: the compiler then knows that reads of one do
   // not alias the copies in flight into the others)
   __shared__ __attribute__((aligned(1024))) char s_0[2 * L::OB];
   __shared__ __attribute__((aligned(1024))) char s_1[2 * L::OB];
-  __shared__ __attribute__((aligned(1024))) char s_2[SLOTS > 2 ? 2 * L::OB : 16];
-  __shared__ __attribute__((aligned(1024))) char s_3[SLOTS > 2 ? 2 * L::OB : 16];
   __shared__ __attribute__((aligned(1024))) char s_e[kGemmWaves * L::EB];
   const int32_t first = static_cast<int32_t>(blockIdx.x % kNumXcd) * per_xcd;
   const int32_t all = static_cast<int32_t>(a.tiles[a.n_lin]);
@@ -356,7 +361,7 @@ int8_linear_kernel(LinearArgs a, int32_t per_wg, int32_t per_xcd) {
       __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
       for (int m = 0; m < T; ++m) {
-        char* const rows = eb + (m & 1) * (32 * L::CH * 16);
+        char* const rows = eb + (m & (L::EN - 1)) * L::ROWS;
         // (the accumulators leave their AGPRs here, not all before the epilogue)
         asm volatile("" : "+a"(acc[2 * np][m]), "+a"(acc[2 * np + 1][m]));
 #pragma unroll
@@ -422,7 +427,7 @@ int8_linear_kernel(LinearArgs a, int32_t per_wg, int32_t per_xcd) {
   TileSrc cur = tile_src<L>(a, static_cast<uint32_t>(item));
 #pragma unroll
   for (int i = 0; i < SLOTS; ++i) {
-    stage(cur, i, i == 0 ? s_0 : i == 1 ? s_1 : i == 2 ? s_2 : s_3);
+    stage(cur, i, i == 0 ? s_0 : s_1);
     __builtin_amdgcn_sched_barrier(0);  // the steps' copies stay in order
   }
   lin_wait_barrier<(SLOTS - 1) * L::OPS>();
@@ -447,15 +452,8 @@ int8_linear_kernel(LinearArgs a, int32_t per_wg, int32_t per_xcd) {
       ft.xbytes = last ? nt.xbytes : cur.xbytes;
       ft.wbytes = last ? nt.wbytes : cur.wbytes;
       const int fs = last ? 0 : s + SLOTS;
-      if constexpr (SLOTS == 2) {
-        step(s_0, s_1, ft, fs);
-        step(s_1, s_0, ft, fs + 1);
-      } else {
-        step(s_0, s_1, ft, fs);
-        step(s_1, s_2, ft, fs + 1);
-        step(s_2, s_3, ft, fs + 2);
-        step(s_3, s_0, ft, fs + 3);
-      }
+      step(s_0, s_1, ft, fs);
+      step(s_1, s_0, ft, fs + 1);
       s += SLOTS;
     } while (s < steps);
     store(cur);
@@ -520,9 +518,10 @@ static int launch_linear(LinearArgs& a, int64_t cus, bool out_f32, hipStream_t s
   const int64_t tiles = count_tiles<L>(a);
   if (tiles >= (int64_t{1} << 30)) return RCSA_ERR_SHAPE;
   a.steps = static_cast<int32_t>((a.K / kKS + L::SLOTS - 1) / L::SLOTS * L::SLOTS);
-  // one workgroup per compute unit, the same number on every XCD
+  // the compute units' workgroups, the same number on every XCD
   const int64_t per_xcd = (tiles + kNumXcd - 1) / kNumXcd;
-  const int64_t per_wg = per_xcd < cus / kNumXcd ? per_xcd : cus / kNumXcd;
+  const int64_t slots = cus / kNumXcd * L::WGS;
+  const int64_t per_wg = per_xcd < slots ? per_xcd : slots;
   const dim3 grid(static_cast<unsigned>(per_wg * kNumXcd)), block(kGemmThreads);
   const int32_t wg = static_cast<int32_t>(per_wg), px = static_cast<int32_t>(per_xcd);
   if (out_f32) int8_linear_kernel<L, true><<<grid, block, 0, stream>>>(a, wg, px);
@@ -567,7 +566,7 @@ extern "C" int rcsa_int8_linear_group(const int8_t* x, const float* x_scale, int
   }
   // The tile size that needs less time for its whole rounds: a round of 128 x 128
   // tiles takes 5/16 of a round of 256 x 256 tiles (14 and 44 us at K 3072; three
-  // projections of 880 tokens: 2 rounds, 32 us, against 1 round, 44 us; of 1760
+  // projections of 880 tokens: 2 rounds, 31 us, against 1 round, 44 us; of 1760
   // tokens: 4 rounds, 59 us, against 1 round, 51 us).
   const int64_t cus = device_cus();
   const int64_t big = (count_tiles<BigTile>(a) + cus - 1) / cus * 16;
