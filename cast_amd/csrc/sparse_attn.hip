@@ -12,16 +12,18 @@ template <bool INT8>
 static int launch_attn(AttnArgs& a, int64_t D, int64_t BM, int64_t BN, hipStream_t s) {
   const int64_t per_xcd = a.xcd_direct + (a.xcd_items - a.xcd_direct) * a.n_split;
   const dim3 grid(static_cast<unsigned>(kNumXcd * per_xcd));
-  // gathered sources exist for the 3-slot rings with validity bits only
-  if (a.kv_tok != nullptr && !(a.kmask != nullptr && D == 128 && BM == 128 && BN == 128))
+  const int64_t cux = cus_per_xcd();
+  const bool cu3 = cux > 0 && a.xcd_items >= 2 * cux;
+  // gathered sources need validity bits, D 128 and 128-key blocks; 64-row query
+  // blocks two rounds of them
+  if (a.kv_tok != nullptr && !(a.kmask != nullptr && D == 128 && BN == 128 &&
+                               (BM == 128 || cu3)))
     return RCSA_ERR_SHAPE;
   // D 128, 128 x 128 blocks: 3-slot rings.  With at least two full rounds of
   // query blocks per XCD, three 4-wavefront workgroups per compute unit
   // (32-key steps); otherwise one 8-wavefront workgroup (int8: 128-key steps
   // of 48 KiB, bf16: 64-key steps of 32 KiB).  Packed and gathered sources of
   // one shape take the same form, so the two forms of a call stay bit-identical.
-  const int64_t cux = cus_per_xcd();
-  const bool cu3 = cux > 0 && a.xcd_items >= 2 * cux;
   if (D == 128 && BM == 128 && BN == 128) {
     const bool bits = a.kmask != nullptr, gather = a.kv_tok != nullptr;
     if constexpr (INT8) {

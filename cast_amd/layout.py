@@ -17,7 +17,7 @@ from __future__ import annotations
 import functools
 import math
 from dataclasses import dataclass
-from typing import Sequence
+from typing import Optional, Sequence
 
 import torch
 
@@ -148,6 +148,9 @@ class RelayLayout:
     query_valid: torch.Tensor       # bool  [n_query_blocks * block_size]
     query_indices: torch.Tensor     # int64 [n_query_tokens], tokens of the query frames
     query_out_row: torch.Tensor     # int32 [n_query_blocks * block_size], row in query_indices
+    # (slot map, output rows) of the blocks' first halves, when no block holds
+    # more query tokens than that
+    query_half: Optional[tuple[torch.Tensor, torch.Tensor]] = None
 
 
 def _bits32(valid: torch.Tensor, block_size: int) -> torch.Tensor:
@@ -210,12 +213,17 @@ def _relay_layout_cached(total_temporal: int, memory_temporal: int, height: int,
     query_tok[q_slot] = q_tok
     out_row = torch.full((n_q,), -1, dtype=torch.long, device=device)
     out_row[q_slot] = torch.arange(q_tok.numel(), device=device)
+    # a block's query tokens come first
+    half = None
+    if bs % 2 == 0 and not bool((query_tok.view(-1, bs)[:, bs // 2:] >= 0).any()):
+        half = tuple(x.view(-1, bs)[:, :bs // 2].reshape(-1).to(torch.int32)
+                     for x in (query_tok, out_row))
     key_valid = key_tok >= 0
     bits = (_bits32(key_valid, bs) if bs % 32 == 0
             else torch.empty(0, dtype=torch.int32, device=device))
     return RelayLayout(bs, n_blocks, key_tok.to(torch.int32), key_valid, bits,
                        q_blocks, query_tok.to(torch.int32), query_tok >= 0, q_tok,
-                       out_row.to(torch.int32))
+                       out_row.to(torch.int32), half)
 
 
 def relay_layout(total_temporal: int, memory_temporal: int, height: int, width: int,

@@ -267,6 +267,14 @@ def relay_attention(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, layout, s
         idx = selected.index_select(2, rows).to(torch.int32).contiguous()
         cnt = counts.index_select(2, rows).to(torch.int32).contiguous()
     n_out = layout.query_indices.numel()
+    # Query blocks that fill at most half their slots run as 64-row blocks, where the
+    # device has two rounds of them (the 128-row form of that size takes the same
+    # steps for every row; fewer blocks take longer steps)
+    n_qblocks = rows.numel()
+    cus = torch.cuda.get_device_properties(q.device).multi_processor_count
+    half = layout.query_half if -(-B * H * n_qblocks // 8) >= 2 * (cus // 8) else None
+    bm, q_slot, out_row = ((bs // 2, *half) if half is not None
+                           else (bs, layout.query_slot_token, layout.query_out_row))
     scale = 1.0 / math.sqrt(D) if sm_scale is None else sm_scale
     if int8:
         # Q quantised over the query rows, K statistics and bits over the key rows
@@ -276,17 +284,18 @@ def relay_attention(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, layout, s
         k_i8, k_scale, _ = ops.quantize_key(k, None, bs, ksum, kmin, kmax,
                                             slot_token=layout.key_slot_token)
         v = v if v.dtype == torch.bfloat16 else v.to(torch.bfloat16)
+        if half is not None:
+            q_i8 = q_i8.view(B, H, n_qblocks, bs, D)[:, :, :, :bm].reshape(B, H, -1, D)
         return ops.sparse_attn_int8(q_i8, q_scale, k_i8, k_scale, v, idx, cnt, None,
-                                    block_m=bs, block_n=bs, sm_scale=scale,
+                                    block_m=bm, block_n=bs, sm_scale=scale,
                                     return_lse=return_lse, n_split=n_split,
-                                    block_mask=k_mask, out_token=layout.query_out_row,
+                                    block_mask=k_mask, out_token=out_row,
                                     out_len=n_out, v_token=layout.key_slot_token,
                                     ordered=ordered)
     qb, kb, vb = (x if x.dtype == torch.bfloat16 else x.to(torch.bfloat16) for x in (q, k, v))
-    return ops.sparse_attn_bf16(qb, kb, vb, idx, cnt, None, block_m=bs, block_n=bs,
+    return ops.sparse_attn_bf16(qb, kb, vb, idx, cnt, None, block_m=bm, block_n=bs,
                                 sm_scale=scale, return_lse=return_lse, n_split=n_split,
-                                block_mask=layout.key_block_mask,
-                                q_token=layout.query_slot_token,
+                                block_mask=layout.key_block_mask, q_token=q_slot,
                                 kv_token=layout.key_slot_token,
-                                out_token=layout.query_out_row, out_len=n_out,
+                                out_token=out_row, out_len=n_out,
                                 ordered=ordered)

@@ -123,3 +123,34 @@ def test_relay_attention_vs_oracle(int8):
     got = out.float().cpu()
     for h in range(H):
         _check_attn(want[0, :, h], got[0, :, h], f"relay int8 {int8} head {h}")
+
+
+@pytest.mark.parametrize("int8", [True, False])
+@pytest.mark.parametrize("query_frames", [[30], [30, 31], [29, 30], [29, 30, 31]])
+def test_relay_half_blocks(int8, query_frames):
+    """At two rounds of query blocks (every head its own) blocks with at most 64 query
+    tokens run as 64-row blocks: the 128-row call's results, whose rows take the same
+    steps (the split plans agree too), up to the last place of bf16."""
+    from dataclasses import replace
+
+    from cast_amd import layout
+    from cast_amd.pipeline import relay_attention
+    dev = torch.device("cuda:0")
+    cus = torch.cuda.get_device_properties(0).multi_processor_count
+    n_frames, mem, hw = 32, 24, (16, 32)
+    lay = layout.relay_layout(n_frames, mem, *hw, SHAPE, query_frames, device=dev)
+    nqb, nb = lay.query_block_ids.numel(), lay.n_blocks
+    heads = -(-2 * cus // nqb)
+    assert (lay.query_half is not None) == (len(query_frames) < 3)
+    g = torch.Generator(device=dev).manual_seed(len(query_frames))
+    q, k, v = (torch.randn(1, n_frames * hw[0] * hw[1], heads, 128, device=dev,
+                           generator=g).bfloat16() for _ in range(3))
+    sel = torch.rand(1, heads, nb, nb, device=dev, generator=g).argsort(-1)[..., :21].int()
+    cnt = torch.randint(0, 22, (1, heads, nb), device=dev, generator=g, dtype=torch.int32)
+    out, lse = relay_attention(q, k, v, lay, sel.contiguous(), cnt, int8=int8, return_lse=True)
+    want, want_lse = relay_attention(q, k, v, replace(lay, query_half=None), sel.contiguous(),
+                                     cnt, int8=int8, return_lse=True)
+    torch.testing.assert_close(out.float(), want.float(), rtol=2.0 ** -7, atol=2.0 ** -12)
+    fin = torch.isfinite(want_lse)
+    assert torch.equal(fin, torch.isfinite(lse))
+    torch.testing.assert_close(lse[fin], want_lse[fin], rtol=0, atol=1e-4)
