@@ -290,13 +290,15 @@ pool_qk_kernel(PoolArgs q, PoolArgs k, int64_t q_tiles, PoolArgs v, int64_t k_en
 // Cosine scores: one workgroup per (bh, 16 RQ query blocks, 64 key blocks), RQ x 4
 // scores per thread, four channels per LDS read (RQ + 4 reads for 16 RQ FMAs;
 // one score per thread and channel reads two words for each FMA and was bound by
-// LDS).  Every score is one FMA chain over the channels in order.  The rows are
-// D + 4 words apart, so the 16 key rows of a read start four banks apart.
-// At 24 heads, D 128: 330 x 330 blocks 26 against 56 us, 28 x 853 11 against 18 us.
+// LDS).  Every score is one FMA chain over the channels in order.  The tiles are
+// staged 64 channels at a time, so that four workgroups share a compute unit and
+// the next channels' loads are in flight during the FMAs; rows are 68 words
+// apart, so the 16 key rows of a read start four banks apart.  At 24 heads, D
+// 128: 330 x 330 blocks 22 against 56 us, 28 x 853 10 against 18 us.
 template <int D, int RQ>
 __device__ __forceinline__ void score_tile(const float* qhat, const float* khat, int64_t nq,
                                            int64_t nk, float* score, int64_t tile) {
-  constexpr int TQ = 16 * RQ, TK = 64, LD = D + 4, C4 = D / 4;
+  constexpr int TQ = 16 * RQ, TK = 64, DC = 64, LD = DC + 4, C4 = DC / 4;
   __shared__ __attribute__((aligned(16))) float sq[TQ][LD];
   __shared__ __attribute__((aligned(16))) float sk[TK][LD];
   constexpr int QL = TQ * C4 / 256;              // float4 loads per thread (query tile)
@@ -306,55 +308,61 @@ __device__ __forceinline__ void score_tile(const float* qhat, const float* khat,
   const int64_t tq = (tile / tiles_k) % tiles_q;
   const int64_t bh = tile / (tiles_k * tiles_q);
   const int t = threadIdx.x;
-  const float4* qb = reinterpret_cast<const float4*>(qhat + (bh * nq + tq * TQ) * D);
-  const float4* kb = reinterpret_cast<const float4*>(khat + (bh * nk + tk * TK) * D);
+  const v4f* qb = reinterpret_cast<const v4f*>(qhat + (bh * nq + tq * TQ) * D);
+  const v4f* kb = reinterpret_cast<const v4f*>(khat + (bh * nk + tk * TK) * D);
   // rows past the end re-read the last row: every load is in bounds
   const int q_last = static_cast<int>(min<int64_t>(nq - tq * TQ, TQ)) - 1;
   const int k_last = static_cast<int>(min<int64_t>(nk - tk * TK, TK)) - 1;
-  float4 qv[QL], kv[KL];
-#pragma unroll
-  for (int i = 0; i < QL; ++i) {
-    const int e = t + 256 * i;
-    qv[i] = qb[min(e / C4, q_last) * C4 + e % C4];
+  v4f qv[QL], kv[KL];
+#define RCSA_SCORE_LOAD(c0)                                                           \
+  _Pragma("unroll") for (int i = 0; i < QL; ++i) {                                    \
+    const int e = t + 256 * i;                                                        \
+    qv[i] = qb[min(e / C4, q_last) * (D / 4) + (c0) / 4 + e % C4];                    \
+  }                                                                                   \
+  _Pragma("unroll") for (int i = 0; i < KL; ++i) {                                    \
+    const int e = t + 256 * i;                                                        \
+    kv[i] = kb[min(e / C4, k_last) * (D / 4) + (c0) / 4 + e % C4];                    \
   }
-#pragma unroll
-  for (int i = 0; i < KL; ++i) {
-    const int e = t + 256 * i;
-    kv[i] = kb[min(e / C4, k_last) * C4 + e % C4];
-  }
-#pragma unroll
-  for (int i = 0; i < QL; ++i) {
-    const int e = t + 256 * i;
-    *reinterpret_cast<float4*>(&sq[e / C4][e % C4 * 4]) = qv[i];
-  }
-#pragma unroll
-  for (int i = 0; i < KL; ++i) {
-    const int e = t + 256 * i;
-    *reinterpret_cast<float4*>(&sk[e / C4][e % C4 * 4]) = kv[i];
-  }
-  __syncthreads();
   const int qi = t / 16 * RQ, kj = t % 16;  // rows qi.., columns kj + 16 u
   float acc[RQ][4];
 #pragma unroll
   for (int r = 0; r < RQ; ++r)
 #pragma unroll
     for (int u = 0; u < 4; ++u) acc[r][u] = 0.0f;
+  RCSA_SCORE_LOAD(0)
+  for (int c0 = 0; c0 < D; c0 += DC) {
+    if (c0 > 0) __syncthreads();  // every thread has read the channels before
+#pragma unroll
+    for (int i = 0; i < QL; ++i) {
+      const int e = t + 256 * i;
+      *reinterpret_cast<v4f*>(&sq[e / C4][e % C4 * 4]) = qv[i];
+    }
+#pragma unroll
+    for (int i = 0; i < KL; ++i) {
+      const int e = t + 256 * i;
+      *reinterpret_cast<v4f*>(&sk[e / C4][e % C4 * 4]) = kv[i];
+    }
+    __syncthreads();
+    if (c0 + DC < D) {
+      RCSA_SCORE_LOAD(c0 + DC)
+    }
 #pragma unroll 4
-  for (int c = 0; c < D; c += 4) {
-    float4 a[RQ], b[4];
+    for (int c = 0; c < DC; c += 4) {
+      v4f a[RQ], b[4];
 #pragma unroll
-    for (int r = 0; r < RQ; ++r) a[r] = *reinterpret_cast<const float4*>(&sq[qi + r][c]);
+      for (int r = 0; r < RQ; ++r) a[r] = *reinterpret_cast<const v4f*>(&sq[qi + r][c]);
 #pragma unroll
-    for (int u = 0; u < 4; ++u) b[u] = *reinterpret_cast<const float4*>(&sk[kj + 16 * u][c]);
+      for (int u = 0; u < 4; ++u) b[u] = *reinterpret_cast<const v4f*>(&sk[kj + 16 * u][c]);
 #pragma unroll
-    for (int r = 0; r < RQ; ++r)
+      for (int r = 0; r < RQ; ++r)
 #pragma unroll
-      for (int u = 0; u < 4; ++u) {
-        acc[r][u] = fmaf(a[r].x, b[u].x, acc[r][u]);
-        acc[r][u] = fmaf(a[r].y, b[u].y, acc[r][u]);
-        acc[r][u] = fmaf(a[r].z, b[u].z, acc[r][u]);
-        acc[r][u] = fmaf(a[r].w, b[u].w, acc[r][u]);
-      }
+        for (int u = 0; u < 4; ++u) {
+          acc[r][u] = fmaf(a[r].x, b[u].x, acc[r][u]);
+          acc[r][u] = fmaf(a[r].y, b[u].y, acc[r][u]);
+          acc[r][u] = fmaf(a[r].z, b[u].z, acc[r][u]);
+          acc[r][u] = fmaf(a[r].w, b[u].w, acc[r][u]);
+        }
+    }
   }
 #pragma unroll
   for (int r = 0; r < RQ; ++r)
@@ -364,6 +372,7 @@ __device__ __forceinline__ void score_tile(const float* qhat, const float* khat,
       if (gi < nq && gj < nk) score[(bh * nq + gi) * nk + gj] = acc[r][u];
     }
 }
+#undef RCSA_SCORE_LOAD
 
 template <int D, int RQ>
 __global__ void __launch_bounds__(256)
@@ -797,7 +806,11 @@ extern "C" int rcsa_block_scores(const float* qhat, const float* khat, int64_t n
   return launch_status();
 }
 
-// The key mean, then the quantiser (with sel: fused with the scores + top-k).
+// Key blocks of a fused call at other shapes than the main one.
+constexpr int64_t kSmallSelect = 256;
+
+// The key mean, then the quantiser (with sel: the scores beside the one, the top-k
+// beside the other).
 static int quantize_key_impl(const void* k, int dtype, int64_t batch, int64_t n_heads,
                              int64_t n_blocks, int64_t block_size, int64_t head_dim,
                              int64_t stride_b, int64_t stride_h, int64_t stride_t,
@@ -806,8 +819,9 @@ static int quantize_key_impl(const void* k, int dtype, int64_t batch, int64_t n_
                              float* kmean, int8_t* k_i8, float* k_scale, const SelArgs* sel,
                              const float* qhat, const float* khat, hipStream_t stream) {
   if (!k || !ksum || !kmin || !kmax || !kmean || !k_i8 || !k_scale) return RCSA_ERR_NULL;
-  // the fused launch exists for the layer call's shape only
-  if (sel && !(dtype == RCSA_BF16 && head_dim == 128 && block_size == 128 && n_blocks <= 1024))
+  // the fused launch: the layer call's main shape, and packed keys of a few blocks
+  const bool main_shape = dtype == RCSA_BF16 && head_dim == 128 && block_size == 128;
+  if (sel && !(main_shape ? n_blocks <= 1024 : slot_token == nullptr && n_blocks <= kSmallSelect))
     return RCSA_ERR_SHAPE;
   if (slot_token && (src_len <= 0 || src_len >= (int64_t{1} << 31))) return RCSA_ERR_SHAPE;
   int st = check_pool_shape(dtype, batch, n_heads, n_blocks, block_size, head_dim,
@@ -821,16 +835,14 @@ static int quantize_key_impl(const void* k, int dtype, int64_t batch, int64_t n_
     const bool rows32 = nq > 16 && nbh * ((nq + 31) / 32) * tiles_k >= 64;
     const int64_t tq = rows32 ? 32 : 16;
     const int64_t n_score = nbh * ((nq + tq - 1) / tq) * tiles_k;
-    const dim3 grid(static_cast<unsigned>(n_score + nbh * 8));
+    const dim3 grid(static_cast<unsigned>(n_score + nbh * (head_dim / 16)));
     float* score = const_cast<float*>(sel->score);
-    if (rows32)
-      kmean_score_kernel<128, 2><<<grid, dim3(256), 0, stream>>>(
-          ksum, valid, slot_token, src_len, n_blocks, n_tokens, kmean, qhat, khat, nq, score,
-          n_score);
-    else
-      kmean_score_kernel<128, 1><<<grid, dim3(256), 0, stream>>>(
-          ksum, valid, slot_token, src_len, n_blocks, n_tokens, kmean, qhat, khat, nq, score,
-          n_score);
+#define RCSA_KS(D_, RQ_)                                                                     \
+  kmean_score_kernel<D_, RQ_><<<grid, dim3(256), 0, stream>>>(                               \
+      ksum, valid, slot_token, src_len, n_blocks, n_tokens, kmean, qhat, khat, nq, score, n_score)
+    if (head_dim == 128) { if (rows32) RCSA_KS(128, 2); else RCSA_KS(128, 1); }
+    else { if (rows32) RCSA_KS(64, 2); else RCSA_KS(64, 1); }
+#undef RCSA_KS
   } else if (head_dim == 128) {
     kmean_kernel<128><<<dim3(nbh * 8), dim3(256), 0, stream>>>(ksum, valid, slot_token, src_len,
                                                                n_blocks, n_tokens, kmean);
@@ -849,13 +861,27 @@ static int quantize_key_impl(const void* k, int dtype, int64_t batch, int64_t n_
     dim3 grid(static_cast<unsigned>(n_sel + nbh * n_blocks));
 #define RCSA_QS(MAP, PER) \
   quant_select_kernel<u16, 128, 128, MAP, PER><<<grid, block, 0, stream>>>(a, kmean, k_i8, k_scale, *sel, n_sel)
-    if (n_blocks <= 384) {
+#define RCSA_QSS(T_, D_, BS_) \
+  quant_select_kernel<T_, D_, BS_, false, kSmallSelect / 64><<<grid, block, 0, stream>>>(a, kmean, k_i8, k_scale, *sel, n_sel)
+    if (!main_shape) {
+      if (dtype == RCSA_BF16) {
+        if (head_dim == 128) RCSA_QSS(u16, 128, 64);
+        else if (block_size == 128) RCSA_QSS(u16, 64, 128);
+        else RCSA_QSS(u16, 64, 64);
+      } else {
+        if (head_dim == 128 && block_size == 128) RCSA_QSS(float, 128, 128);
+        else if (head_dim == 128) RCSA_QSS(float, 128, 64);
+        else if (block_size == 128) RCSA_QSS(float, 64, 128);
+        else RCSA_QSS(float, 64, 64);
+      }
+    } else if (n_blocks <= 384) {
       if (slot_token) RCSA_QS(true, 6); else RCSA_QS(false, 6);
     } else if (n_blocks <= 512) {
       if (slot_token) RCSA_QS(true, 8); else RCSA_QS(false, 8);
     } else {
       if (slot_token) RCSA_QS(true, 16); else RCSA_QS(false, 16);
     }
+#undef RCSA_QSS
 #undef RCSA_QS
     return launch_status();
   }
@@ -906,7 +932,6 @@ extern "C" int rcsa_quantize_key_select(
   if (n_qblocks <= 0 || max_k <= 0 || batch <= 0 || n_heads <= 0) return RCSA_ERR_SHAPE;
   if (mask_stride_bh < 0 || row_k_stride_bh < 0) return RCSA_ERR_STRIDE;
   if (!aligned16(qhat) || !aligned16(khat)) return RCSA_ERR_ALIGN;
-  if (head_dim != 128) return RCSA_ERR_SHAPE;  // the fused scores are unrolled for 128
   const SelArgs sel{score, batch * n_heads * n_qblocks, n_qblocks, n_blocks, row_k,
                     row_k_stride_bh, k_fixed, forced, allowed, mask_stride_bh, indices, max_k,
                     counts, false};

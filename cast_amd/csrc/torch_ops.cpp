@@ -661,7 +661,8 @@ std::vector<at::Tensor> layer_call(
   const at::Tensor indices = at::empty({B, H, nq, max_k}, i32), counts = at::empty({B, H, nq}, i32);
   const int32_t* rk = ptr<const int32_t>(row_k);
   const uint8_t *fm = ptr<const uint8_t>(forced), *am = ptr<const uint8_t>(allowed);
-  if (int8 && code == RCSA_BF16 && D == 128 && bs == 128 && nk <= 1024) {
+  const bool main_shape = code == RCSA_BF16 && D == 128 && bs == 128;
+  if (int8 && (main_shape ? nk <= 1024 : !map && nk <= 256)) {
     check_status(a, "quantize_key_select", a.quantize_key_select(
         k.data_ptr(), code, B, H, nk, bs, D, k.stride(0), k.stride(th), k.stride(tl), kv, km,
         k_src, ksum, kmin, kmax, ptr<float>(kmean), ptr<int8_t>(k_i8), ptr<float>(k_scale),

@@ -289,7 +289,8 @@ int rcsa_quantize_key(const void* k, int dtype, int64_t batch, int64_t n_heads,
  * [n_bh][n_blocks][D] come from the pooling pass; score receives
  * [n_bh][n_qblocks][n_blocks]; the selection arguments are those of
  * rcsa_select_topk.  bf16 keys, head_dim 128, block_size 128 and n_blocks <=
- * 1024 only (RCSA_ERR_SHAPE otherwise: use the separate calls).
+ * 1024, or any other shape of packed keys (no slot_token) and n_blocks <= 256
+ * (RCSA_ERR_SHAPE otherwise: use the separate calls).
  */
 int rcsa_quantize_key_select(const void* k, int dtype, int64_t batch, int64_t n_heads,
                              int64_t n_blocks, int64_t block_size, int64_t head_dim,
