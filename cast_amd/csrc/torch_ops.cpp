@@ -9,13 +9,14 @@
 // bad layout.  Every tensor is checked to span the elements the call's dims
 // and strides reach, so no argument combination makes a kernel read or write
 // past the tensors it was given.  Nothing here synchronises, and nothing but
-// layer_call, which allocates its outputs, allocates device memory.
+// layer_call and order_lists, which allocate their outputs, allocates device memory.
 //
 // The C ABI is bound at load time (rcsa::bind_library) from the library the
 // Python side loaded, so one librcsa.so serves both the ctypes binding and
 // these ops.
 #include <dlfcn.h>
 
+#include <algorithm>
 #include <cstdint>
 #include <mutex>
 #include <string>
@@ -40,6 +41,7 @@ struct Api {
   decltype(&rcsa_quantize_rows_int8) quantize_rows_int8 = nullptr;
   decltype(&rcsa_int8_linear) int8_linear = nullptr;
   decltype(&rcsa_int8_linear_group) int8_linear_group = nullptr;
+  decltype(&rcsa_order_lists) order_lists = nullptr;
   decltype(&rcsa_block_scores) block_scores = nullptr;
   decltype(&rcsa_select_topk) select_topk = nullptr;
   decltype(&rcsa_quantize_key) quantize_key = nullptr;
@@ -71,6 +73,7 @@ void bind_library(const std::string& path) {
   bind_one(h, "rcsa_quantize_rows_int8", api.quantize_rows_int8);
   bind_one(h, "rcsa_int8_linear", api.int8_linear);
   bind_one(h, "rcsa_int8_linear_group", api.int8_linear_group);
+  bind_one(h, "rcsa_order_lists", api.order_lists);
   bind_one(h, "rcsa_block_scores", api.block_scores);
   bind_one(h, "rcsa_select_topk", api.select_topk);
   bind_one(h, "rcsa_quantize_key", api.quantize_key);
@@ -574,6 +577,54 @@ void int8_linear_group(const at::Tensor& x_i8, const at::Tensor& x_scale, at::Te
                                           dt == at::kFloat, M, K, l.stream));
 }
 
+// Ascending block lists (indices [B|1, H|1, N, maxK], counts [B|1, H|1, N], rows of
+// them, int32) and, with valid (byte flags, a multiple of 32), their bits, in one
+// launch; a list that heads or batches share (stride 0) is ordered once.
+std::vector<at::Tensor> order_lists(const at::Tensor& indices, const at::Tensor& counts,
+                                    int64_t n_kblocks, const c10::optional<at::Tensor>& rows,
+                                    const c10::optional<at::Tensor>& valid) {
+  const char* op = "order_lists";
+  const Api& a = api(op);
+  int dev = -1;
+  on_device(op, dev, indices, "indices");
+  on_device(op, dev, counts, "counts");
+  on_device(op, dev, rows, "rows");
+  on_device(op, dev, valid, "valid");
+  want(op, indices, at::kInt, "indices");
+  want(op, counts, at::kInt, "counts");
+  want(op, rows, at::kLong, "rows");
+  want_bytes(op, valid, "valid");
+  TORCH_CHECK(indices.dim() == 4 && counts.dim() == 3 && indices.stride(3) == 1 &&
+                  indices.size(2) == counts.size(2), op,
+              ": indices must be [B, H, N, maxK], lens [B, H, N]");
+  TORCH_CHECK((!rows.has_value() || rows->is_contiguous()) &&
+                  (!valid.has_value() || (valid->is_contiguous() && valid->numel() % 32 == 0)),
+              op, ": rows and valid must be contiguous, valid whole words");
+  const int64_t B = std::max(indices.size(0), counts.size(0));
+  const int64_t H = std::max(indices.size(1), counts.size(1));
+  const int64_t n_src = indices.size(2), max_k = indices.size(3);
+  const int64_t n_rows = rows.has_value() ? rows->numel() : n_src;
+  const at::Tensor idx = indices.expand({B, H, n_src, max_k}), cnt = counts.expand({B, H, n_src});
+  const int64_t b = idx.stride(0) == 0 && cnt.stride(0) == 0 ? 1 : B;
+  const int64_t h = idx.stride(1) == 0 && cnt.stride(1) == 0 ? 1 : H;
+  for (int64_t i = 0; i < 3; ++i)
+    TORCH_CHECK(idx.stride(i) >= 0 && cnt.stride(i) >= 0, op, ": strides must not be negative");
+  const Launch l(device_of(op, dev));
+  const at::Tensor out = at::empty({b, h, n_rows, max_k}, indices.options());
+  const at::Tensor lens = at::empty({b, h, n_rows}, indices.options());
+  at::Tensor bits;
+  if (valid.has_value()) bits = at::empty({valid->numel() / 32}, indices.options());
+  check_status(a, op, a.order_lists(
+      ptr<int32_t>(idx), ptr<int32_t>(cnt), idx.stride(0), idx.stride(1), idx.stride(2),
+      cnt.stride(0), cnt.stride(1), cnt.stride(2), ptr<const int64_t>(rows), n_src, b, h, n_rows,
+      max_k, n_kblocks, ptr<int32_t>(out), ptr<int32_t>(lens), ptr<const uint8_t>(valid),
+      valid.has_value() ? valid->numel() : 0, valid.has_value() ? ptr<uint32_t>(bits) : nullptr,
+      l.stream));
+  std::vector<at::Tensor> res{out.expand({B, H, n_rows, max_k}), lens.expand({B, H, n_rows})};
+  if (valid.has_value()) res.push_back(bits);
+  return res;
+}
+
 // The layer call of cast_amd/pipeline.py (rcsa_attention) in one op: its launches
 // in stream order on one stream, its outputs allocated here.  A call of a few
 // blocks is bound by the host work between its launches (4 heads x 4 query blocks
@@ -770,6 +821,9 @@ TORCH_LIBRARY(rcsa, m) {
       "int8_linear_group(Tensor x_i8, Tensor x_scale, Tensor[] w, Tensor[] w_scale, "
       "Tensor?[] bias, Tensor(a!)[] out) -> ()",
       &int8_linear_group);
+  m.def("order_lists(Tensor indices, Tensor counts, int n_kblocks, Tensor? rows, Tensor? valid) "
+        "-> Tensor[]",
+        &order_lists);
   m.def(
       "layer_call(Tensor q, Tensor k, Tensor v, Tensor? q_valid, Tensor? k_valid, int block_size, "
       "Tensor? row_k, int row_k_stride_bh, int k_fixed, int max_k, Tensor? forced, "

@@ -34,24 +34,26 @@ def longcat_active(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, indices: t
             and k.shape[2] % block_size == 0:
         # the validity as bits (32 keys a word): the attention then reads 8 bytes
         # per wavefront and block instead of staging the bytes (about 6% faster)
-        indices, counts, bits, ordered = _lists_and_bits(k, indices, counts, key_valid,
-                                                         block_size)
+        ready = _lists_and_bits(k, indices, counts, key_valid, block_size)
+        indices, counts, bits = ready or (indices, counts, ops.valid_bits(key_valid, block_size))
         return ops.sparse_attn_bf16(q, k, v, indices, counts, None, block_m=block_size,
-                                    block_n=block_size, block_mask=bits, ordered=ordered)
+                                    block_n=block_size, block_mask=bits,
+                                    ordered=ready is not None)
     return ops.sparse_attn_bf16(q, k, v, indices, counts, key_valid.to(torch.uint8).contiguous(),
                                 block_m=block_size, block_n=block_size)
 
 
 def _lists_and_bits(k, indices, counts, key_valid, block_n):
-    """The lists in ascending order where that helps (and they have the attention's
-    form; otherwise it refuses them itself) and the validity bits, in one launch."""
+    """(lists in ascending order, validity bits) from one launch where the order helps,
+    else None (also when the lists have not the attention's form, which then refuses
+    them itself)."""
     B, H, L, D = k.shape
     if (k.is_cuda and indices.is_cuda and counts.is_cuda and key_valid.is_cuda
             and indices.ndim == 4 and counts.shape == indices.shape[:3]
             and indices.shape[:2] in ((B, H), (1, H), (B, 1), (1, 1))
             and ops.order_helps(B * H, L, 4 * D, block_n, indices.shape[3])):
-        return (*ops.order_lists(indices, counts, L // block_n, valid=key_valid), True)
-    return indices, counts, ops.valid_bits(key_valid, block_n), False
+        return ops.order_lists(indices, counts, L // block_n, valid=key_valid)
+    return None
 
 
 def longcat_asymmetric(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor,
@@ -68,10 +70,12 @@ def longcat_asymmetric(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor,
              else valid.to(torch.uint8).contiguous())
     if q.shape[2] % query_block_size or k.shape[2] % key_block_size:
         raise RuntimeError("asymmetric sparse storage is not block aligned")
-    if key_block_size % 32 == 0 and valid.numel() == k.shape[2] and valid.is_cuda:
-        indices, counts, bits, ordered = _lists_and_bits(k, indices, counts, valid,
-                                                         key_block_size)
-        return ops.sparse_attn_bf16(q, k, v, indices, counts, None, block_m=query_block_size,
-                                    block_n=key_block_size, block_mask=bits, ordered=ordered)
+    if key_block_size % 32 == 0 and valid.numel() == k.shape[2]:
+        ready = _lists_and_bits(k, indices, counts, valid, key_block_size)
+        if ready is not None:  # (a few blocks: the bytes, without another launch)
+            indices, counts, bits = ready
+            return ops.sparse_attn_bf16(q, k, v, indices, counts, None,
+                                        block_m=query_block_size, block_n=key_block_size,
+                                        block_mask=bits, ordered=True)
     return ops.sparse_attn_bf16(q, k, v, indices, counts, valid, block_m=query_block_size,
                                 block_n=key_block_size)

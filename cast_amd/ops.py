@@ -657,29 +657,11 @@ def order_lists(indices: torch.Tensor, counts: torch.Tensor, n_kblocks: int, *,
     if indices.ndim != 4 or counts.ndim != 3 or indices.stride(3) != 1 \
             or indices.shape[2] != counts.shape[2]:
         raise ValueError(f"{fn}: indices must be [B, H, N, maxK], lens [B, H, N]")
-    B, H = torch.broadcast_shapes(indices.shape[:2], counts.shape[:2])
-    indices, counts = _expand_lists(indices, counts, B, H)
-    # a broadcast list is ordered once
-    b = 1 if indices.stride(0) == 0 and counts.stride(0) == 0 else B
-    h = 1 if indices.stride(1) == 0 and counts.stride(1) == 0 else H
-    n_src, max_k = indices.shape[2:]
-    n_rows = n_src
     if rows is not None:
         rows = rows.to(device=indices.device, dtype=torch.int64).contiguous()
-        n_rows = rows.numel()
-    out = torch.empty(b, h, n_rows, max_k, device=indices.device, dtype=torch.int32)
-    lens = torch.empty(b, h, n_rows, device=indices.device, dtype=torch.int32)
-    bits = None
     if valid is not None:
         valid = _bytes_mask(valid.reshape(-1), indices.device)
-        bits = torch.empty(valid.numel() // 32, device=indices.device, dtype=torch.int32)
-    check(_lib.load().rcsa_order_lists(
-        indices.data_ptr(), counts.data_ptr(), *indices.stride()[:3], *counts.stride(),
-        _ptr(rows), n_src, b, h, n_rows, max_k, int(n_kblocks), out.data_ptr(),
-        lens.data_ptr(), _ptr(valid), 0 if valid is None else valid.numel(), _ptr(bits),
-        _stream()), fn)
-    out, lens = out.expand(B, H, -1, -1), lens.expand(B, H, -1)
-    return (out, lens) if valid is None else (out, lens, bits)
+    return tuple(_lib.torch_ops().order_lists(indices, counts, int(n_kblocks), rows, valid))
 
 
 def valid_bits(valid: torch.Tensor, block_size: int) -> torch.Tensor:

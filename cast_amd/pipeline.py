@@ -271,8 +271,11 @@ def relay_attention(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, layout, s
     # device has two rounds of them (the 128-row form of that size takes the same
     # steps for every row; fewer blocks take longer steps)
     n_qblocks = rows.numel()
-    cus = torch.cuda.get_device_properties(q.device).multi_processor_count
-    half = layout.query_half if -(-B * H * n_qblocks // 8) >= 2 * (cus // 8) else None
+    half = None
+    if q.is_cuda and layout.query_half is not None:
+        cus = torch.cuda.get_device_properties(q.device).multi_processor_count
+        if -(-B * H * n_qblocks // 8) >= 2 * (cus // 8):
+            half = layout.query_half
     bm, q_slot, out_row = ((bs // 2, *half) if half is not None
                            else (bs, layout.query_slot_token, layout.query_out_row))
     scale = 1.0 / math.sqrt(D) if sm_scale is None else sm_scale

@@ -251,8 +251,8 @@ def compact_cwca_attention(weave, module: Any, q: torch.Tensor, k: torch.Tensor,
             layer = getattr(current, "rcsa_layer", None)
             if layer is not None and layer.degrees.device == dev:
                 # the whole layer's rows, memory ones at mean_degree, from one launch
-                degrees, row_k = layer.degrees64, layer.degrees
-                degrees.rcsa_layer = layer
+                degrees, row_k = layer.degrees64.view(-1), layer.degrees
+                degrees.rcsa_layer = layer  # (on a view: the layer's tensors keep no cycle)
             else:
                 layer = None
                 degrees = torch.full((blocks,), mean_degree, device=dev, dtype=torch.long)
