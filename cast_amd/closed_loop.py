@@ -37,6 +37,22 @@ _STATUS_ERRORS = ((1, "compact Current frame lies outside CWCA tiles"),
                   (2, "compact Closed-Loop CWCA exhausted key capacity"))
 
 
+def _carry(degrees: torch.Tensor, layer, rows) -> None:
+    """Let ``degrees`` carry the launch results they are a view of; ``rows``: the total
+    blocks, memory blocks and mean degree the launch was given."""
+    if not degrees.is_inference():  # (whose writes are not counted)
+        degrees.rcsa_layer = (layer, rows, degrees._version)
+
+
+def _carried(degrees: torch.Tensor, rows=None):
+    """The launch results that ``degrees`` carry; None once the degrees were written to
+    (the results hold copies of them), or for other ``rows``."""
+    layer, made_for, version = getattr(degrees, "rcsa_layer", (None, None, 0))
+    if layer is None or degrees._version != version or rows not in (None, made_for):
+        return None
+    return layer
+
+
 class _DeviceStats:
     """min / max / mean / std (population) of a device tensor, computed when
     read (``_stats`` of P/control_response_cwca_attention.py:1532-1541)."""
@@ -122,7 +138,7 @@ class DeviceClosedLoopBudget:
         pending.append(layer.status)
         # (the layer's degrees, memory rows included, ride along for the caller)
         current = layer.degrees64[int(memory_blocks):].view(cells, spatial)
-        current.rcsa_layer = layer
+        _carry(current, layer, (int(total_blocks), int(memory_blocks), int(mean_degree)))
         worldline = cells * int(mean_degree)
         current_edges = cells * spatial * int(mean_degree)
         metadata = {
@@ -151,7 +167,7 @@ class DeviceClosedLoopBudget:
                               local_support_preserved: bool, native_qk_topk: bool) -> None:
         record = dict(metadata)
         d = degrees.detach()
-        layer = getattr(degrees, "rcsa_layer", None)
+        layer = _carried(degrees)
         k_min, k_max, k_mean = ((d.min(), d.max(), d.float().mean()) if layer is None
                                 else (*layer.min_max.unbind(), layer.mean))
         record.update({

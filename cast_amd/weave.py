@@ -41,6 +41,7 @@ import torch
 
 from . import layout as rlayout
 from . import ops
+from .closed_loop import _carried, _carry
 
 
 def _cache(layout, device: torch.device) -> dict:
@@ -248,11 +249,12 @@ def compact_cwca_attention(weave, module: Any, q: torch.Tensor, k: torch.Tensor,
                 total_blocks=blocks, memory_blocks=memory_blocks)
             if int(current.numel()) != current_blocks:
                 raise RuntimeError("compact Closed-Loop degree layout differs from packed rows")
-            layer = getattr(current, "rcsa_layer", None)
+            rows = (blocks, memory_blocks, mean_degree)
+            layer = _carried(current, rows)
             if layer is not None and layer.degrees.device == dev:
                 # the whole layer's rows, memory ones at mean_degree, from one launch
                 degrees, row_k = layer.degrees64.view(-1), layer.degrees
-                degrees.rcsa_layer = layer  # (on a view: the layer's tensors keep no cycle)
+                _carry(degrees, layer, rows)  # (on a view: the layer's tensors keep no cycle)
             else:
                 layer = None
                 degrees = torch.full((blocks,), mean_degree, device=dev, dtype=torch.long)
