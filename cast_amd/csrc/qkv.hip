@@ -549,10 +549,7 @@ extern "C" int rcsa_int8_linear_group(const int8_t* x, const float* x_scale, int
   a.n_lin = static_cast<int32_t>(n_linear);
   for (int g = 0; g < a.n_lin; ++g) {
     if (!w[g] || !w_scale[g] || !out[g]) return RCSA_ERR_NULL;
-    // (the stores address a tile's rows with 32-bit offsets)
-    if (N[g] <= 0 || N[g] % BigTile::B || ldo[g] < N[g] || ldo[g] % 4 ||
-        ldo[g] >= (int64_t{1} << 30) / BigTile::B)
-      return RCSA_ERR_SHAPE;
+    if (N[g] <= 0 || N[g] % BigTile::B || ldo[g] < N[g] || ldo[g] % 4) return RCSA_ERR_SHAPE;
     if ((reinterpret_cast<uintptr_t>(w[g]) & 15u) ||
         (reinterpret_cast<uintptr_t>(w_scale[g]) & 15u) ||
         (reinterpret_cast<uintptr_t>(out[g]) & 7u) || (reinterpret_cast<uintptr_t>(bias[g]) & 7u))
@@ -563,6 +560,27 @@ extern "C" int rcsa_int8_linear_group(const int8_t* x, const float* x_scale, int
     a.out[g] = out[g];
     a.N[g] = N[g];
     a.ldo[g] = ldo[g];
+  }
+  // The stores address a tile's rows with 32-bit offsets.  Rows further apart than
+  // that (8 MiB and more each, so they are few) go one by one, in parts of a row.
+  constexpr int64_t kFar = (int64_t{1} << 30) / BigTile::B, kPart = kFar / 2;
+  bool far = false;
+  for (int g = 0; g < a.n_lin; ++g) far = far || ldo[g] >= kFar;
+  if (far) {
+    const int64_t elt = out_f32 != 0 ? 4 : 2;
+    for (int g = 0; g < a.n_lin; ++g)
+      for (int64_t r = 0; r < M; ++r)
+        for (int64_t n = 0; n < N[g]; n += kPart) {
+          const int64_t part = N[g] - n < kPart ? N[g] - n : kPart;
+          const int8_t* const wn = w[g] + n * K;
+          const float* const wsn = w_scale[g] + n;
+          const void* const bn = bias[g] ? static_cast<const char*>(bias[g]) + n * 2 : nullptr;
+          void* const on = static_cast<char*>(out[g]) + (r * ldo[g] + n) * elt;
+          const int st = rcsa_int8_linear_group(x + r * K, x_scale + r, 1, &wn, &wsn, &bn, &part,
+                                                &on, &part, out_f32, 1, K, stream);
+          if (st != RCSA_OK) return st;
+        }
+    return RCSA_OK;
   }
   // The tile size that needs less time for its whole rounds: a round of 128 x 128
   // tiles takes 5/16 of a round of 256 x 256 tiles (14 and 44 us at K 3072; three

@@ -51,6 +51,24 @@ def test_int8_linear_leaves_a_wide_output_alone(dev):
         assert (wide[M:] == 7).all() and (wide[:, 3072:] == 7).all()
 
 
+@pytest.mark.parametrize("stride", [(1 << 22) - 4, 1 << 22, (1 << 22) + 4])
+def test_int8_linear_rows_far_apart(dev, stride):
+    """Output rows at the limit of a tile's 32-bit offsets and past it."""
+    from cast_amd import ops
+    g = torch.Generator().manual_seed(3)
+    M, N = 3, 512
+    x = torch.randint(-127, 128, (M, 256), generator=g, dtype=torch.int8)
+    w = torch.randint(-127, 128, (N, 256), generator=g, dtype=torch.int8)
+    xs, ws = torch.rand(M, generator=g), torch.rand(N, generator=g)
+    bias = torch.randn(N, generator=g).bfloat16()
+    wide = torch.full((M, stride), 7.0, dtype=torch.bfloat16, device=dev)
+    ops.int8_linear(x.to(dev), xs.to(dev), w.to(dev), ws.to(dev), bias.to(dev),
+                    out=wide[:, :N])
+    wide = wide.cpu()
+    assert torch.equal(wide[:, :N], orc.int8_linear(x, xs, w, ws, bias))
+    assert (wide[:, N:] == 7).all()
+
+
 @pytest.mark.parametrize("C", [8, 1016, 1032, 2048, 3064, 5120, 5128])
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
 def test_quantize_rows_lengths(dev, C, dtype):
