@@ -22,6 +22,7 @@ RCSA_F32 = 1
 RCSA_ORDER_INDEX = 0
 RCSA_ORDER_RANK = 1
 RCSA_ORDER_RANK_LOCAL = 2
+RCSA_ORDER_SPLIT = 3
 
 _P = c_void_p
 _I = c_int64
@@ -72,6 +73,7 @@ SIGNATURES: dict[str, list] = {
     "rcsa_int8_linear": [_P, _P, _P, _P, _P, _I, _I, _I, _P, _I, _P],
     "rcsa_order_lists_max_blocks": [],
     "rcsa_order_lists": [_P, _P] + [_I] * 6 + [_P] + [_I] * 6 + [_P, _P, _P, _I, _P, _P],
+    "rcsa_order_split_lists": [_P, _P] + [_I] * 6 + [_P] + [_I] * 7 + [_P, _P, _P, _I, _P, _P],
     "rcsa_pack_tokens": [_P, c_int, _I, _I, _I, _I, _I, _I, _I, _P, _I, _P, _P],
     "rcsa_unpack_tokens": [_P, _I, _I, _I, _I, _P, _I, _P, _P],
     "rcsa_status_string": [c_int],

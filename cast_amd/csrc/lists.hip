@@ -10,6 +10,13 @@
 // LDS, and every block number is written as often as it is listed, at the
 // wavefront's running prefix.  A list of n entries over nb blocks costs
 // n + nb LDS accesses whatever its order.
+//
+// A list that the attention cuts into shares is ordered share by share: which
+// entries a share holds stays the caller's.  The shares' partial outputs are
+// rounded to bf16, and those of a run of neighbouring blocks, whose keys resemble
+// each other, are larger than those of a mixture: from float64, 1 head x 1 query
+// block x 89 of 215 key blocks in random order 1.89e-3 as given, 2.21e-3 where the
+// shares are cut from the ascending list, 1.89e-3 so.
 #include "rcsa_common.h"
 
 namespace rcsa {
@@ -23,6 +30,9 @@ struct ListArgs {
   int64_t H, n_rows, max_k;
   int32_t n_blocks;     // key blocks
   int64_t n_lists;      // B * H * n_rows
+  // lists [x xcd_items + xcd_direct, (x + 1) xcd_items) of XCD x are cut into n_split shares
+  int64_t xcd_items, xcd_direct;
+  uint32_t n_split;
   int32_t* out_idx;     // [n_lists][max_k]
   int32_t* out_lens;    // [n_lists]
   const uint8_t* valid;  // nullable
@@ -56,30 +66,42 @@ order_lists_kernel(ListArgs a, int64_t list_wgs) {
   int64_t n = a.lens[b * a.slz + h * a.slh + row * a.slm];
   n = n < 0 ? 0 : (n > a.max_k ? a.max_k : n);
   uint32_t* tally = s_tally + wave * a.n_blocks;
-  for (int j = lane; j < a.n_blocks; j += kWave) tally[j] = 0;
-  // the tallies are this wavefront's own: its LDS operations stay in order
-  __builtin_amdgcn_wave_barrier();
-  for (int64_t e = lane; e < n; e += kWave) {
-    const uint32_t j = static_cast<uint32_t>(src[e]);
-    if (j < static_cast<uint32_t>(a.n_blocks)) atomicAdd(&tally[j], 1u);
-  }
-  __builtin_amdgcn_wave_barrier();
   int32_t* out = a.out_idx + list * a.max_k;
-  uint32_t base = 0;
-  for (int j0 = 0; j0 < a.n_blocks; j0 += kWave) {
-    const int j = j0 + lane;
-    const uint32_t c = j < a.n_blocks ? tally[j] : 0u;
-    uint32_t pre = c;  // inclusive prefix over the wavefront
-#pragma unroll
-    for (int o = 1; o < kWave; o <<= 1) {
-      const uint32_t up = __shfl_up(pre, o, kWave);
-      if (lane >= o) pre += up;
+  const uint32_t ns =
+      a.n_split > 1 && list % a.xcd_items >= a.xcd_direct ? a.n_split : 1;
+  const uint32_t n32 = static_cast<uint32_t>(n);  // (n < 2^24, ns <= 16)
+  uint32_t len = n32;
+  for (uint32_t s = 0; s < ns; ++s) {
+    const uint32_t first = n32 * s / ns, end = n32 * (s + 1) / ns;  // the attention's shares
+    for (int j = lane; j < a.n_blocks; j += kWave) tally[j] = 0;
+    // the tallies are this wavefront's own: its LDS operations stay in order
+    __builtin_amdgcn_wave_barrier();
+    for (uint32_t e = first + lane; e < end; e += kWave) {
+      const uint32_t j = static_cast<uint32_t>(src[e]);
+      if (j < static_cast<uint32_t>(a.n_blocks)) atomicAdd(&tally[j], 1u);
     }
-    for (uint32_t t = 0; t < c; ++t) out[base + pre - c + t] = j;
-    base += __shfl(pre, kWave - 1, kWave);
+    __builtin_amdgcn_wave_barrier();
+    uint32_t base = first;
+    for (int j0 = 0; j0 < a.n_blocks; j0 += kWave) {
+      const int j = j0 + lane;
+      const uint32_t c = j < a.n_blocks ? tally[j] : 0u;
+      uint32_t pre = c;  // inclusive prefix over the wavefront
+#pragma unroll
+      for (int o = 1; o < kWave; o <<= 1) {
+        const uint32_t up = __shfl_up(pre, o, kWave);
+        if (lane >= o) pre += up;
+      }
+      for (uint32_t t = 0; t < c; ++t) out[base + pre - c + t] = j;
+      base += __shfl(pre, kWave - 1, kWave);
+    }
+    __builtin_amdgcn_wave_barrier();
+    // (entries that name no block leave the list, but not a share's run: the others
+    // keep theirs)
+    for (uint32_t e = base + lane; e < end; e += kWave) out[e] = -1;
+    if (ns == 1) len = base;
   }
-  for (int64_t e = base + lane; e < a.max_k; e += kWave) out[e] = -1;
-  if (lane == 0) a.out_lens[list] = static_cast<int32_t>(base);
+  for (int64_t e = n + lane; e < a.max_k; e += kWave) out[e] = -1;
+  if (lane == 0) a.out_lens[list] = static_cast<int32_t>(len);
 }
 
 }  // namespace rcsa
@@ -88,13 +110,15 @@ using namespace rcsa;
 
 extern "C" int64_t rcsa_order_lists_max_blocks(void) { return kListMaxBlocks; }
 
-extern "C" int rcsa_order_lists(const int32_t* block_indices, const int32_t* block_indices_lens,
-                                int64_t stride_bz, int64_t stride_bh, int64_t stride_bm,
-                                int64_t stride_lz, int64_t stride_lh, int64_t stride_lm,
-                                const int64_t* rows, int64_t n_src_rows, int64_t B, int64_t H,
-                                int64_t n_rows, int64_t max_k, int64_t n_kblocks,
-                                int32_t* out_indices, int32_t* out_lens, const uint8_t* valid,
-                                int64_t n_valid, uint32_t* valid_bits, hipStream_t stream) {
+extern "C" int rcsa_order_split_lists(const int32_t* block_indices,
+                                      const int32_t* block_indices_lens,
+                                      int64_t stride_bz, int64_t stride_bh, int64_t stride_bm,
+                                      int64_t stride_lz, int64_t stride_lh, int64_t stride_lm,
+                                      const int64_t* rows, int64_t n_src_rows, int64_t B,
+                                      int64_t H, int64_t n_rows, int64_t max_k,
+                                      int64_t n_kblocks, int64_t n_split, int32_t* out_indices,
+                                      int32_t* out_lens, const uint8_t* valid, int64_t n_valid,
+                                      uint32_t* valid_bits, hipStream_t stream) {
   if ((valid == nullptr) != (valid_bits == nullptr)) return RCSA_ERR_NULL;
   if (block_indices == nullptr && valid == nullptr) return RCSA_ERR_NULL;
   ListArgs a{};
@@ -106,6 +130,7 @@ extern "C" int rcsa_order_lists(const int32_t* block_indices, const int32_t* blo
         max_k >= (int64_t{1} << 24) || n_kblocks <= 0 || n_kblocks > kListMaxBlocks)
       return RCSA_ERR_SHAPE;
     if (!rows && n_rows > n_src_rows) return RCSA_ERR_SHAPE;
+    if (n_split < 1 || n_split > 16) return RCSA_ERR_SHAPE;
     a.idx = block_indices;
     a.lens = block_indices_lens;
     a.sbz = stride_bz; a.sbh = stride_bh; a.sbm = stride_bm;
@@ -117,6 +142,9 @@ extern "C" int rcsa_order_lists(const int32_t* block_indices, const int32_t* blo
     a.max_k = max_k;
     a.n_blocks = static_cast<int32_t>(n_kblocks);
     a.n_lists = B * H * n_rows;
+    a.xcd_items = (a.n_lists + kNumXcd - 1) / kNumXcd;
+    a.xcd_direct = n_split > 1 ? whole_items(a.xcd_items, cus_per_xcd()) : a.xcd_items;
+    a.n_split = static_cast<uint32_t>(n_split);
     a.out_idx = out_indices;
     a.out_lens = out_lens;
     list_wgs = (a.n_lists + kListWaves - 1) / kListWaves;
@@ -134,4 +162,17 @@ extern "C" int rcsa_order_lists(const int32_t* block_indices, const int32_t* blo
   order_lists_kernel<<<dim3(static_cast<unsigned>(list_wgs + valid_wgs)),
                        dim3(kListWaves * kWave), lds, stream>>>(a, list_wgs);
   return launch_status();
+}
+
+extern "C" int rcsa_order_lists(const int32_t* block_indices, const int32_t* block_indices_lens,
+                                int64_t stride_bz, int64_t stride_bh, int64_t stride_bm,
+                                int64_t stride_lz, int64_t stride_lh, int64_t stride_lm,
+                                const int64_t* rows, int64_t n_src_rows, int64_t B, int64_t H,
+                                int64_t n_rows, int64_t max_k, int64_t n_kblocks,
+                                int32_t* out_indices, int32_t* out_lens, const uint8_t* valid,
+                                int64_t n_valid, uint32_t* valid_bits, hipStream_t stream) {
+  return rcsa_order_split_lists(block_indices, block_indices_lens, stride_bz, stride_bh, stride_bm,
+                                stride_lz, stride_lh, stride_lm, rows, n_src_rows, B, H, n_rows,
+                                max_k, n_kblocks, 1, out_indices, out_lens, valid, n_valid,
+                                valid_bits, stream);
 }

@@ -934,7 +934,7 @@ extern "C" int rcsa_quantize_key_select(
   if (!aligned16(qhat) || !aligned16(khat)) return RCSA_ERR_ALIGN;
   const SelArgs sel{score, batch * n_heads * n_qblocks, n_qblocks, n_blocks, row_k,
                     row_k_stride_bh, k_fixed, forced, allowed, mask_stride_bh, indices, max_k,
-                    counts, false};
+                    counts, false, 0, 0};
   return quantize_key_impl(k, dtype, batch, n_heads, n_blocks, block_size, head_dim, stride_b,
                            stride_h, stride_t, valid, slot_token, src_len, ksum, kmin, kmax,
                            kmean, k_i8, k_scale, &sel, qhat, khat, stream);

@@ -86,6 +86,23 @@ inline int launch_status() {
   return e == hipSuccess ? RCSA_OK : RCSA_ERR_LAUNCH;
 }
 
+// Compute units per XCD of the current device (0 when it cannot be read);
+// one attention workgroup fills a compute unit.
+inline int64_t cus_per_xcd() {
+  int dev = 0, cus = 0;
+  if (hipGetDevice(&dev) != hipSuccess ||
+      hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess ||
+      cus < kNumXcd)
+    return 0;
+  return cus / kNumXcd;
+}
+
+// Of an XCD's query blocks, those in its full rounds: a split launch runs them
+// whole and cuts the lists of the rest.
+inline int64_t whole_items(int64_t xcd_items, int64_t cux) {
+  return cux > 0 ? xcd_items / cux * cux : xcd_items;
+}
+
 inline bool aligned16(const void* p) {
   return (reinterpret_cast<uintptr_t>(p) & 15u) == 0;
 }

@@ -33,6 +33,9 @@ struct SelArgs {
   int32_t* counts;
   // forced columns rank among themselves by fl(score + 1e6) (RCSA_ORDER_RANK_LOCAL)
   bool coarse_forced;
+  // MIXED: rank order for rows [x xcd_items + xcd_direct, (x + 1) xcd_items) only, index
+  // order for the others (RCSA_ORDER_SPLIT)
+  int64_t xcd_items, xcd_direct;
 };
 
 constexpr int kSelWaves = 4;
@@ -85,7 +88,7 @@ __device__ __forceinline__ void write_ranked(const uint32_t* v, const uint16_t* 
 
 // PER > 0: values held in registers (PER per lane, n_k <= 64 * PER).
 // PER == 0: values recomputed from memory on every pass (any n_k <= 65536).
-template <int PER, bool RANK>
+template <int PER, bool RANK, bool MIXED = false>
 __device__ __forceinline__ void select_rows(const SelArgs& a, int64_t block, char* s_rank) {
   static_assert(PER <= 32, "one forced bit per pass");
   const int lane = threadIdx.x % kWave, wave = threadIdx.x / kWave;
@@ -160,6 +163,7 @@ __device__ __forceinline__ void select_rows(const SelArgs& a, int64_t block, cha
     for (int p = 0; p < passes; ++p) above += __popcll(__ballot(cut_value(p) > thr));
     const int ties = kk - above;  // columns at the threshold to take, lowest first
 
+    const bool ranked = RANK && (!MIXED || row % a.xcd_items >= a.xcd_direct);
     const uint64_t lt_mask = (1ull << lane) - 1ull;
     const int64_t slots = RANK ? rank_slots(a.max_k) : 0;
     uint32_t* rv = RANK ? reinterpret_cast<uint32_t*>(s_rank) + wave * slots : nullptr;
@@ -179,7 +183,7 @@ __device__ __forceinline__ void select_rows(const SelArgs& a, int64_t block, cha
                        || (f && !cut_forced);
       taken += __popcll(eq);
       const uint64_t m = __ballot(sel);
-      if constexpr (RANK) {
+      if (ranked) {
         const uint64_t mf = __ballot(sel && f);
         if (sel) {
           const int s = f ? base_f + __popcll(mf & lt_mask)
@@ -193,7 +197,7 @@ __device__ __forceinline__ void select_rows(const SelArgs& a, int64_t block, cha
       }
       base += __popcll(m);
     }
-    if constexpr (RANK) {
+    if (ranked) {
       // the padding of both classes' last groups outranks nothing
       const int n_b = k_eff - n_a;
       if (lane < b0 - n_a) rv[n_a + lane] = 0;

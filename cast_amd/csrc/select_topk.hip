@@ -4,11 +4,11 @@
 
 namespace rcsa {
 
-template <int PER, bool RANK>
+template <int PER, bool RANK, bool MIXED>
 __global__ void __launch_bounds__(kSelWaves * kWave)
 select_kernel(SelArgs a) {
   extern __shared__ __attribute__((aligned(16))) char s_rank[];  // RANK: kSelWaves rank lists
-  select_rows<PER, RANK>(a, blockIdx.x, s_rank);
+  select_rows<PER, RANK, MIXED>(a, blockIdx.x, s_rank);
 }
 
 // The selection's certificate: per row the repeated neighbours of its list
@@ -74,21 +74,21 @@ __global__ void __launch_bounds__(1024) check_sum_kernel(CheckArgs a) {
   }
 }
 
-template <bool RANK>
+template <bool RANK, bool MIXED = false>
 static void launch_select(const SelArgs& a, hipStream_t stream) {
   const int64_t per = (a.n_k + kWave - 1) / kWave;
   dim3 grid(static_cast<unsigned>((a.n_rows + kSelWaves - 1) / kSelWaves));
   dim3 block(kSelWaves * kWave);
   const size_t lds = RANK ? static_cast<size_t>(kSelWaves * rank_slots(a.max_k) * kRankSlotBytes)
                           : 0;
-  if (per <= 1) select_kernel<1, RANK><<<grid, block, lds, stream>>>(a);
-  else if (per <= 2) select_kernel<2, RANK><<<grid, block, lds, stream>>>(a);
-  else if (per <= 4) select_kernel<4, RANK><<<grid, block, lds, stream>>>(a);
-  else if (per <= 6) select_kernel<6, RANK><<<grid, block, lds, stream>>>(a);
-  else if (per <= 8) select_kernel<8, RANK><<<grid, block, lds, stream>>>(a);
-  else if (per <= 16) select_kernel<16, RANK><<<grid, block, lds, stream>>>(a);
-  else if (per <= 32) select_kernel<32, RANK><<<grid, block, lds, stream>>>(a);
-  else select_kernel<0, RANK><<<grid, block, lds, stream>>>(a);
+  if (per <= 1) select_kernel<1, RANK, MIXED><<<grid, block, lds, stream>>>(a);
+  else if (per <= 2) select_kernel<2, RANK, MIXED><<<grid, block, lds, stream>>>(a);
+  else if (per <= 4) select_kernel<4, RANK, MIXED><<<grid, block, lds, stream>>>(a);
+  else if (per <= 6) select_kernel<6, RANK, MIXED><<<grid, block, lds, stream>>>(a);
+  else if (per <= 8) select_kernel<8, RANK, MIXED><<<grid, block, lds, stream>>>(a);
+  else if (per <= 16) select_kernel<16, RANK, MIXED><<<grid, block, lds, stream>>>(a);
+  else if (per <= 32) select_kernel<32, RANK, MIXED><<<grid, block, lds, stream>>>(a);
+  else select_kernel<0, RANK, MIXED><<<grid, block, lds, stream>>>(a);
 }
 
 }  // namespace rcsa
@@ -105,15 +105,23 @@ extern "C" int rcsa_select_topk(const float* score, int64_t n_bh, int64_t n_qblo
   if (!score || !indices || !counts) return RCSA_ERR_NULL;
   if (n_bh <= 0 || n_qblocks <= 0 || n_kblocks <= 0 || max_k <= 0) return RCSA_ERR_SHAPE;
   if (n_kblocks > 65536) return RCSA_ERR_SHAPE;
-  if (order != RCSA_ORDER_INDEX && order != RCSA_ORDER_RANK && order != RCSA_ORDER_RANK_LOCAL)
+  if (order != RCSA_ORDER_INDEX && order != RCSA_ORDER_RANK && order != RCSA_ORDER_RANK_LOCAL &&
+      order != RCSA_ORDER_SPLIT)
     return RCSA_ERR_SHAPE;
   if (order != RCSA_ORDER_INDEX && max_k > 2048) return RCSA_ERR_SHAPE;
   if (mask_stride_bh < 0 || row_k_stride_bh < 0) return RCSA_ERR_STRIDE;
   SelArgs a{score, n_bh * n_qblocks, n_qblocks, n_kblocks, row_k, row_k_stride_bh,
             k_fixed, forced, allowed, mask_stride_bh, indices, max_k, counts,
-            order == RCSA_ORDER_RANK_LOCAL};
-  if (order != RCSA_ORDER_INDEX) launch_select<true>(a, stream);
-  else launch_select<false>(a, stream);
+            order == RCSA_ORDER_RANK_LOCAL, 0, 0};
+  if (order == RCSA_ORDER_SPLIT) {
+    a.xcd_items = (a.n_rows + kNumXcd - 1) / kNumXcd;
+    a.xcd_direct = whole_items(a.xcd_items, cus_per_xcd());
+    launch_select<true, true>(a, stream);
+  } else if (order != RCSA_ORDER_INDEX) {
+    launch_select<true>(a, stream);
+  } else {
+    launch_select<false>(a, stream);
+  }
   return launch_status();
 }
 

@@ -6,7 +6,6 @@
 
 namespace rcsa {
 
-static int64_t cus_per_xcd();
 
 template <bool INT8>
 static int launch_attn(AttnArgs& a, int64_t D, int64_t BM, int64_t BN, hipStream_t s) {
@@ -64,17 +63,6 @@ static int launch_attn_split(AttnArgs& a, int64_t D, int64_t BM, int64_t BN, hip
   return launch_status();
 }
 
-// Compute units per XCD of the current device (0 when it cannot be read);
-// one attention workgroup fills a compute unit.
-static int64_t cus_per_xcd() {
-  int dev = 0, cus = 0;
-  if (hipGetDevice(&dev) != hipSuccess ||
-      hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess ||
-      cus < kNumXcd)
-    return 0;
-  return cus / kNumXcd;
-}
-
 // Workspace of a split launch: normalised bf16 partials, then (m, l) pairs,
 // for n_tail tail query blocks of block_m rows.
 static int64_t ws_o_bytes(int64_t n_tail, int64_t block_m, int64_t d, int64_t n_split) {
@@ -105,7 +93,7 @@ static int plan_split(AttnArgs& a, int64_t n_split) {
   const int64_t cux = cus_per_xcd();
   if (cux <= 0) return RCSA_ERR_LAUNCH;
   const int64_t p = a.xcd_items;
-  const int64_t direct = p % cux == 0 ? p : p / cux * cux;
+  const int64_t direct = whole_items(p, cux);
   if (direct == p) return RCSA_OK;  // every round full: nothing to split
   a.xcd_direct = direct;
   a.n_split = n_split;

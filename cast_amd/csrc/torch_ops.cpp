@@ -41,7 +41,7 @@ struct Api {
   decltype(&rcsa_quantize_rows_int8) quantize_rows_int8 = nullptr;
   decltype(&rcsa_int8_linear) int8_linear = nullptr;
   decltype(&rcsa_int8_linear_group) int8_linear_group = nullptr;
-  decltype(&rcsa_order_lists) order_lists = nullptr;
+  decltype(&rcsa_order_split_lists) order_split_lists = nullptr;
   decltype(&rcsa_block_scores) block_scores = nullptr;
   decltype(&rcsa_select_topk) select_topk = nullptr;
   decltype(&rcsa_quantize_key) quantize_key = nullptr;
@@ -73,7 +73,7 @@ void bind_library(const std::string& path) {
   bind_one(h, "rcsa_quantize_rows_int8", api.quantize_rows_int8);
   bind_one(h, "rcsa_int8_linear", api.int8_linear);
   bind_one(h, "rcsa_int8_linear_group", api.int8_linear_group);
-  bind_one(h, "rcsa_order_lists", api.order_lists);
+  bind_one(h, "rcsa_order_split_lists", api.order_split_lists);
   bind_one(h, "rcsa_block_scores", api.block_scores);
   bind_one(h, "rcsa_select_topk", api.select_topk);
   bind_one(h, "rcsa_quantize_key", api.quantize_key);
@@ -579,10 +579,11 @@ void int8_linear_group(const at::Tensor& x_i8, const at::Tensor& x_scale, at::Te
 
 // Ascending block lists (indices [B|1, H|1, N, maxK], counts [B|1, H|1, N], rows of
 // them, int32) and, with valid (byte flags, a multiple of 32), their bits, in one
-// launch; a list that heads or batches share (stride 0) is ordered once.
+// launch; a list that heads or batches share (stride 0) is ordered once, except for
+// a launch of n_split shares, which cuts some of them.
 std::vector<at::Tensor> order_lists(const at::Tensor& indices, const at::Tensor& counts,
                                     int64_t n_kblocks, const c10::optional<at::Tensor>& rows,
-                                    const c10::optional<at::Tensor>& valid) {
+                                    const c10::optional<at::Tensor>& valid, int64_t n_split) {
   const char* op = "order_lists";
   const Api& a = api(op);
   int dev = -1;
@@ -605,8 +606,8 @@ std::vector<at::Tensor> order_lists(const at::Tensor& indices, const at::Tensor&
   const int64_t n_src = indices.size(2), max_k = indices.size(3);
   const int64_t n_rows = rows.has_value() ? rows->numel() : n_src;
   const at::Tensor idx = indices.expand({B, H, n_src, max_k}), cnt = counts.expand({B, H, n_src});
-  const int64_t b = idx.stride(0) == 0 && cnt.stride(0) == 0 ? 1 : B;
-  const int64_t h = idx.stride(1) == 0 && cnt.stride(1) == 0 ? 1 : H;
+  const int64_t b = n_split == 1 && idx.stride(0) == 0 && cnt.stride(0) == 0 ? 1 : B;
+  const int64_t h = n_split == 1 && idx.stride(1) == 0 && cnt.stride(1) == 0 ? 1 : H;
   for (int64_t i = 0; i < 3; ++i)
     TORCH_CHECK(idx.stride(i) >= 0 && cnt.stride(i) >= 0, op, ": strides must not be negative");
   const Launch l(device_of(op, dev));
@@ -614,12 +615,12 @@ std::vector<at::Tensor> order_lists(const at::Tensor& indices, const at::Tensor&
   const at::Tensor lens = at::empty({b, h, n_rows}, indices.options());
   at::Tensor bits;
   if (valid.has_value()) bits = at::empty({valid->numel() / 32}, indices.options());
-  check_status(a, op, a.order_lists(
+  check_status(a, op, a.order_split_lists(
       ptr<int32_t>(idx), ptr<int32_t>(cnt), idx.stride(0), idx.stride(1), idx.stride(2),
       cnt.stride(0), cnt.stride(1), cnt.stride(2), ptr<const int64_t>(rows), n_src, b, h, n_rows,
-      max_k, n_kblocks, ptr<int32_t>(out), ptr<int32_t>(lens), ptr<const uint8_t>(valid),
-      valid.has_value() ? valid->numel() : 0, valid.has_value() ? ptr<uint32_t>(bits) : nullptr,
-      l.stream));
+      max_k, n_kblocks, n_split, ptr<int32_t>(out), ptr<int32_t>(lens),
+      ptr<const uint8_t>(valid), valid.has_value() ? valid->numel() : 0,
+      valid.has_value() ? ptr<uint32_t>(bits) : nullptr, l.stream));
   std::vector<at::Tensor> res{out.expand({B, H, n_rows, max_k}), lens.expand({B, H, n_rows})};
   if (valid.has_value()) res.push_back(bits);
   return res;
@@ -821,8 +822,8 @@ TORCH_LIBRARY(rcsa, m) {
       "int8_linear_group(Tensor x_i8, Tensor x_scale, Tensor[] w, Tensor[] w_scale, "
       "Tensor?[] bias, Tensor(a!)[] out) -> ()",
       &int8_linear_group);
-  m.def("order_lists(Tensor indices, Tensor counts, int n_kblocks, Tensor? rows, Tensor? valid) "
-        "-> Tensor[]",
+  m.def("order_lists(Tensor indices, Tensor counts, int n_kblocks, Tensor? rows, Tensor? valid, "
+        "int n_split=1) -> Tensor[]",
         &order_lists);
   m.def(
       "layer_call(Tensor q, Tensor k, Tensor v, Tensor? q_valid, Tensor? k_valid, int block_size, "

@@ -34,7 +34,7 @@ def longcat_active(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, indices: t
             and k.shape[2] % block_size == 0:
         # the validity as bits (32 keys a word): the attention then reads 8 bytes
         # per wavefront and block instead of staging the bytes (about 6% faster)
-        ready = _lists_and_bits(k, indices, counts, key_valid, block_size)
+        ready = _lists_and_bits(q, k, indices, counts, key_valid, block_size, block_size)
         indices, counts, bits = ready or (indices, counts, ops.valid_bits(key_valid, block_size))
         return ops.sparse_attn_bf16(q, k, v, indices, counts, None, block_m=block_size,
                                     block_n=block_size, block_mask=bits,
@@ -43,7 +43,7 @@ def longcat_active(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, indices: t
                                 block_m=block_size, block_n=block_size)
 
 
-def _lists_and_bits(k, indices, counts, key_valid, block_n):
+def _lists_and_bits(q, k, indices, counts, key_valid, block_m, block_n):
     """(lists in ascending order, validity bits) from one launch where the order helps,
     else None (also when the lists have not the attention's form, which then refuses
     them itself)."""
@@ -52,7 +52,8 @@ def _lists_and_bits(k, indices, counts, key_valid, block_n):
             and indices.ndim == 4 and counts.shape == indices.shape[:3]
             and indices.shape[:2] in ((B, H), (1, H), (B, 1), (1, 1))
             and ops.order_helps(B * H, L, 4 * D, block_n, indices.shape[3])):
-        return ops.order_lists(indices, counts, L // block_n, valid=key_valid)
+        return ops.order_for_attention(indices, counts, q.shape, L, block_m, block_n,
+                                       valid=key_valid)
     return None
 
 
@@ -71,7 +72,7 @@ def longcat_asymmetric(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor,
     if q.shape[2] % query_block_size or k.shape[2] % key_block_size:
         raise RuntimeError("asymmetric sparse storage is not block aligned")
     if key_block_size % 32 == 0 and valid.numel() == k.shape[2]:
-        ready = _lists_and_bits(k, indices, counts, valid, key_block_size)
+        ready = _lists_and_bits(q, k, indices, counts, valid, query_block_size, key_block_size)
         if ready is not None:  # (a few blocks: the bytes, without another launch)
             indices, counts, bits = ready
             return ops.sparse_attn_bf16(q, k, v, indices, counts, None,

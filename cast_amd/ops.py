@@ -14,7 +14,7 @@ import torch
 
 from . import _lib
 from ._lib import (RCSA_BF16, RCSA_F32, RCSA_ORDER_INDEX, RCSA_ORDER_RANK,
-                   RCSA_ORDER_RANK_LOCAL, check)
+                   RCSA_ORDER_RANK_LOCAL, RCSA_ORDER_SPLIT, check)
 
 __all__ = [
     "pool_query", "pool_key", "block_scores", "select_topk", "quantize_key",
@@ -415,9 +415,10 @@ def select_topk(score: torch.Tensor, k, *, forced: Optional[torch.Tensor] = None
     Order of preference: forced, then score descending, then block index
     ascending (the stable-argsort tie rule of
     P/qk_uncertainty_tangent_attention.py:978-980); "rank_local" ranks the forced
-    blocks among themselves by the fp32 value of score + 1e6.  ``k`` is an int, or an
-    int tensor of shape [NQ] (shared by heads) or [NBH, NQ].  Returns
-    ``(indices int32 [NBH, NQ, max_k], counts int32 [NBH, NQ])``; unused
+    blocks among themselves by the fp32 value of score + 1e6, and "split" is the rank order
+    for the rows whose lists a split attention launch cuts, index order for the others.
+    ``k`` is an int, or an int tensor of shape [NQ] (shared by heads) or [NBH, NQ].
+    Returns ``(indices int32 [NBH, NQ, max_k], counts int32 [NBH, NQ])``; unused
     slots hold -1.
     """
     fn = "select_topk"
@@ -439,7 +440,7 @@ def select_topk(score: torch.Tensor, k, *, forced: Optional[torch.Tensor] = None
 
 
 _ORDERS = {"index": RCSA_ORDER_INDEX, "rank": RCSA_ORDER_RANK,
-           "rank_local": RCSA_ORDER_RANK_LOCAL}
+           "rank_local": RCSA_ORDER_RANK_LOCAL, "split": RCSA_ORDER_SPLIT}
 
 
 def select_check(selected: torch.Tensor, counts: torch.Tensor, local: torch.Tensor,
@@ -490,7 +491,7 @@ def _selection_args(nbh, nq, nk, k, forced, allowed, max_k, order, device, fn):
     if max_k is None:
         max_k = max(1, min(kmax, nk))
     if order not in _ORDERS:
-        raise ValueError(f"{fn}: order must be 'index', 'rank' or 'rank_local'")
+        raise ValueError(f"{fn}: order must be one of {', '.join(_ORDERS)}")
     fm, fstride = _mask_u8(forced, nbh, nq, nk, device, fn)
     am, astride = _mask_u8(allowed, nbh, nq, nk, device, fn)
     if fm is not None and am is not None and fstride != astride:
@@ -599,18 +600,31 @@ def _split_plan(B, H, Lq, D, block_m, max_k, n_split, device, fn):
     ``n_split=None`` asks the library for the count that fills the device's
     compute units best (rcsa_attn_split_plan); the workspace holds the
     partial results that the merge pass combines."""
-    lib = _lib.load()
     if n_split is None:
-        ns = ctypes.c_int64(1)
-        check(lib.rcsa_attn_split_plan(B, H, Lq, block_m, max_k, ctypes.byref(ns)), fn)
-        n_split = ns.value
+        n_split = _planned_split(B, H, Lq, block_m, max_k, fn)
     n_split = int(n_split)
     if n_split < 1:
         raise ValueError(f"{fn}: n_split must be >= 1")
     if n_split == 1:
         return 1, None, 0
-    nbytes = int(lib.rcsa_attn_workspace_bytes(B, H, Lq, D, n_split))
+    nbytes = int(_lib.load().rcsa_attn_workspace_bytes(B, H, Lq, D, n_split))
     return n_split, torch.empty(nbytes, dtype=torch.uint8, device=device), nbytes
+
+
+def _planned_split(B, H, Lq, block_m, max_k, fn) -> int:
+    ns = ctypes.c_int64(1)
+    check(_lib.load().rcsa_attn_split_plan(B, H, Lq, block_m, max_k, ctypes.byref(ns)), fn)
+    return ns.value
+
+
+def split_rows(B: int, H: int, Lq: int, block_m: int, max_k: int) -> str:
+    """Of the attention's query blocks, those whose lists it cuts into shares by its own
+    choice of n_split: "none", "some" (each XCD's past its full rounds) or "all"."""
+    if _planned_split(B, H, Lq, block_m, max_k, "split_rows") == 1:
+        return "none"
+    per_xcd = -(-B * H * -(-Lq // block_m) // 8)
+    cus = torch.cuda.get_device_properties(torch.cuda.current_device()).multi_processor_count
+    return "some" if per_xcd >= cus // 8 else "all"
 
 
 def _expand_lists(indices, counts, B, H):
@@ -647,12 +661,16 @@ def order_helps(n_bh: int, k_len: int, key_bytes: int, block_n: int, max_k: int)
 
 
 def order_lists(indices: torch.Tensor, counts: torch.Tensor, n_kblocks: int, *,
-                rows: Optional[torch.Tensor] = None, valid: Optional[torch.Tensor] = None):
-    """Block lists in ascending block order (``rcsa_order_lists``): ``(indices, counts)``
+                rows: Optional[torch.Tensor] = None, valid: Optional[torch.Tensor] = None,
+                n_split: int = 1):
+    """Block lists in ascending block order (``rcsa_order_split_lists``): ``(indices, counts)``
     of the entries in ``[0, n_kblocks)``, repeats kept.  indices int32 ``[B|1, H|1, N,
     maxK]``, counts int32 ``[B|1, H|1, N]``; ``rows`` (int64) picks rows of them.  With
     ``valid`` (one flag per key, a multiple of 32) a third value follows: its bits as
-    :func:`valid_bits` gives them, flat, from the same launch."""
+    :func:`valid_bits` gives them, flat, from the same launch.  With ``n_split`` (B, H and
+    the rows then being those of the attention call that is given it) the lists that this
+    call cuts are ordered share by share, each share keeping its entries: its partial
+    output is rounded to bf16, and that of a run of an ascending list is larger."""
     fn = "order_lists"
     _require_cuda(fn, indices, counts)
     if indices.dtype != torch.int32 or counts.dtype != torch.int32:
@@ -664,7 +682,22 @@ def order_lists(indices: torch.Tensor, counts: torch.Tensor, n_kblocks: int, *,
         rows = rows.to(device=indices.device, dtype=torch.int64).contiguous()
     if valid is not None:
         valid = _bytes_mask(valid.reshape(-1), indices.device)
-    return tuple(_lib.torch_ops().order_lists(indices, counts, int(n_kblocks), rows, valid))
+    return tuple(_lib.torch_ops().order_lists(indices, counts, int(n_kblocks), rows, valid,
+                                              int(n_split)))
+
+
+def order_for_attention(indices, counts, q_shape, k_len: int, block_m: int, block_n: int,
+                        n_split: Optional[int] = None, rows=None, valid=None):
+    """:func:`order_lists` for the attention over ``q_shape`` ([B, H, Lq, ...]) with this
+    ``n_split`` (None: the one that the call will choose)."""
+    B, H, Lq = q_shape[:3]
+    indices, counts = _expand_lists(indices, counts, B, H)
+    if n_split is None:
+        n_split = _planned_split(B, H, Lq, block_m, indices.shape[3], "order_lists")
+    elif not 1 <= int(n_split) <= 16:  # (refused by the attention)
+        n_split = 1
+    return order_lists(indices, counts, -(-k_len // block_n), rows=rows, valid=valid,
+                       n_split=n_split)
 
 
 def valid_bits(valid: torch.Tensor, block_size: int) -> torch.Tensor:
@@ -759,7 +792,8 @@ def sparse_attn_bf16(q, k, v, indices, counts, valid=None, *, block_m=128, block
     else:
         kv = _valid_u8(valid, Lk, q.device, fn)
     if not ordered and order_helps(B * H, Lk, 4 * D, block_n, indices.shape[3]):
-        indices, counts = order_lists(indices, counts, -(-Lk // block_n))
+        indices, counts = order_for_attention(indices, counts, (B, H, Lq), Lk, block_m, block_n,
+                                              n_split)
     n_rows = n_out if gathered else Lq
     if out is None:
         out = (torch.empty(B, n_out, H, D, device=q.device, dtype=torch.bfloat16) if gathered
@@ -832,7 +866,8 @@ def sparse_attn_int8(q_i8, q_scale, k_i8, k_scale, v, indices, counts, valid=Non
     else:
         kv = _valid_u8(valid, Lk, q_i8.device, fn)
     if not ordered and order_helps(B * H, Lk, 3 * D, block_n, indices.shape[3]):
-        indices, counts = order_lists(indices, counts, nkb)
+        indices, counts = order_for_attention(indices, counts, (B, H, Lq), Lk, block_m, block_n,
+                                              n_split)
     if out_token is not None:
         om = _slot_map(out_token, block_m, q_i8.device, fn)
         if om.numel() < Lq or out_len is None or int(out_len) <= 0:

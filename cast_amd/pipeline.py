@@ -262,7 +262,8 @@ def relay_attention(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, layout, s
                and ops.order_helps(B * H, n_kblocks * bs, (3 if int8 else 4) * D, bs,
                                    selected.shape[3]))
     if ordered:  # the query blocks' rows, ascending, in one launch
-        idx, cnt = ops.order_lists(selected, counts, n_kblocks, rows=rows)
+        idx, cnt = ops.order_for_attention(selected, counts, (B, H, rows.numel() * bs),
+                                           n_kblocks * bs, bs, bs, n_split, rows=rows)
     else:
         idx = selected.index_select(2, rows).to(torch.int32).contiguous()
         cnt = counts.index_select(2, rows).to(torch.int32).contiguous()

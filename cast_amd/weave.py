@@ -328,10 +328,16 @@ def compact_cwca_attention(weave, module: Any, q: torch.Tensor, k: torch.Tensor,
     # ---- top-k at each row's degree, local blocks first (:5829-5832) ----
     if row_k is None:
         row_k = degrees.to(torch.int32)
-    # only the router reads the rank order; the attention takes ascending lists
-    ordered = route != "refine"
+    # The router reads the rank order; the attention takes ascending lists, but in rank
+    # order those that it cuts into shares: a share of an ascending list is a run of
+    # neighbouring frames, whose partial output is larger and rounds further off (1 head,
+    # 8 + 12 frames, int8: 2.44e-3 from float64, 2.41e-3 in rank order).  Where it cuts
+    # them all, it orders every share itself.
+    cut = ops.split_rows(B, H, blocks * bs, bs, width)
+    ordered = route != "refine" and cut != "all"
     indices, _ = ops.select_topk(score, row_k, forced=local, max_k=width,
-                                 order="index" if ordered else "rank")
+                                 order="rank" if not ordered else
+                                 "index" if cut == "none" or width > 2048 else "split")
     selected = indices.view(B, H, blocks, width)
     counts = row_k[None, None].expand(B, H, -1)
     if not ordered:  # the router's own kernels read it whole

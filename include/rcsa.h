@@ -46,8 +46,11 @@ enum { RCSA_BF16 = 0, RCSA_F32 = 1 };
 enum {
   RCSA_ORDER_INDEX = 0, /* ascending block index (what the attention kernel streams best) */
   RCSA_ORDER_RANK = 1,  /* descending rank: forced first, then score desc, index asc */
-  RCSA_ORDER_RANK_LOCAL = 2 /* rank order, the forced columns among themselves by the
+  RCSA_ORDER_RANK_LOCAL = 2, /* rank order, the forced columns among themselves by the
                                fp32 value of score + 1e6 (as score + 1e6 * local ranks) */
+  RCSA_ORDER_SPLIT = 3      /* for a split attention launch over these rows: rank order where
+                               it cuts the list into shares (the rows of an XCD's run past
+                               its full rounds), ascending block index elsewhere */
 };
 
 /* Human-readable text for a status code (static storage). */
@@ -617,6 +620,14 @@ int rcsa_route_check(const int32_t* base, const int32_t* selected, const int32_t
  * valid (one byte per key, n_valid of them) with valid_bits (ceil(n_valid / 32)
  * words: bit i of word w = key 32 w + i), both or neither, in the same launch;
  * block_indices may be NULL when only the bits are wanted.
+ *
+ * rcsa_order_split_lists: for an attention launch over B, H and n_rows query
+ * blocks that is given n_split (1 to 16).  The lists that the launch will cut into
+ * shares (a split entry point's tail query blocks) keep their length and each
+ * share's entries, [floor(len s / n_split), floor(len (s + 1) / n_split)) for share s,
+ * in ascending order there, -1 for those that name no block.  (A share's partial
+ * output is rounded to bf16, and that of a run of neighbouring blocks is larger
+ * than that of a mixture: shares of the ascending list would round further off.)
  */
 int64_t rcsa_order_lists_max_blocks(void);
 int rcsa_order_lists(const int32_t* block_indices, const int32_t* block_indices_lens,
@@ -626,6 +637,13 @@ int rcsa_order_lists(const int32_t* block_indices, const int32_t* block_indices_
                      int64_t n_rows, int64_t max_k, int64_t n_kblocks, int32_t* out_indices,
                      int32_t* out_lens, const uint8_t* valid, int64_t n_valid,
                      uint32_t* valid_bits, hipStream_t stream);
+int rcsa_order_split_lists(const int32_t* block_indices, const int32_t* block_indices_lens,
+                           int64_t stride_bz, int64_t stride_bh, int64_t stride_bm,
+                           int64_t stride_lz, int64_t stride_lh, int64_t stride_lm,
+                           const int64_t* rows, int64_t n_src_rows, int64_t B, int64_t H,
+                           int64_t n_rows, int64_t max_k, int64_t n_kblocks, int64_t n_split,
+                           int32_t* out_indices, int32_t* out_lens, const uint8_t* valid,
+                           int64_t n_valid, uint32_t* valid_bits, hipStream_t stream);
 
 /*
  * Shared int8 Q/K/V projection (P/matrix_shared_int8_qkv.py:19-92): the

@@ -91,3 +91,82 @@ def test_attention_over_ordered_lists(int8):
     a, b = run().float(), run(ordered=True).float()
     assert torch.allclose(a, b, rtol=2 ** -7, atol=2 ** -9)
     assert not a[0, 1, :128].any()  # the empty list
+
+
+@pytest.mark.parametrize("ns", [2, 3, 7, 16])
+@pytest.mark.parametrize("N,H", [(28, 24), (5, 3), (64, 4)])
+def test_lists_of_a_split_launch(ns, N, H):
+    """The lists of an XCD's query blocks past its full rounds, which the launch cuts into
+    shares, keep every share's entries (those that name no block last, as -1) and are
+    ascending within it; the others are ascending."""
+    from cast_amd import ops
+    cux = torch.cuda.get_device_properties(0).multi_processor_count // 8
+    g = torch.Generator().manual_seed(ns + N)
+    nkb, K = 70, 50
+    idx = torch.randint(-1, nkb + 2, (1, 1, N, K), generator=g, dtype=torch.int32)
+    cnt = torch.randint(0, K + 3, (1, 1, N), generator=g, dtype=torch.int32)
+    cnt[0, 0, :4] = torch.tensor([0, 1, ns, ns + 1])  # shares without an entry
+    got, lens = ops.order_lists(idx.cuda().expand(1, H, N, K), cnt.cuda().expand(1, H, N), nkb,
+                                n_split=ns)
+    want, want_lens = _want(idx, cnt, nkb, range(N))
+    cut = torch.full((N, K), -1, dtype=torch.int32)  # the lists as the launch cuts them
+    for r in range(N):
+        n = min(int(cnt[0, 0, r]), K)
+        for s in range(ns):
+            a, b = n * s // ns, n * (s + 1) // ns
+            live = sorted(j for j in idx[0, 0, r, a:b].tolist() if 0 <= j < nkb)
+            cut[r, a:a + len(live)] = torch.tensor(live, dtype=torch.int32)
+    per = -(-H * N // 8)
+    item = torch.arange(H * N)
+    tail = (item % per >= per // cux * cux)[:, None]
+    row = item % N
+    assert torch.equal(got.cpu().reshape(H * N, K), torch.where(tail, cut[row], want[0, 0, row]))
+    assert torch.equal(lens.cpu().reshape(-1),
+                       torch.where(tail[:, 0], cnt[0, 0].clamp_max(K)[row], want_lens[0, 0, row]))
+
+
+@pytest.mark.parametrize("int8", [False, True])
+@pytest.mark.parametrize("H,Lq,ns", [(1, 128, 4), (2, 256, None), (8, 512, 2)])
+def test_ordered_shares_round_no_further(int8, H, Lq, ns):
+    """Split lists that the library orders stay as close to float64 as in the random
+    order they came in, for values that resemble each other within a frame (a share's
+    partial output is rounded to bf16; contiguous shares of an ascending list are 10 to
+    20 per cent further off).  Both sides round the same partial outputs, up to the order
+    of the sums in them; each is a mean over at least 16384 values, whose error varies by
+    less than 1 per cent."""
+    from cast_amd import ops
+    dev, D, nkb, keys = "cuda", 128, 210, 90
+    g = torch.Generator(device=dev).manual_seed(4)
+
+    def tokens(n):
+        frames = torch.randn(1, H, -(-n // 880), D, device=dev, generator=g) * 0.3
+        x = torch.randn(1, H, n, D, device=dev, generator=g) / D ** 0.5
+        return (x + frames.repeat_interleave(880, 2)[:, :, :n]).bfloat16()
+    q, k, v = tokens(Lq), tokens(nkb * 128), tokens(nkb * 128)
+    rows = Lq // 128
+    idx = torch.rand(1, H, rows, nkb, device=dev, generator=g).argsort(-1)[..., :keys].int()
+    idx = idx.contiguous()
+    cnt = torch.full((1, H, rows), keys, dtype=torch.int32, device=dev)
+    assert ops.order_helps(H, nkb * 128, (3 if int8 else 4) * D, 128, keys)
+    if int8:
+        _, q8, qs = ops.pool_query(q, None, 128, quantize=True)
+        _, ks, kn, kx = ops.pool_key(k, None, 128, stats=True)
+        k8, sc, kmean = ops.quantize_key(k, None, 128, ks, kn, kx)
+        qd = q8.double().view(1, H, rows, 128, D) * qs.view(1, H, rows, 1, 1).double()
+        kd = k8.double().view(1, H, nkb, 128, D) * sc.view(1, H, nkb, 1, 1).double()
+        qd, kd = qd.view(1, H, Lq, D), kd.view(1, H, nkb * 128, D)
+        run = lambda **kw: ops.sparse_attn_int8(q8, qs, k8, sc, v, idx, cnt, n_split=ns, **kw)
+    else:
+        qd, kd = q.double(), k.double()
+        run = lambda **kw: ops.sparse_attn_bf16(q, k, v, idx, cnt, n_split=ns, **kw)
+    ref = torch.empty(1, H, Lq, D, dtype=torch.float64, device=dev)
+    for h in range(H):
+        for r in range(rows):
+            tok = (idx[0, h, r].long()[:, None] * 128 + torch.arange(128, device=dev)).reshape(-1)
+            p = torch.softmax(qd[0, h, r * 128:(r + 1) * 128] @ kd[0, h, tok].T / D ** 0.5, -1)
+            ref[0, h, r * 128:(r + 1) * 128] = p @ v[0, h, tok].double()
+    err = lambda x: ((x.double() - ref).norm() / ref.norm()).item()
+    given, ours = err(run(ordered=True)), err(run())
+    print(f"ordered shares int8 {int8} H {H} n_split {ns}: {given:.4e} as given, {ours:.4e}",
+          flush=True)
+    assert ours <= 1.02 * given

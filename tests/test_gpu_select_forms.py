@@ -66,6 +66,26 @@ def test_select_forms(dev, nk, order):
             assert idx[r].tolist() == w + [-1] * (max_k - len(w)), (r, order)
 
 
+@pytest.mark.parametrize("nbh,nq,nk", [(24, 28, 130), (3, 130, 65), (2, 9, 40)])
+def test_select_split_order(dev, nbh, nq, nk):
+    """Rank order for the rows past the full rounds of an XCD's run, index order for the
+    others (all, some and none of the rows)."""
+    from cast_amd import ops
+    g = torch.Generator().manual_seed(nk)
+    score = torch.randn(nbh, nq, nk, generator=g).to(dev)
+    forced = (torch.rand(nq, nk, generator=g) < 0.1).to(dev)
+    k = torch.randint(0, 30, (nq,), generator=g).to(dev)
+    args = dict(forced=forced, max_k=30)
+    got, cnt = ops.select_topk(score, k, order="split", **args)
+    rank, want_cnt = ops.select_topk(score, k, order="rank", **args)
+    index, _ = ops.select_topk(score, k, order="index", **args)
+    per = -(-nbh * nq // 8)
+    cux = torch.cuda.get_device_properties(0).multi_processor_count // 8
+    tail = (torch.arange(nbh * nq) % per >= per // cux * cux).view(nbh, nq, 1).to(dev)
+    assert torch.equal(cnt, want_cnt)
+    assert torch.equal(got, torch.where(tail, rank, index))
+
+
 def test_select_check_sums(dev):
     from cast_amd import ops
     g = torch.Generator().manual_seed(3)

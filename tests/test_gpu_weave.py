@@ -310,3 +310,26 @@ def test_woven_layers_in_sequence_int8(dev):
         "compact_cwca_curvature_bootstrap"] + \
         ["compact_centered_multiplicative_curvature_control_response_lambda_0.6"] * 2
     assert [r["previous_layer"] for r in recs] == [None, 0, 1]
+
+
+def test_woven_lists_of_cut_rows_stay_ranked(dev):
+    """Lists that the attention cuts into shares (every one here: one head of 120 query blocks)
+    go to it in rank order, the stencil's blocks first: shares of the ascending list round
+    further off."""
+    from cast_amd import layout as rlayout
+    from cast_amd import ops
+    q, k, v, curvature, response = _inputs(5)
+    q, k, v = (x[:, :, :1].contiguous().to(dev) for x in (q, k, v))
+    lay = _layout(dev)
+    prov = _provider(curvature.to(dev))
+    prov._responses[0] = response.to(dev)
+    cap = {}
+    _run(_weave(prov), q, k, v, lay, 1, cap)
+    sel, cnt = cap["selected"].cpu().long(), cap["counts"].cpu()
+    n = sel.shape[2]
+    assert ops.split_rows(1, 1, n * 128, 128, sel.shape[3]) == "all"
+    local = rlayout.local_stencil(n, 6, 5)
+    for r in range(n):
+        near = torch.nonzero(local[r]).flatten().tolist()
+        assert int(cnt[0, 0, r]) >= len(near)
+        assert sorted(sel[0, 0, r, :len(near)].tolist()) == near
