@@ -49,8 +49,9 @@ def _lists_and_bits(q, k, indices, counts, key_valid, block_m, block_n):
     them itself)."""
     B, H, L, D = k.shape
     if (k.is_cuda and indices.is_cuda and counts.is_cuda and key_valid.is_cuda
-            and indices.ndim == 4 and counts.shape == indices.shape[:3]
-            and indices.shape[:2] in ((B, H), (1, H), (B, 1), (1, 1))
+            and indices.ndim == 4 and counts.ndim == 3
+            and all(t.shape[:2] in ((B, H), (1, H), (B, 1), (1, 1)) for t in (indices, counts))
+            and ops.lists_cover(indices, counts, q.shape[2], block_m)
             and ops.order_helps(B * H, L, 4 * D, block_n, indices.shape[3])):
         return ops.order_for_attention(indices, counts, q.shape, L, block_m, block_n,
                                        valid=key_valid)

@@ -686,12 +686,22 @@ def order_lists(indices: torch.Tensor, counts: torch.Tensor, n_kblocks: int, *,
                                               int(n_split)))
 
 
+def lists_cover(indices, counts, q_len: int, block_m: int) -> bool:
+    """Whether lists and lengths have a row for every query block (either may have more:
+    the attention reads those it needs)."""
+    return min(indices.shape[2], counts.shape[2]) * block_m >= q_len
+
+
 def order_for_attention(indices, counts, q_shape, k_len: int, block_m: int, block_n: int,
                         n_split: Optional[int] = None, rows=None, valid=None):
     """:func:`order_lists` for the attention over ``q_shape`` ([B, H, Lq, ...]) with this
-    ``n_split`` (None: the one that the call will choose)."""
+    ``n_split`` (None: the one that the call will choose).  Without ``rows`` the first rows
+    are its query blocks (:func:`lists_cover`); more are left out."""
     B, H, Lq = q_shape[:3]
     indices, counts = _expand_lists(indices, counts, B, H)
+    if rows is None:
+        nqb = -(-Lq // block_m)
+        indices, counts = indices[:, :, :nqb], counts[:, :, :nqb]
     if n_split is None:
         n_split = _planned_split(B, H, Lq, block_m, indices.shape[3], "order_lists")
     elif not 1 <= int(n_split) <= 16:  # (refused by the attention)
@@ -791,7 +801,8 @@ def sparse_attn_bf16(q, k, v, indices, counts, valid=None, *, block_m=128, block
         kv = None
     else:
         kv = _valid_u8(valid, Lk, q.device, fn)
-    if not ordered and order_helps(B * H, Lk, 4 * D, block_n, indices.shape[3]):
+    if not ordered and order_helps(B * H, Lk, 4 * D, block_n, indices.shape[3]) \
+            and lists_cover(indices, counts, Lq, block_m):
         indices, counts = order_for_attention(indices, counts, (B, H, Lq), Lk, block_m, block_n,
                                               n_split)
     n_rows = n_out if gathered else Lq
@@ -865,7 +876,8 @@ def sparse_attn_int8(q_i8, q_scale, k_i8, k_scale, v, indices, counts, valid=Non
         kv = None
     else:
         kv = _valid_u8(valid, Lk, q_i8.device, fn)
-    if not ordered and order_helps(B * H, Lk, 3 * D, block_n, indices.shape[3]):
+    if not ordered and order_helps(B * H, Lk, 3 * D, block_n, indices.shape[3]) \
+            and lists_cover(indices, counts, Lq, block_m):
         indices, counts = order_for_attention(indices, counts, (B, H, Lq), Lk, block_m, block_n,
                                               n_split)
     if out_token is not None:

@@ -170,3 +170,36 @@ def test_ordered_shares_round_no_further(int8, H, Lq, ns):
     print(f"ordered shares int8 {int8} H {H} n_split {ns}: {given:.4e} as given, {ours:.4e}",
           flush=True)
     assert ours <= 1.02 * given
+
+
+@pytest.mark.parametrize("int8", [False, True])
+def test_rows_past_the_query_blocks(int8):
+    """Lists and lengths may each have more rows than the query has blocks, whatever the
+    size of the keys; fewer are refused by the attention."""
+    from cast_amd import ops
+    from cast_amd.kernel import longcat_active
+    g = torch.Generator(device="cuda").manual_seed(6)
+    H, Lq, D = 2, 256, 128
+    for nkb in (20, 90):  # keys within an XCD's L2, and beyond it
+        q, k, v = (torch.randn(1, H, n, D, device="cuda", generator=g).bfloat16()
+                   for n in (Lq, nkb * 128, nkb * 128))
+        idx = torch.rand(1, H, 4, nkb, device="cuda", generator=g).argsort(-1)[..., :9].int()
+        idx, cnt = idx.contiguous(), torch.full((1, H, 3), 9, dtype=torch.int32, device="cuda")
+        if int8:
+            _, q8, qs = ops.pool_query(q, None, 128, quantize=True)
+            _, ks, kn, kx = ops.pool_key(k, None, 128, stats=True)
+            k8, sc, _ = ops.quantize_key(k, None, 128, ks, kn, kx)
+            run = lambda i, c: ops.sparse_attn_int8(q8, qs, k8, sc, v, i, c)
+        else:
+            run = lambda i, c: ops.sparse_attn_bf16(q, k, v, i, c)
+        want = run(idx[:, :, :2].contiguous(), cnt[:, :, :2].contiguous())
+        assert ops.order_helps(H, nkb * 128, (3 if int8 else 4) * D, 128, 9) == (nkb == 90)
+        for i, c in ((idx, cnt), (idx[:, :, :2], cnt), (idx, cnt[:, :, :2].contiguous())):
+            assert torch.equal(run(i, c), want)
+        with pytest.raises(RuntimeError, match="spans"):
+            run(idx[:, :, :1].contiguous(), cnt)
+        if not int8:
+            flags = torch.ones(nkb * 128, dtype=torch.bool, device="cuda")
+            got = [longcat_active(q, k, v, i, c, flags, 128)
+                   for i, c in ((idx, cnt), (idx[:, :, :2], cnt[:, :, :2]))]
+            assert torch.equal(*got)
