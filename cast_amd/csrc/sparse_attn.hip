@@ -13,10 +13,8 @@ static int launch_attn(AttnArgs& a, int64_t D, int64_t BM, int64_t BN, hipStream
   const dim3 grid(static_cast<unsigned>(kNumXcd * per_xcd));
   const int64_t cux = cus_per_xcd();
   const bool cu3 = cux > 0 && a.xcd_items >= 2 * cux;
-  // gathered sources need validity bits, D 128 and 128-key blocks; 64-row query
-  // blocks two rounds of them
-  if (a.kv_tok != nullptr && !(a.kmask != nullptr && D == 128 && BN == 128 &&
-                               (BM == 128 || cu3)))
+  // gathered sources need validity bits, D 128 and 128-key blocks
+  if (a.kv_tok != nullptr && !(a.kmask != nullptr && D == 128 && BN == 128))
     return RCSA_ERR_SHAPE;
   // D 128, 128 x 128 blocks: 3-slot rings.  With at least two full rounds of
   // query blocks per XCD, three 4-wavefront workgroups per compute unit

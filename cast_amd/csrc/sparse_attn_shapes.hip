@@ -33,9 +33,10 @@ static int launch_form(AttnArgs& a, dim3 grid, hipStream_t s) {
   return launch_status();
 }
 
-// 64-row query blocks over gathered sources (a relay layer whose blocks hold at
-// most 64 query tokens: two frames, int8, 24 heads x 30 blocks, the relay call
-// takes 401 us against 472 with 128-row blocks)
+// 64-row query blocks over gathered sources, any number of them (a relay layer whose
+// blocks hold at most 64 query tokens uses them for two rounds and more of query
+// blocks: two frames, int8, 24 heads x 30 blocks, the relay call takes 401 us
+// against 472 with 128-row blocks)
 template <bool INT8>
 static int launch_half_gather(AttnArgs& a, dim3 grid, hipStream_t s) {
   sparse_attn_kernel<INT8, 128, 64, 128, 32, 1, true, true, 2><<<grid, dim3(128), 0, s>>>(a);

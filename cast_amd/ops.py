@@ -750,7 +750,7 @@ def sparse_attn_bf16(q, k, v, indices, counts, valid=None, *, block_m=128, block
     afterwards); None picks it from the device's compute-unit count.
 
     ``q_token`` / ``kv_token`` (slot -> token maps of the packed query and key
-    slots, both or neither; needs ``block_mask``, D 128, 128-token blocks):
+    slots, both or neither; needs ``block_mask``, D 128, 128-key blocks):
     q is token-major ``[B, Lq_tokens, H, D]`` and k, v ``[B, Lk_tokens, H, D]``;
     the kernel reads their rows through the maps (the q[:, flat] / k[:, flat] /
     v[:, flat] packing of P/matrix_curvature_phase_frame_weave.py:5677-5684)
@@ -837,7 +837,7 @@ def sparse_attn_int8(q_i8, q_scale, k_i8, k_scale, v, indices, counts, valid=Non
     LSE into ``[B, H, out_len]``): ``unpack_tokens`` fused into the epilogue
     (P/matrix_curvature_phase_frame_weave.py:6095).  Every token must own a slot.
     ``v_token`` (a slot -> token map of the packed keys; needs ``block_mask``,
-    D 128, 128-token blocks) reads V rows from a token-major ``[B, Lv_tokens, H, D]``
+    D 128, 128-key blocks) reads V rows from a token-major ``[B, Lv_tokens, H, D]``
     v through the map inside the attention's copy ring (the v[:, flat] packing
     of P/matrix_curvature_phase_frame_weave.py:5677-5684); empty slots read zeros.
     ``ordered``: the lists are ascending already (:func:`order_lists` is not run)."""

@@ -405,7 +405,7 @@ int rcsa_sparse_attn_int8(const int8_t* Q, const float* q_scale,
  * to row out_token[r] of [B, out_len, H, D] / [B, H, out_len] (-1 rows are
  * dropped), as out_token does for the int8 variant; with out_token NULL they
  * go to row q_token[r] of q_tokens rows.  Needs K_block_mask,
- * HEAD_DIM 128, BLOCK_M = BLOCK_N = 128, K_LEN a multiple of 128 and
+ * HEAD_DIM 128, BLOCK_N 128 (BLOCK_M 64 or 128), K_LEN a multiple of 128 and
  * kv_len x (V, bf16 also K) row stride below 2^31 bytes; else RCSA_ERR_SHAPE.
  */
 int rcsa_sparse_attn_bf16_split(const void* Q, const void* K, const void* V,

@@ -270,3 +270,43 @@ def test_gathered_call_repeats_bit_exact_at_layer_size(int8):
         if not torch.equal(got, want):
             bad.append(it)
     assert not bad, f"calls {bad} differ"
+
+
+@pytest.mark.parametrize("int8", [True, False])
+@pytest.mark.parametrize("n_split", [1, 3])
+@pytest.mark.parametrize("heads", [1, 24])
+def test_half_query_blocks_read_through_maps(heads, n_split, int8):
+    """64-row query blocks over gathered sources, a few of them and more than two rounds
+    (24 heads x 28): the call on packed sources up to the order of its sums (bf16 outputs:
+    half a place either side; an empty list's rows are zero in both)."""
+    from cast_amd import ops
+    dev = torch.device("cuda:0")
+    g = torch.Generator().manual_seed(51 + n_split)
+    B, D, nqb, nkb, max_k, n_tok = 1, 128, 28, 12, 7, 1400
+    k_tok, v_tok = (torch.randn(B, n_tok, heads, D, generator=g).bfloat16().to(dev)
+                    for _ in range(2))
+    kmap = _holey_map(n_tok, nkb * 128, g, dev)
+    kp, vp = ops.pack_tokens(k_tok, kmap), ops.pack_tokens(v_tok, kmap)
+    _, ksum, kmin, kmax, mask = ops.pool_key(kp, (kmap >= 0) & (kmap < n_tok), 128, stats=True,
+                                             block_mask=True)
+    idx = torch.rand(B, heads, nqb, nkb, generator=g).argsort(-1)[..., :max_k].int().to(dev)
+    cnt = torch.randint(0, max_k + 1, (B, heads, nqb), generator=g, dtype=torch.int32).to(dev)
+    kw = dict(block_m=64, block_mask=mask, return_lse=True, n_split=n_split)
+    print(f"half blocks: heads {heads} n_split {n_split} int8 {int8}", flush=True)
+    if int8:
+        qp = torch.randn(B, heads, nqb * 64, D, generator=g).bfloat16().to(dev)
+        _, q8, qs = ops.pool_query(qp, None, 64, quantize=True)
+        k8, ks, _ = ops.quantize_key(kp, (kmap >= 0) & (kmap < n_tok), 128, ksum, kmin, kmax)
+        want, want_lse = ops.sparse_attn_int8(q8, qs, k8, ks, vp, idx, cnt, **kw)
+        got, lse = ops.sparse_attn_int8(q8, qs, k8, ks, v_tok, idx, cnt, v_token=kmap, **kw)
+    else:
+        q_tok = torch.randn(B, nqb * 64, heads, D, generator=g).bfloat16().to(dev)
+        qmap = torch.randperm(nqb * 64, generator=g).int().to(dev)
+        want, want_lse = ops.sparse_attn_bf16(ops.pack_tokens(q_tok, qmap), kp, vp, idx, cnt, **kw)
+        got, lse = ops.sparse_attn_bf16(q_tok, k_tok, v_tok, idx, cnt, q_token=qmap,
+                                        kv_token=kmap, **kw)
+        got, lse = got[:, qmap.long()].transpose(1, 2), lse[:, :, qmap.long()]
+    torch.testing.assert_close(got.float(), want.float(), rtol=2.0 ** -7, atol=2.0 ** -9)
+    fin = torch.isfinite(want_lse)
+    assert torch.equal(fin, torch.isfinite(lse))
+    torch.testing.assert_close(lse[fin], want_lse[fin], rtol=0, atol=1e-4)
