@@ -106,8 +106,9 @@ def rcsa_attention(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor,
         B, H, Lq, D = q.shape
         Lk = k.shape[2]
     bs = block_size
+    ring_maps = v_token is not None and q_slot_token.ndim == k_slot_token.ndim == 1
     if overlap and fuse_select and order == "index" and _one_op(q, k, v, bs, Lq, Lk, int8, gathered,
-                                                                v_token is not None, n_split):
+                                                                ring_maps, n_split):
         return _layer_call(q, k, v, q_valid, k_valid, bs, Lq, Lk, k_select, forced, allowed, int8,
                            max_k, sm_scale, return_lse, n_split,
                            q_slot_token if gathered else None,
@@ -188,7 +189,7 @@ def rcsa_attention(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor,
                       kmean, k_mask)
 
 
-def _one_op(q, k, v, bs, Lq, Lk, int8, gathered, ring_gather, n_split) -> bool:
+def _one_op(q, k, v, bs, Lq, Lk, int8, gathered, ring_maps, n_split) -> bool:
     """Whether the call runs as the native op: well-formed operands (the general path
     words the errors of the others), and no selection worth a stream of its own, i.e.
     one inside the key quantiser's launch, no quantiser (bf16), or one of a few
@@ -203,7 +204,7 @@ def _one_op(q, k, v, bs, Lq, Lk, int8, gathered, ring_gather, n_split) -> bool:
     D = q.shape[3]
     if (k.shape[0], k.shape[heads], k.shape[3]) != (q.shape[0], q.shape[heads], D) \
             or D not in (64, 128) or bs not in (64, 128) or min(Lq, Lk) <= 0 \
-            or Lq % bs or Lk % bs or (gathered and not ring_gather) \
+            or Lq % bs or Lk % bs or (gathered and not ring_maps) \
             or (n_split is not None and int(n_split) < 1):
         return False
     if not int8 or (q.dtype == torch.bfloat16 and D == 128 and bs == 128 and Lk // bs <= 1024):

@@ -71,3 +71,14 @@ def test_layer_op_refuses_as_before(dev):
         rcsa_attention(q, q, q, None, None, forced=torch.ones(3, 1, device=dev), **args)
     with pytest.raises(TypeError):
         rcsa_attention(q, q.float(), q, None, None, **args)
+
+
+@pytest.mark.parametrize("int8", [True, False])
+def test_layer_op_refuses_maps_that_are_no_vectors(dev, int8):
+    from cast_amd.pipeline import rcsa_attention
+    q = torch.zeros(1, 256, 1, 128, dtype=torch.bfloat16, device=dev)
+    slots = torch.arange(256, dtype=torch.int32, device=dev)
+    for qm, km in ((slots.view(2, 128), slots), (slots, slots.view(2, 128))):
+        with pytest.raises(ValueError, match="slot map must be a vector"):
+            rcsa_attention(q, q, q, None, None, block_size=128, k_select=1, int8=int8,
+                           q_slot_token=qm, k_slot_token=km)
