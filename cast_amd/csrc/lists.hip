@@ -6,7 +6,7 @@
 // workgroups of a head sweep its keys together and share them in their XCD's
 // L2; in score order each re-reads them from the Infinity Cache or HBM.
 //
-// One wavefront sorts one list by counting: entries are tallied per block in
+// One wavefront sorts one list (or one share of it) by counting: entries are tallied per block in
 // LDS, and every block number is written as often as it is listed, at the
 // wavefront's running prefix.  A list of n entries over nb blocks costs
 // n + nb LDS accesses whatever its order.
@@ -43,7 +43,9 @@ struct ListArgs {
 constexpr int kListWaves = 4;
 constexpr int64_t kListMaxBlocks = 4096;  // LDS tallies: 4 x 16 KiB
 
-// Workgroups [0, list_wgs): kListWaves lists each.  The rest: 256 flags each.
+// Workgroups [0, list_wgs): kListWaves wavefronts, n_split for each list (those
+// of a list that is not cut but its first end at once: shares side by side take
+// as long as one).  The rest: 256 flags each.
 __global__ void __launch_bounds__(kListWaves * kWave)
 order_lists_kernel(ListArgs a, int64_t list_wgs) {
   extern __shared__ uint32_t s_tally[];  // kListWaves * n_blocks
@@ -56,52 +58,49 @@ order_lists_kernel(ListArgs a, int64_t list_wgs) {
       a.bits[first / 32 + lane] = static_cast<uint32_t>(m >> (32 * lane));
     return;
   }
-  const int64_t list = static_cast<int64_t>(blockIdx.x) * kListWaves + wave;
+  const int64_t unit = static_cast<int64_t>(blockIdx.x) * kListWaves + wave;
+  const int64_t list = unit / a.n_split;
+  const uint32_t s = static_cast<uint32_t>(unit % a.n_split);
   if (list >= a.n_lists) return;  // whole wavefronts; no barrier below
+  const bool cut = a.n_split > 1 && list % a.xcd_items >= a.xcd_direct;
+  if (!cut && s > 0) return;
+  const uint32_t ns = cut ? a.n_split : 1;
   const int64_t r = list % a.n_rows, bh = list / a.n_rows;
   const int64_t b = bh / a.H, h = bh % a.H;
   int64_t row = a.rows ? a.rows[r] : r;
   row = row < 0 ? 0 : (row < a.n_src_rows ? row : a.n_src_rows - 1);
   const int32_t* src = a.idx + b * a.sbz + h * a.sbh + row * a.sbm;
-  int64_t n = a.lens[b * a.slz + h * a.slh + row * a.slm];
-  n = n < 0 ? 0 : (n > a.max_k ? a.max_k : n);
+  int64_t n64 = a.lens[b * a.slz + h * a.slh + row * a.slm];
+  n64 = n64 < 0 ? 0 : (n64 > a.max_k ? a.max_k : n64);
+  const uint32_t n = static_cast<uint32_t>(n64);  // (< 2^24, ns <= 16)
+  const uint32_t first = n * s / ns, end = n * (s + 1) / ns;  // the attention's shares
   uint32_t* tally = s_tally + wave * a.n_blocks;
-  int32_t* out = a.out_idx + list * a.max_k;
-  const uint32_t ns =
-      a.n_split > 1 && list % a.xcd_items >= a.xcd_direct ? a.n_split : 1;
-  const uint32_t n32 = static_cast<uint32_t>(n);  // (n < 2^24, ns <= 16)
-  uint32_t len = n32;
-  for (uint32_t s = 0; s < ns; ++s) {
-    const uint32_t first = n32 * s / ns, end = n32 * (s + 1) / ns;  // the attention's shares
-    for (int j = lane; j < a.n_blocks; j += kWave) tally[j] = 0;
-    // the tallies are this wavefront's own: its LDS operations stay in order
-    __builtin_amdgcn_wave_barrier();
-    for (uint32_t e = first + lane; e < end; e += kWave) {
-      const uint32_t j = static_cast<uint32_t>(src[e]);
-      if (j < static_cast<uint32_t>(a.n_blocks)) atomicAdd(&tally[j], 1u);
-    }
-    __builtin_amdgcn_wave_barrier();
-    uint32_t base = first;
-    for (int j0 = 0; j0 < a.n_blocks; j0 += kWave) {
-      const int j = j0 + lane;
-      const uint32_t c = j < a.n_blocks ? tally[j] : 0u;
-      uint32_t pre = c;  // inclusive prefix over the wavefront
-#pragma unroll
-      for (int o = 1; o < kWave; o <<= 1) {
-        const uint32_t up = __shfl_up(pre, o, kWave);
-        if (lane >= o) pre += up;
-      }
-      for (uint32_t t = 0; t < c; ++t) out[base + pre - c + t] = j;
-      base += __shfl(pre, kWave - 1, kWave);
-    }
-    __builtin_amdgcn_wave_barrier();
-    // (entries that name no block leave the list, but not a share's run: the others
-    // keep theirs)
-    for (uint32_t e = base + lane; e < end; e += kWave) out[e] = -1;
-    if (ns == 1) len = base;
+  for (int j = lane; j < a.n_blocks; j += kWave) tally[j] = 0;
+  // the tallies are this wavefront's own: its LDS operations stay in order
+  __builtin_amdgcn_wave_barrier();
+  for (uint32_t e = first + lane; e < end; e += kWave) {
+    const uint32_t j = static_cast<uint32_t>(src[e]);
+    if (j < static_cast<uint32_t>(a.n_blocks)) atomicAdd(&tally[j], 1u);
   }
-  for (int64_t e = n + lane; e < a.max_k; e += kWave) out[e] = -1;
-  if (lane == 0) a.out_lens[list] = static_cast<int32_t>(len);
+  __builtin_amdgcn_wave_barrier();
+  int32_t* out = a.out_idx + list * a.max_k;
+  uint32_t base = first;
+  for (int j0 = 0; j0 < a.n_blocks; j0 += kWave) {
+    const int j = j0 + lane;
+    const uint32_t c = j < a.n_blocks ? tally[j] : 0u;
+    uint32_t pre = c;  // inclusive prefix over the wavefront
+#pragma unroll
+    for (int o = 1; o < kWave; o <<= 1) {
+      const uint32_t up = __shfl_up(pre, o, kWave);
+      if (lane >= o) pre += up;
+    }
+    for (uint32_t t = 0; t < c; ++t) out[base + pre - c + t] = j;
+    base += __shfl(pre, kWave - 1, kWave);
+  }
+  // entries that name no block leave a whole list; a share keeps its place in it
+  const int64_t stop = s + 1 < ns ? end : a.max_k;
+  for (int64_t e = base + lane; e < stop; e += kWave) out[e] = -1;
+  if (s == 0 && lane == 0) a.out_lens[list] = static_cast<int32_t>(cut ? n : base);
 }
 
 }  // namespace rcsa
@@ -147,7 +146,7 @@ extern "C" int rcsa_order_split_lists(const int32_t* block_indices,
     a.n_split = static_cast<uint32_t>(n_split);
     a.out_idx = out_indices;
     a.out_lens = out_lens;
-    list_wgs = (a.n_lists + kListWaves - 1) / kListWaves;
+    list_wgs = (a.n_lists * n_split + kListWaves - 1) / kListWaves;
     lds = static_cast<size_t>(kListWaves * n_kblocks) * sizeof(uint32_t);
   }
   int64_t valid_wgs = 0;

@@ -37,25 +37,37 @@ def longcat_active(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, indices: t
         ready = _lists_and_bits(q, k, indices, counts, key_valid, block_size, block_size)
         indices, counts, bits = ready or (indices, counts, ops.valid_bits(key_valid, block_size))
         return ops.sparse_attn_bf16(q, k, v, indices, counts, None, block_m=block_size,
-                                    block_n=block_size, block_mask=bits,
-                                    ordered=ready is not None)
+                                    block_n=block_size, block_mask=bits, ordered=True)
     return ops.sparse_attn_bf16(q, k, v, indices, counts, key_valid.to(torch.uint8).contiguous(),
                                 block_m=block_size, block_n=block_size)
 
 
 def _lists_and_bits(q, k, indices, counts, key_valid, block_m, block_n):
-    """(lists in ascending order, validity bits) from one launch where the order helps,
+    """(lists in ascending order, validity bits) from one launch where the order pays,
     else None (also when the lists have not the attention's form, which then refuses
     them itself)."""
     B, H, L, D = k.shape
-    if (k.is_cuda and indices.is_cuda and counts.is_cuda and key_valid.is_cuda
-            and indices.ndim == 4 and counts.ndim == 3
+    if not (indices.ndim == 4 and k.is_cuda
+            and ops.order_pays(B * H, q.shape[2], L, 4 * D, block_m, block_n, indices.shape[3])):
+        return None
+    if (indices.is_cuda and counts.is_cuda and key_valid.is_cuda and counts.ndim == 3
             and all(t.shape[:2] in ((B, H), (1, H), (B, 1), (1, 1)) for t in (indices, counts))
-            and ops.lists_cover(indices, counts, q.shape[2], block_m)
-            and ops.order_helps(B * H, L, 4 * D, block_n, indices.shape[3])):
+            and ops.lists_cover(indices, counts, q.shape[2], block_m)):
         return ops.order_for_attention(indices, counts, q.shape, L, block_m, block_n,
                                        valid=key_valid)
     return None
+
+
+def _bits_pay(q, k, block_m, block_n, max_k) -> bool:
+    """Whether the validity as bits, whose forms of the attention are faster, is worth the
+    launch that makes them: keys beyond an XCD's L2, and two rounds of query blocks or
+    48 MB of listed blocks (64 x 128 blocks, 24 heads x 3520 rows x 12 of 42 blocks 102 us
+    against 145 with bytes, 8 x 1760 x 38 of 128 63 against 71, x 12 31 against 29)."""
+    B, H, L, D = k.shape
+    n_bh = B * H
+    return (k.is_cuda and ops.order_helps(n_bh, L, 4 * D, block_n, max_k)
+            and (ops.two_rounds(n_bh, q.shape[2], block_m)
+                 or ops.listed_bytes(n_bh, q.shape[2], 4 * D, block_m, block_n, max_k) > 48 << 20))
 
 
 def longcat_asymmetric(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor,
@@ -74,10 +86,15 @@ def longcat_asymmetric(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor,
         raise RuntimeError("asymmetric sparse storage is not block aligned")
     if key_block_size % 32 == 0 and valid.numel() == k.shape[2]:
         ready = _lists_and_bits(q, k, indices, counts, valid, query_block_size, key_block_size)
-        if ready is not None:  # (a few blocks: the bytes, without another launch)
+        bits = None
+        if ready is not None:
             indices, counts, bits = ready
+        elif indices.ndim == 4 and _bits_pay(q, k, query_block_size, key_block_size,
+                                             indices.shape[3]):
+            bits = ops.valid_bits(valid, key_block_size)
+        if bits is not None:  # (a few blocks: the bytes, without another launch)
             return ops.sparse_attn_bf16(q, k, v, indices, counts, None,
                                         block_m=query_block_size, block_n=key_block_size,
                                         block_mask=bits, ordered=True)
     return ops.sparse_attn_bf16(q, k, v, indices, counts, valid, block_m=query_block_size,
-                                block_n=key_block_size)
+                                block_n=key_block_size, ordered=True)

@@ -647,17 +647,46 @@ _L2_BYTES = 4 << 20  # one XCD's L2
 
 
 def order_helps(n_bh: int, k_len: int, key_bytes: int, block_n: int, max_k: int) -> bool:
-    """Whether the attention orders its block lists: when the K and V rows
-    (``key_bytes`` per key) of the heads an XCD works on exceed its L2, ascending
-    lists let the query blocks of a head share what they stream (bf16, 24 heads x
-    28 query blocks x 85 of 303 key blocks listed at random: the attention takes
-    473 us ordered against 540 us as given, the ordering itself under 5).  Smaller
-    planes stay in L2 in any order.  Past the line with it, 8 heads x 3520 queries:
-    53 us as given, 54 ordered at 4.3 MB a head, 124 and 123 at 12 MB; 64-row blocks,
-    1760 queries: 49 and 47, 121 and 107; relay, 24 heads: 61 and 58 at 17 MB, 219 and
-    164 at 34 MB."""
+    """Whether ascending block lists can spare the attention cache misses: the K and V
+    rows (``key_bytes`` per key) of the heads an XCD works on exceed its L2.  Smaller
+    planes stay there in any order."""
     return (max_k > 2 and -(-n_bh // 8) * k_len * key_bytes > _L2_BYTES
             and -(-k_len // block_n) <= _lib.load().rcsa_order_lists_max_blocks())
+
+
+def listed_bytes(n_bh: int, q_len: int, key_bytes: int, block_m: int, block_n: int,
+                 max_k: int) -> int:
+    """What the query blocks of one XCD stream, at most."""
+    return -(-n_bh * -(-q_len // block_m) // 8) * max_k * block_n * key_bytes
+
+
+def two_rounds(n_bh: int, q_len: int, block_m: int) -> bool:
+    """Whether every XCD has two rounds of query blocks: the attention then runs several
+    workgroups to a compute unit."""
+    cus = torch.cuda.get_device_properties(torch.cuda.current_device()).multi_processor_count
+    return -(-n_bh * -(-q_len // block_m) // 8) >= 2 * (cus // 8)
+
+
+def order_pays(n_bh: int, q_len: int, k_len: int, key_bytes: int, block_m: int, block_n: int,
+               max_k: int, int8: bool = False) -> bool:
+    """Whether the ordering launch (5 us, with host work 13) gains more than it costs.
+
+    64-row query blocks are bound by what they stream: from 2.5 L2s of keys and 48 MB of
+    listed blocks on (8 heads x 1760 rows x 81 of 272 blocks: 122 us ordered, 131 as
+    given; 24 x 1760 x 19 of 64: 77 and 94; below it 24 x 880 x 12 of 42: 52 and 48).
+    128-row blocks are bound by the matrix cores until several workgroups share a
+    compute unit and the keys are six times the L2 (bf16, 24 heads x 3520 rows x 90 of 303
+    blocks: 545 ordered, 628 as given; x 27 of 90: 155 and 156; 8 heads x 3520 x 115 of
+    384: 217 and 212); int8 keys, which stream less, only with more work (24 x 3520 x 91
+    of 303 blocks: 424 and 446; x 25 of 256: 131 and 124)."""
+    if not order_helps(n_bh, k_len, key_bytes, block_n, max_k):
+        return False
+    plane = -(-n_bh // 8) * k_len * key_bytes
+    listed = listed_bytes(n_bh, q_len, key_bytes, block_m, block_n, max_k)
+    if block_m <= 64:
+        return plane > 10 << 20 and listed > 48 << 20
+    return (plane > 24 << 20 and listed > (256 if int8 else 96) << 20
+            and two_rounds(n_bh, q_len, block_m))
 
 
 def order_lists(indices: torch.Tensor, counts: torch.Tensor, n_kblocks: int, *,
@@ -756,7 +785,7 @@ def sparse_attn_bf16(q, k, v, indices, counts, valid=None, *, block_m=128, block
     v[:, flat] packing of P/matrix_curvature_phase_frame_weave.py:5677-5684)
     and writes the output (and LSE) to the token rows, ``[B, Lq_tokens, H, D]``
     (P/matrix_curvature_phase_frame_weave.py:6095).  Empty slots read zeros.
-    ``ordered``: the lists are ascending already (:func:`order_lists` is not run).
+    ``ordered``: the lists are read as they are (:func:`order_lists` is not run).
     ``out_token`` / ``out_len`` (with the maps) write output row r to row
     ``out_token[r]`` of ``[B, out_len, H, D]`` instead, e.g. a relay layer's
     query-frame rows (P/matrix_curvature_phase_frame_weave.py:8990-8994).
@@ -801,7 +830,7 @@ def sparse_attn_bf16(q, k, v, indices, counts, valid=None, *, block_m=128, block
         kv = None
     else:
         kv = _valid_u8(valid, Lk, q.device, fn)
-    if not ordered and order_helps(B * H, Lk, 4 * D, block_n, indices.shape[3]) \
+    if not ordered and order_pays(B * H, Lq, Lk, 4 * D, block_m, block_n, indices.shape[3]) \
             and lists_cover(indices, counts, Lq, block_m):
         indices, counts = order_for_attention(indices, counts, (B, H, Lq), Lk, block_m, block_n,
                                               n_split)
@@ -840,7 +869,7 @@ def sparse_attn_int8(q_i8, q_scale, k_i8, k_scale, v, indices, counts, valid=Non
     D 128, 128-key blocks) reads V rows from a token-major ``[B, Lv_tokens, H, D]``
     v through the map inside the attention's copy ring (the v[:, flat] packing
     of P/matrix_curvature_phase_frame_weave.py:5677-5684); empty slots read zeros.
-    ``ordered``: the lists are ascending already (:func:`order_lists` is not run)."""
+    ``ordered``: the lists are read as they are (:func:`order_lists` is not run)."""
     fn = "sparse_attn_int8"
     _require_cuda(fn, q_i8, q_scale, k_i8, k_scale, v, indices, counts)
     _attn_common(q_i8, k_i8, v, indices, counts, fn)
@@ -876,7 +905,7 @@ def sparse_attn_int8(q_i8, q_scale, k_i8, k_scale, v, indices, counts, valid=Non
         kv = None
     else:
         kv = _valid_u8(valid, Lk, q_i8.device, fn)
-    if not ordered and order_helps(B * H, Lk, 3 * D, block_n, indices.shape[3]) \
+    if not ordered and order_pays(B * H, Lq, Lk, 3 * D, block_m, block_n, indices.shape[3], True) \
             and lists_cover(indices, counts, Lq, block_m):
         indices, counts = order_for_attention(indices, counts, (B, H, Lq), Lk, block_m, block_n,
                                               n_split)

@@ -69,7 +69,7 @@ def test_order_lists_refuses():
 
 @pytest.mark.parametrize("int8", [False, True])
 def test_attention_over_ordered_lists(int8):
-    """The attention orders lists whose keys exceed an XCD's L2: the result is that
+    """Lists in ascending order, for keys that exceed an XCD's L2: the result is that
     of the given order up to the rounding of its sums (bf16 output: half a unit in
     the last place either side, 2^-8 relative, of values below 1)."""
     from cast_amd import ops
@@ -85,10 +85,11 @@ def test_attention_over_ordered_lists(int8):
         _, q8, qs = ops.pool_query(q, None, 128, quantize=True)
         _, ks, kn, kx = ops.pool_key(k, None, 128, stats=True)
         k8, sc, _ = ops.quantize_key(k, None, 128, ks, kn, kx)
-        run = lambda **kw: ops.sparse_attn_int8(q8, qs, k8, sc, v, idx, cnt, **kw)
+        run = lambda i, c: ops.sparse_attn_int8(q8, qs, k8, sc, v, i, c, ordered=True)
     else:
-        run = lambda **kw: ops.sparse_attn_bf16(q, k, v, idx, cnt, **kw)
-    a, b = run().float(), run(ordered=True).float()
+        run = lambda i, c: ops.sparse_attn_bf16(q, k, v, i, c, ordered=True)
+    a = run(*ops.order_for_attention(idx, cnt, q.shape, Lk, 128, 128)).float()
+    b = run(idx, cnt).float()
     assert torch.allclose(a, b, rtol=2 ** -7, atol=2 ** -9)
     assert not a[0, 1, :128].any()  # the empty list
 
@@ -155,10 +156,10 @@ def test_ordered_shares_round_no_further(int8, H, Lq, ns):
         qd = q8.double().view(1, H, rows, 128, D) * qs.view(1, H, rows, 1, 1).double()
         kd = k8.double().view(1, H, nkb, 128, D) * sc.view(1, H, nkb, 1, 1).double()
         qd, kd = qd.view(1, H, Lq, D), kd.view(1, H, nkb * 128, D)
-        run = lambda **kw: ops.sparse_attn_int8(q8, qs, k8, sc, v, idx, cnt, n_split=ns, **kw)
+        run = lambda i, c: ops.sparse_attn_int8(q8, qs, k8, sc, v, i, c, n_split=ns, ordered=True)
     else:
         qd, kd = q.double(), k.double()
-        run = lambda **kw: ops.sparse_attn_bf16(q, k, v, idx, cnt, n_split=ns, **kw)
+        run = lambda i, c: ops.sparse_attn_bf16(q, k, v, i, c, n_split=ns, ordered=True)
     ref = torch.empty(1, H, Lq, D, dtype=torch.float64, device=dev)
     for h in range(H):
         for r in range(rows):
@@ -166,7 +167,8 @@ def test_ordered_shares_round_no_further(int8, H, Lq, ns):
             p = torch.softmax(qd[0, h, r * 128:(r + 1) * 128] @ kd[0, h, tok].T / D ** 0.5, -1)
             ref[0, h, r * 128:(r + 1) * 128] = p @ v[0, h, tok].double()
     err = lambda x: ((x.double() - ref).norm() / ref.norm()).item()
-    given, ours = err(run(ordered=True)), err(run())
+    given = err(run(idx, cnt))
+    ours = err(run(*ops.order_for_attention(idx, cnt, q.shape, nkb * 128, 128, 128, ns)))
     print(f"ordered shares int8 {int8} H {H} n_split {ns}: {given:.4e} as given, {ours:.4e}",
           flush=True)
     assert ours <= 1.02 * given
@@ -174,32 +176,50 @@ def test_ordered_shares_round_no_further(int8, H, Lq, ns):
 
 @pytest.mark.parametrize("int8", [False, True])
 def test_rows_past_the_query_blocks(int8):
-    """Lists and lengths may each have more rows than the query has blocks, whatever the
-    size of the keys; fewer are refused by the attention."""
+    """Lists and lengths may each have more rows than the query has blocks, whether the
+    call orders them or not; fewer are refused by the attention."""
     from cast_amd import ops
-    from cast_amd.kernel import longcat_active
+    from cast_amd.kernel import longcat_asymmetric
     g = torch.Generator(device="cuda").manual_seed(6)
-    H, Lq, D = 2, 256, 128
-    for nkb in (20, 90):  # keys within an XCD's L2, and beyond it
+    H, Lq, D, K = 2, 1024, 128, 300
+    nqb = Lq // 64
+    for nkb in (20, 400):
         q, k, v = (torch.randn(1, H, n, D, device="cuda", generator=g).bfloat16()
                    for n in (Lq, nkb * 128, nkb * 128))
-        idx = torch.rand(1, H, 4, nkb, device="cuda", generator=g).argsort(-1)[..., :9].int()
-        idx, cnt = idx.contiguous(), torch.full((1, H, 3), 9, dtype=torch.int32, device="cuda")
+        idx = torch.rand(1, H, nqb + 2, 400, device="cuda", generator=g).argsort(-1)[..., :K]
+        idx = idx.int().contiguous()  # (the short keys: most entries name no block)
+        cnt = torch.full((1, H, nqb + 1), K, dtype=torch.int32, device="cuda")
         if int8:
-            _, q8, qs = ops.pool_query(q, None, 128, quantize=True)
+            _, q8, qs = ops.pool_query(q, None, 64, quantize=True)
             _, ks, kn, kx = ops.pool_key(k, None, 128, stats=True)
             k8, sc, _ = ops.quantize_key(k, None, 128, ks, kn, kx)
-            run = lambda i, c: ops.sparse_attn_int8(q8, qs, k8, sc, v, i, c)
+            run = lambda i, c: ops.sparse_attn_int8(q8, qs, k8, sc, v, i, c, block_m=64)
         else:
-            run = lambda i, c: ops.sparse_attn_bf16(q, k, v, i, c)
-        want = run(idx[:, :, :2].contiguous(), cnt[:, :, :2].contiguous())
-        assert ops.order_helps(H, nkb * 128, (3 if int8 else 4) * D, 128, 9) == (nkb == 90)
-        for i, c in ((idx, cnt), (idx[:, :, :2], cnt), (idx, cnt[:, :, :2].contiguous())):
+            run = lambda i, c: ops.sparse_attn_bf16(q, k, v, i, c, block_m=64)
+        i0, c0 = idx[:, :, :nqb].contiguous(), cnt[:, :, :nqb].contiguous()
+        want = run(i0, c0)
+        assert ops.order_pays(H, Lq, nkb * 128, (3 if int8 else 4) * D, 64, 128, K,
+                              int8) == (nkb == 400)
+        for i, c in ((idx, cnt), (idx[:, :, :nqb], cnt), (idx, c0)):
             assert torch.equal(run(i, c), want)
         with pytest.raises(RuntimeError, match="spans"):
             run(idx[:, :, :1].contiguous(), cnt)
         if not int8:
             flags = torch.ones(nkb * 128, dtype=torch.bool, device="cuda")
-            got = [longcat_active(q, k, v, i, c, flags, 128)
-                   for i, c in ((idx, cnt), (idx[:, :, :2], cnt[:, :, :2]))]
+            got = [longcat_asymmetric(q, k, v, i, c, flags, query_block_size=64,
+                                      key_block_size=128) for i, c in ((idx, cnt), (i0, c0))]
             assert torch.equal(*got)
+
+
+# either side of every line of the two rules (bytes of a listed block: 64 KiB bf16)
+@pytest.mark.parametrize("bm,H,Lq,nkb,K,int8,pays", [
+    (64, 8, 1760, 161, 28, False, True), (64, 8, 1760, 161, 27, False, False),
+    (64, 8, 1760, 160, 28, False, False), (128, 24, 3520, 129, 19, False, True),
+    (128, 24, 3520, 129, 18, False, False), (128, 24, 3520, 128, 19, False, False),
+    (128, 24, 1760, 303, 90, False, False), (128, 24, 3520, 303, 66, True, True),
+    (128, 24, 3520, 303, 65, True, False), (128, 8, 3520, 60, 60, False, False)])
+def test_order_rule(bm, H, Lq, nkb, K, int8, pays):
+    from cast_amd import ops
+    if torch.cuda.get_device_properties(0).multi_processor_count != 256:
+        pytest.skip("sizes for 256 compute units")
+    assert ops.order_pays(H, Lq, nkb * 128, (3 if int8 else 4) * 128, bm, 128, K, int8) == pays
