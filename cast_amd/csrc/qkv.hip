@@ -408,8 +408,7 @@ int8_linear_kernel(LinearArgs a, int32_t per_wg, int32_t per_xcd) {
           const uint32_t row = wm * 32 * T + m * 32 + i * (kWave / L::CH);
           // (no scalar offset: with one, the compiler lets the next instruction
           // overwrite the registers that a 16-byte store is still reading)
-          const int voff = static_cast<int>(row * row_bytes + lane_out) +
-                           np * 64 * static_cast<int>(kOutBytes);
+          const int voff = static_cast<int>(row * row_bytes + lane_out + np * 64u * kOutBytes);
           if constexpr (OUT32) {
             const v4u lo = {v[0] << 16, v[0] & 0xffff0000u, v[1] << 16, v[1] & 0xffff0000u};
             const v4u hi = {v[2] << 16, v[2] & 0xffff0000u, v[3] << 16, v[3] & 0xffff0000u};
@@ -561,13 +560,13 @@ extern "C" int rcsa_int8_linear_group(const int8_t* x, const float* x_scale, int
     a.N[g] = N[g];
     a.ldo[g] = ldo[g];
   }
-  // The stores address a tile's rows with 32-bit offsets.  Rows further apart than
-  // that (8 MiB and more each, so they are few) go one by one, in parts of a row.
-  constexpr int64_t kFar = (int64_t{1} << 30) / BigTile::B, kPart = kFar / 2;
+  // The stores address a tile's rows with offsets below 2^31.  Rows 8 MiB and more
+  // apart (so they are few) go one by one, in parts of a row.
+  constexpr int64_t kFarBytes = (int64_t{1} << 31) / BigTile::B, kPart = kFarBytes / 8;
+  const int64_t elt = out_f32 != 0 ? 4 : 2;
   bool far = false;
-  for (int g = 0; g < a.n_lin; ++g) far = far || ldo[g] >= kFar;
+  for (int g = 0; g < a.n_lin; ++g) far = far || ldo[g] * elt >= kFarBytes;
   if (far) {
-    const int64_t elt = out_f32 != 0 ? 4 : 2;
     for (int g = 0; g < a.n_lin; ++g)
       for (int64_t r = 0; r < M; ++r)
         for (int64_t n = 0; n < N[g]; n += kPart) {

@@ -53,7 +53,7 @@ def test_int8_linear_leaves_a_wide_output_alone(dev):
 
 @pytest.mark.parametrize("stride", [(1 << 22) - 4, 1 << 22, (1 << 22) + 4])
 def test_int8_linear_rows_far_apart(dev, stride):
-    """Output rows at the limit of a tile's 32-bit offsets and past it."""
+    """Output rows on either side of the stride from which they go one by one."""
     from cast_amd import ops
     g = torch.Generator().manual_seed(3)
     M, N = 3, 512
@@ -67,6 +67,29 @@ def test_int8_linear_rows_far_apart(dev, stride):
     wide = wide.cpu()
     assert torch.equal(wide[:, :N], orc.int8_linear(x, xs, w, ws, bias))
     assert (wide[:, N:] == 7).all()
+
+
+# the widest stride of a tile's own stores, and the first past it, in bytes: 8 MiB
+@pytest.mark.parametrize("past", [False, True])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("N", [512, 49408])
+def test_int8_linear_whole_tile_of_far_rows(dev, N, dtype, past):
+    """All rows of a tile, 128 (few channels) and 256 (many: more than three rounds of the
+    small tiles): the last of the 256 begins just below 2^31 bytes from the first."""
+    from cast_amd import _lib
+    g = torch.Generator().manual_seed(7)
+    M = 256
+    stride = (8 << 20) // dtype.itemsize - (0 if past else 4)
+    x = torch.randint(-127, 128, (M, 128), generator=g, dtype=torch.int8)
+    w = torch.randint(-127, 128, (N, 128), generator=g, dtype=torch.int8)
+    xs, ws = torch.rand(M, generator=g), torch.rand(N, generator=g)
+    bias = torch.randn(N, generator=g).bfloat16()
+    print(f"int8 linear, {N} channels, rows {stride} of {dtype}", flush=True)
+    wide = torch.full((M, stride), 7.0, dtype=dtype, device=dev)
+    _lib.torch_ops().int8_linear_group(x.to(dev), xs.to(dev), [w.to(dev)], [ws.to(dev)],
+                                       [bias.to(dev)], [wide[:, :N]])
+    assert torch.equal(wide[:, :N].cpu(), orc.int8_linear(x, xs, w, ws, bias).to(dtype))
+    assert bool((wide[:, N:] == 7).all())
 
 
 @pytest.mark.parametrize("C", [8, 1016, 1032, 2048, 3064, 5120, 5128])
