@@ -150,11 +150,12 @@ __device__ __forceinline__ void lin_wait_barrier() {
 }
 
 // A workgroup tile of 4 wavefronts (2 along tokens x 2 along channels), each
-// T x T MFMA tiles of 32 x 32, over a ring of SLOTS K steps.
+// T x T MFMA tiles of 32 x 32, over a ring of two K steps.
 // WGS workgroups share a compute unit.
-template <int T_, int SLOTS_, int WGS_>
+template <int T_, int WGS_>
 struct LinTile {
-  static constexpr int T = T_, SLOTS = SLOTS_, WGS = WGS_;
+  static constexpr int T = T_, WGS = WGS_;
+  static constexpr int SLOTS = 2;                      // (the ring is unrolled by hand)
   static constexpr int B = 2 * 32 * T;                 // tokens and channels of a tile
   static constexpr int OB = B * kKS;                   // bytes of one operand's step
   static constexpr int U = OB / 1024 / kGemmWaves;     // 1 KiB copies per wavefront and operand
@@ -168,11 +169,11 @@ struct LinTile {
   static_assert(WGS * (SLOTS * 2 * OB + kGemmWaves * EB) <= 160 * 1024, "LDS of a compute unit");
 };
 
-using BigTile = LinTile<4, 2, 1>;  // 256 x 256, 64 KiB steps
+using BigTile = LinTile<4, 1>;  // 256 x 256, 64 KiB steps
 // 128 x 128, 32 KiB steps: two workgroups fill each other's waits (three
 // projections of 880 tokens 31.4 us against 33.1 with one of four slots, 2640
 // tokens 81 against 87)
-using MidTile = LinTile<2, 2, 2>;
+using MidTile = LinTile<2, 2>;
 
 // Where a tile's operands are and where its outputs go.
 struct TileSrc {
@@ -211,7 +212,6 @@ template <class L, bool OUT32>
 __global__ void __launch_bounds__(kGemmThreads) __attribute__((amdgpu_waves_per_eu(L::WGS, L::WGS)))
 int8_linear_kernel(LinearArgs a, int32_t per_wg, int32_t per_xcd) {
   constexpr int T = L::T, SLOTS = L::SLOTS, KS = L::KS;
-  static_assert(SLOTS == 2, "the unrolled ring");
   // (slots in arrays of their own: the compiler then knows that reads of one do
   // not alias the copies in flight into the others)
   __shared__ __attribute__((aligned(1024))) char s_0[2 * L::OB];

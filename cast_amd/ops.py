@@ -520,9 +520,10 @@ def quantize_key_select(k, valid, block_size, ksum, kmin, kmax, qhat, khat, k_se
         sm, src_len = None, 0
         B, H, L, D, NB = _bhld(k, block_size, fn)
         strides = (k.stride(0), k.stride(1), k.stride(2))
-    if not (k.dtype == torch.bfloat16 and D == 128 and block_size == 128 and NB <= 1024):
-        raise NotImplementedError(f"{fn}: fused launch needs bf16 keys, D 128, 128-key "
-                                  "blocks and at most 1024 blocks")
+    main_shape = k.dtype == torch.bfloat16 and D == 128 and block_size == 128
+    if not (NB <= 1024 if main_shape else sm is None and NB <= 256):
+        raise NotImplementedError(f"{fn}: the fused launch takes at most 1024 blocks of bf16 keys "
+                                  "with D 128 and 128-key blocks, else 256 of packed keys")
     for t in (ksum, kmin, kmax):
         if t.shape != (B * H, NB, D) or t.dtype != torch.float32 or not t.is_contiguous():
             raise ValueError(f"{fn}: statistics must be contiguous float32 [{B * H}, {NB}, {D}]")

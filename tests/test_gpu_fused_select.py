@@ -119,3 +119,25 @@ def test_fused_select_slot_token():
     names = ("k_i8", "k_scale", "kmean", "score", "indices", "counts")
     for name, a, b in zip(names, want, got):
         assert a.shape == b.shape and torch.equal(a, b), name
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("D,bs", [(128, 128), (128, 64), (64, 128), (64, 64)])
+def test_fused_select_of_a_few_blocks(D, bs, dtype):
+    """Packed keys of any shape up to 256 blocks, the main shape's up to 1024."""
+    from cast_amd import ops
+    dev = torch.device("cuda:0")
+    g = torch.Generator().manual_seed(D + bs)
+    main = dtype == torch.bfloat16 and D == 128 and bs == 128
+    for nb in (256, 257):
+        q, k = (torch.randn(1, 2, n * bs, D, generator=g).to(dtype).to(dev) for n in (17, nb))
+        qhat, _, _ = ops.pool_query(q, None, bs)
+        khat, ks, kn, kx = ops.pool_key(k, None, bs, stats=True)
+        if nb > 256 and not main:
+            with pytest.raises(NotImplementedError):
+                ops.quantize_key_select(k, None, bs, ks, kn, kx, qhat, khat, 9)
+            continue
+        sc = ops.block_scores(qhat, khat)
+        want = ops.quantize_key(k, None, bs, ks, kn, kx) + (sc, *ops.select_topk(sc, 9))
+        got = ops.quantize_key_select(k, None, bs, ks, kn, kx, qhat, khat, 9)
+        assert all(torch.equal(a, b) for a, b in zip(want, got))
