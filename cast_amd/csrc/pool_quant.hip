@@ -387,8 +387,11 @@ static void launch_score(const float* qhat, const float* khat, int64_t n_bh, int
   auto grid = [&](int64_t tq) {
     return dim3(static_cast<unsigned>(n_bh * ((nq + tq - 1) / tq) * tiles_k));
   };
-  // the largest query tile that the rows fill and that leaves the device a
-  // workgroup per compute unit
+  // the largest query tile that the rows fill and that leaves the device two
+  // (64 rows) or one (32) workgroups per compute unit: us with 64-, 32- and 16-row
+  // tiles, D 128, 24 x 330 x 853 (2016 tiles of 64) 35 / 37 / 46, 24 x 120 x 330 (288)
+  // 11.4 / 11.0 / 11.9, 24 x 60 x 330 (288 of 32) 9.3 / 8.4 / 8.6, 8 x 60 x 853 (224)
+  // 8.9 / 6.8 / 6.9, 1 x 60 x 330 (12) 8.7 / 6.2 / 5.1
   if (nq > 32 && n_bh * ((nq + 63) / 64) * tiles_k >= 512)
     score_kernel<D, 4><<<grid(64), dim3(256), 0, s>>>(qhat, khat, nq, nk, score);
   else if (nq > 16 && n_bh * ((nq + 31) / 32) * tiles_k >= 256)
@@ -832,7 +835,10 @@ static int quantize_key_impl(const void* k, int dtype, int64_t batch, int64_t n_
   const int64_t n_tokens = n_blocks * block_size;
   if (sel) {
     const int64_t nq = sel->n_q, tiles_k = (n_blocks + 63) / 64;
-    const bool rows32 = nq > 16 && nbh * ((nq + 31) / 32) * tiles_k >= 64;
+    // 32-row tiles from 160 of them on (us with 32- and 16-row tiles, 24 heads: 60 x 303
+    // (240 tiles) 7.0 / 7.6, 28 x 600 (240) 9.2 / 10.1, 28 x 303 (120) 7.1 / 6.0; 8 heads:
+    // 60 x 600 (160) 6.3 / 6.6, 60 x 303 (80) 6.7 / 5.7)
+    const bool rows32 = nq > 16 && nbh * ((nq + 31) / 32) * tiles_k >= 160;
     const int64_t tq = rows32 ? 32 : 16;
     const int64_t n_score = nbh * ((nq + tq - 1) / tq) * tiles_k;
     const dim3 grid(static_cast<unsigned>(n_score + nbh * (head_dim / 16)));

@@ -15,8 +15,21 @@
 //   int8 D 128, 64 x 128         298 / 355 / 522       64 /  75 / 102
 //   int8 D 64, 64 x 64           202 / 214 / 261       51 /  47 /  53
 // and at 8 heads x 1024 rows x 32 of 64 key blocks, int8 D 128, 64 x 128:
-// 51 / 41 / 48.  (bf16 D 64 keeps FEW throughout: within 5% at 3584 rows.)
-// Validity bytes are read by callers of the C ABI without bits only: FEW.
+// 51 / 41 / 48.  bf16 D 64 keeps FEW throughout: 24 heads, FEW / MANY,
+//                1792 query rows    3584 query rows
+//   128 x 128    165 / 165          294 / 288
+//   128 x 64     203 / 211          288 / 281
+//   64 x 128     180 / 211          317 / 280
+//   64 x 64      202 / 198          350 / 279
+// (64-row blocks pass to MANY's side between 84 and 168 query blocks an XCD; no
+// line is drawn there.)
+// Validity bytes: FEW.
+//
+// Wavefronts per SIMD that MANY's register budget allows: as many as the
+// workgroups that the LDS holds come to, three at most (159 to 170 VGPRs).  A
+// bf16 ring of D 128 takes 50 KiB, so three workgroups share a compute unit: 128-row
+// blocks (four wavefronts) three, 64-row blocks (two) two.  int8 rings take 38 KiB,
+// four workgroups: 64-row blocks two.  D 64 rings of 19 to 38 KiB: three.
 #include "sparse_attn_kernel.h"
 
 namespace rcsa {
