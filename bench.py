@@ -470,6 +470,12 @@ def main() -> int:
     torch.cuda.synchronize()
     ms_per_step = (time.perf_counter() - t0) * 1e3 / args.steps
     host_ms_per_step = (t_enqueued - t0) * 1e3 / args.steps
+    # (twice, the second time counts: on a cold machine one of the first events' entries
+    # takes 35 ms on the host, between its two events)
+    instrumented(names, args.steps)
+    torch.cuda.synchronize()
+    for ev in events.values():
+        ev.clear()
     instrumented(names, args.steps)
     torch.cuda.synchronize()
     # the same steps issued by the eager Python call, for comparison
