@@ -69,10 +69,11 @@ def rcsa_attention(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor,
     With ``int8`` QK^T runs on int8 MFMA over smoothed per-block quantised
     Q/K; otherwise on bf16 MFMA.  ``n_split`` splits every block list over
     that many workgroups (None: chosen from the device's compute-unit count).
-    ``fuse_select`` (int8, index order, bf16 keys of D 128 in 128-key blocks)
-    scores and selects inside the key quantiser's launch; otherwise
-    ``overlap`` runs the scores and the top-k on a side stream beside the
-    int8 key pass.  Results are identical either way.
+    ``fuse_select`` (int8, index order; up to 1024 blocks of bf16 keys with D 128
+    and 128-key blocks, up to 256 of packed keys in other shapes) scores in the
+    key mean's launch and selects in the key quantiser's; otherwise ``overlap``
+    runs the scores and the top-k on a side stream beside the int8 key pass
+    (of 4096 key tiles at most: before it).  Results are identical either way.
 
     ``q_slot_token`` / ``k_slot_token`` (both or neither; e.g. a
     ``CompactLayout.slot_token``): q, k and v are token-major ``[B, L, H, D]``

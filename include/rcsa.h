@@ -662,8 +662,8 @@ int rcsa_order_split_lists(const int32_t* block_indices, const int32_t* block_in
  * [N][K] (both 16-byte aligned), w_scale fp32 [N] (16-byte aligned), bias bf16
  * [N] or NULL (then out = bf16(float(acc) * x_scale * w_scale)); out bf16 with
  * row stride ldo (8-byte aligned).  N a multiple of 256, K a multiple of 128.
- * The launch is persistent (one workgroup per compute unit, each with a fixed
- * share of the tiles): it expects the device to itself, and beside other
+ * The launch is persistent (one workgroup per compute unit for 256 x 256 tiles, two
+ * for 128 x 128 ones, each with a fixed share of the tiles): it expects the device to itself, and beside other
  * kernels it stays correct but runs as slowly as its latest workgroup.
  *
  * rcsa_int8_linear_group: n_linear (1 to 4) such projections of one x in one
