@@ -9,7 +9,8 @@
 // bad layout.  Every tensor is checked to span the elements the call's dims
 // and strides reach, so no argument combination makes a kernel read or write
 // past the tensors it was given.  Nothing here synchronises, and nothing but
-// layer_call and order_lists, which allocate their outputs, allocates device memory.
+// layer_call, order_lists and valid_bits, which allocate their outputs, allocates device
+// memory.
 //
 // The C ABI is bound at load time (rcsa::bind_library) from the library the
 // Python side loaded, so one librcsa.so serves both the ctypes binding and
@@ -626,6 +627,25 @@ std::vector<at::Tensor> order_lists(const at::Tensor& indices, const at::Tensor&
   return res;
 }
 
+// Byte flags (whole blocks of block_size keys) as bits: int32 [blocks, block_size / 32].
+at::Tensor valid_bits(const at::Tensor& valid, int64_t block_size) {
+  const char* op = "valid_bits";
+  const Api& a = api(op);
+  int dev = -1;
+  on_device(op, dev, valid, "valid");
+  want_bytes(op, valid, "valid");
+  TORCH_CHECK(valid.is_contiguous() && block_size > 0 && block_size % 32 == 0 &&
+                  valid.numel() > 0 && valid.numel() % block_size == 0, op,
+              ": valid must be contiguous, whole blocks of a multiple of 32");
+  const Launch l(device_of(op, dev));
+  const at::Tensor bits = at::empty({valid.numel() / block_size, block_size / 32},
+                                    valid.options().dtype(at::kInt));
+  check_status(a, op, a.order_split_lists(
+      nullptr, nullptr, 0, 0, 0, 0, 0, 0, nullptr, 0, 0, 0, 0, 0, 0, 1, nullptr, nullptr,
+      ptr<const uint8_t>(valid), valid.numel(), ptr<uint32_t>(bits), l.stream));
+  return bits;
+}
+
 // The layer call of cast_amd/pipeline.py (rcsa_attention) in one op: its launches
 // in stream order on one stream, its outputs allocated here.  A call of a few
 // blocks is bound by the host work between its launches (4 heads x 4 query blocks
@@ -825,6 +845,7 @@ TORCH_LIBRARY(rcsa, m) {
   m.def("order_lists(Tensor indices, Tensor counts, int n_kblocks, Tensor? rows, Tensor? valid, "
         "int n_split=1) -> Tensor[]",
         &order_lists);
+  m.def("valid_bits(Tensor valid, int block_size) -> Tensor", &valid_bits);
   m.def(
       "layer_call(Tensor q, Tensor k, Tensor v, Tensor? q_valid, Tensor? k_valid, int block_size, "
       "Tensor? row_k, int row_k_stride_bh, int k_fixed, int max_k, Tensor? forced, "

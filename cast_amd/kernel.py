@@ -61,13 +61,17 @@ def _lists_and_bits(q, k, indices, counts, key_valid, block_m, block_n):
 def _bits_pay(q, k, block_m, block_n, max_k) -> bool:
     """Whether the validity as bits, whose forms of the attention are faster, is worth the
     launch that makes them: keys beyond an XCD's L2, and two rounds of query blocks or
-    48 MB of listed blocks (64 x 128 blocks, 24 heads x 3520 rows x 12 of 42 blocks 102 us
-    against 145 with bytes, 8 x 1760 x 38 of 128 63 against 71, x 12 31 against 29)."""
+    28 MB of listed blocks an XCD, 48 MB where its keys are 16 MB (64 x 128 blocks, 24
+    heads x 3520 rows x 12 of 42 blocks 102 us against 145 with bytes, 8 x 1760 x 38 of 128
+    63 against 71, 24 x 880 x 11 of 43 41.6 against 43.0, 8 x 1760 x 12 of 128 31 against
+    29, 12 x 880 x 30 of 303 57.0 against 55.8)."""
     B, H, L, D = k.shape
     n_bh = B * H
-    return (k.is_cuda and ops.order_helps(n_bh, L, 4 * D, block_n, max_k)
-            and (ops.two_rounds(n_bh, q.shape[2], block_m)
-                 or ops.listed_bytes(n_bh, q.shape[2], 4 * D, block_m, block_n, max_k) > 48 << 20))
+    if not (k.is_cuda and ops.order_helps(n_bh, L, 4 * D, block_n, max_k)):
+        return False
+    least = 28 if -(-n_bh // 8) * L * 4 * D <= 16 << 20 else 48
+    return (ops.two_rounds(n_bh, q.shape[2], block_m)
+            or ops.listed_bytes(n_bh, q.shape[2], 4 * D, block_m, block_n, max_k) > least << 20)
 
 
 def longcat_asymmetric(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor,

@@ -7,6 +7,7 @@ stream.  No function reads device memory back to the host.
 from __future__ import annotations
 
 import ctypes
+import functools
 import math
 from typing import NamedTuple, Optional
 
@@ -602,7 +603,7 @@ def _split_plan(B, H, Lq, D, block_m, max_k, n_split, device, fn):
     compute units best (rcsa_attn_split_plan); the workspace holds the
     partial results that the merge pass combines."""
     if n_split is None:
-        n_split = _planned_split(B, H, Lq, block_m, max_k, fn)
+        n_split = planned_split(B, H, Lq, block_m, max_k, fn)
     n_split = int(n_split)
     if n_split < 1:
         raise ValueError(f"{fn}: n_split must be >= 1")
@@ -612,20 +613,17 @@ def _split_plan(B, H, Lq, D, block_m, max_k, n_split, device, fn):
     return n_split, torch.empty(nbytes, dtype=torch.uint8, device=device), nbytes
 
 
-def _planned_split(B, H, Lq, block_m, max_k, fn) -> int:
+def planned_split(B, H, Lq, block_m, max_k, fn) -> int:
+    """The n_split that the attention chooses (rcsa_attn_split_plan)."""
     ns = ctypes.c_int64(1)
     check(_lib.load().rcsa_attn_split_plan(B, H, Lq, block_m, max_k, ctypes.byref(ns)), fn)
     return ns.value
 
 
-def split_rows(B: int, H: int, Lq: int, block_m: int, max_k: int) -> str:
-    """Of the attention's query blocks, those whose lists it cuts into shares by its own
-    choice of n_split: "none", "some" (each XCD's past its full rounds) or "all"."""
-    if _planned_split(B, H, Lq, block_m, max_k, "split_rows") == 1:
-        return "none"
-    per_xcd = -(-B * H * -(-Lq // block_m) // 8)
-    cus = torch.cuda.get_device_properties(torch.cuda.current_device()).multi_processor_count
-    return "some" if per_xcd >= cus // 8 else "all"
+@functools.lru_cache(maxsize=None)
+def _xcd_cus(device: int) -> int:
+    """Compute units of an XCD."""
+    return torch.cuda.get_device_properties(device).multi_processor_count // 8
 
 
 def _expand_lists(indices, counts, B, H):
@@ -664,8 +662,8 @@ def listed_bytes(n_bh: int, q_len: int, key_bytes: int, block_m: int, block_n: i
 def two_rounds(n_bh: int, q_len: int, block_m: int) -> bool:
     """Whether every XCD has two rounds of query blocks: the attention then runs several
     workgroups to a compute unit."""
-    cus = torch.cuda.get_device_properties(torch.cuda.current_device()).multi_processor_count
-    return -(-n_bh * -(-q_len // block_m) // 8) >= 2 * (cus // 8)
+    per_xcd = -(-n_bh * -(-q_len // block_m) // 8)
+    return per_xcd >= 2 * _xcd_cus(torch.cuda.current_device())
 
 
 def order_pays(n_bh: int, q_len: int, k_len: int, key_bytes: int, block_m: int, block_n: int,
@@ -728,12 +726,13 @@ def order_for_attention(indices, counts, q_shape, k_len: int, block_m: int, bloc
     ``n_split`` (None: the one that the call will choose).  Without ``rows`` the first rows
     are its query blocks (:func:`lists_cover`); more are left out."""
     B, H, Lq = q_shape[:3]
-    indices, counts = _expand_lists(indices, counts, B, H)
+    if not indices.shape[:2] == counts.shape[:2] == (B, H):
+        indices, counts = _expand_lists(indices, counts, B, H)
     if rows is None:
         nqb = -(-Lq // block_m)
         indices, counts = indices[:, :, :nqb], counts[:, :, :nqb]
     if n_split is None:
-        n_split = _planned_split(B, H, Lq, block_m, indices.shape[3], "order_lists")
+        n_split = planned_split(B, H, Lq, block_m, indices.shape[3], "order_lists")
     elif not 1 <= int(n_split) <= 16:  # (refused by the attention)
         n_split = 1
     return order_lists(indices, counts, -(-k_len // block_n), rows=rows, valid=valid,
@@ -747,14 +746,8 @@ def valid_bits(valid: torch.Tensor, block_size: int) -> torch.Tensor:
     if block_size % 32 or valid.numel() % block_size:
         raise ValueError("valid_bits: block_size must be a multiple of 32 dividing the keys")
     if valid.is_cuda and valid.numel() > 0:
-        flags = _bytes_mask(valid.reshape(-1), valid.device)
-        bits = torch.empty(flags.numel() // block_size, block_size // 32, device=valid.device,
-                           dtype=torch.int32)
-        with torch.cuda.device(valid.device):
-            check(_lib.load().rcsa_order_lists(
-                None, None, 0, 0, 0, 0, 0, 0, None, 0, 0, 0, 0, 0, 0, None, None,
-                flags.data_ptr(), flags.numel(), bits.data_ptr(), _stream()), "valid_bits")
-        return bits
+        return _lib.torch_ops().valid_bits(_bytes_mask(valid.reshape(-1), valid.device),
+                                           block_size)
     words = (valid.reshape(-1, block_size // 32, 32) != 0).to(torch.int64)
     bits = (words << torch.arange(32, device=valid.device)).sum(-1)
     return torch.where(bits >= 2 ** 31, bits - 2 ** 32, bits).to(torch.int32)

@@ -263,6 +263,9 @@ def relay_attention(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, layout, s
                and selected.shape[2] == layout.n_blocks
                and ops.order_helps(B * H, n_kblocks * bs, (3 if int8 else 4) * D, bs,
                                    selected.shape[3]))
+    if n_split is None:
+        n_split = ops.planned_split(B, H, rows.numel() * bs, bs, selected.shape[3],
+                                    "relay_attention")
     if ordered:  # the query blocks' rows, ascending, in one launch instead of two gathers
         # (0.99 to 1.58 times as fast over 1 to 24 heads, 12 to 44 frames, from one L2 of keys on)
         idx, cnt = ops.order_for_attention(selected, counts, (B, H, rows.numel() * bs),
@@ -277,8 +280,7 @@ def relay_attention(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, layout, s
     n_qblocks = rows.numel()
     half = None
     if q.is_cuda and layout.query_half is not None:
-        cus = torch.cuda.get_device_properties(q.device).multi_processor_count
-        if -(-B * H * n_qblocks // 8) >= 2 * (cus // 8):
+        if ops.two_rounds(B * H, n_qblocks * bs, bs):
             half = layout.query_half
     bm, q_slot, out_row = ((bs // 2, *half) if half is not None
                            else (bs, layout.query_slot_token, layout.query_out_row))

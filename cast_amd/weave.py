@@ -169,7 +169,7 @@ def _available_layers(weave):
 
 
 def _attention(q, k, v, idx4, cnt3, slot, token_to_packed, mask, bs, int8: bool, kq=None,
-               ordered=False):
+               ordered=False, n_split=None):
     """Block-sparse attention of the packed blocks named by the slot map, the
     output in the token rows [B, L, H, D] (bf16).  The copy rings read the
     token-major sources through the slot map for D 128 and 128-token blocks;
@@ -182,14 +182,16 @@ def _attention(q, k, v, idx4, cnt3, slot, token_to_packed, mask, bs, int8: bool,
         return ops.sparse_attn_int8(q_i8, q_scale, k_i8, k_scale,
                                     vb if ring else ops.pack_tokens(vb, slot), idx4, cnt3, None,
                                     block_m=bs, block_n=bs, block_mask=mask, out_token=slot,
-                                    out_len=L, v_token=slot if ring else None, ordered=ordered)
+                                    out_len=L, v_token=slot if ring else None, ordered=ordered,
+                                    n_split=n_split)
     qb, kb = (x if x.dtype == torch.bfloat16 else x.to(torch.bfloat16) for x in (q, k))
     if ring:
         return ops.sparse_attn_bf16(qb, kb, vb, idx4, cnt3, None, block_m=bs, block_n=bs,
-                                    block_mask=mask, q_token=slot, kv_token=slot, ordered=ordered)
+                                    block_mask=mask, q_token=slot, kv_token=slot, ordered=ordered,
+                                    n_split=n_split)
     packed = [ops.pack_tokens(x, slot) for x in (qb, kb, vb)]
     out = ops.sparse_attn_bf16(*packed, idx4, cnt3, None, block_m=bs, block_n=bs,
-                               block_mask=mask, ordered=ordered)
+                               block_mask=mask, ordered=ordered, n_split=n_split)
     return ops.unpack_tokens(out, token_to_packed.to(device=q.device, dtype=torch.long))
 
 
@@ -331,13 +333,12 @@ def compact_cwca_attention(weave, module: Any, q: torch.Tensor, k: torch.Tensor,
     # The router reads the rank order; the attention takes ascending lists, but in rank
     # order those that it cuts into shares: a share of an ascending list is a run of
     # neighbouring frames, whose partial output is larger and rounds further off (1 head,
-    # 8 + 12 frames, int8: 2.44e-3 from float64, 2.41e-3 in rank order).  Where it cuts
-    # them all, it orders every share itself.
-    cut = ops.split_rows(B, H, blocks * bs, bs, width)
-    ordered = route != "refine" and cut != "all"
+    # 8 + 12 frames, int8: 2.44e-3 from float64, 2.41e-3 in rank order).
+    n_split = ops.planned_split(B, H, blocks * bs, bs, width, "compact_cwca_attention")
+    ordered = route != "refine"
     indices, _ = ops.select_topk(score, row_k, forced=local, max_k=width,
                                  order="rank" if not ordered else
-                                 "index" if cut == "none" or width > 2048 else "split")
+                                 "index" if n_split == 1 or width > 2048 else "split")
     selected = indices.view(B, H, blocks, width)
     counts = row_k[None, None].expand(B, H, -1)
     if not ordered:  # the router's own kernels read it whole
@@ -393,7 +394,7 @@ def compact_cwca_attention(weave, module: Any, q: torch.Tensor, k: torch.Tensor,
 
     # ---- attention and unpack (:6086-6095) ----
     out = _attention(q, k, v, selected.to(torch.int32).contiguous(), counts, slot,
-                     layout.compact_token_to_packed, mask, bs, int8, kq, ordered)
+                     layout.compact_token_to_packed, mask, bs, int8, kq, ordered, n_split)
     if provider is not None:  # the closed loop conserves blocks * mean_degree edges
         edges, mean_f = blocks * mean_degree, float(mean_degree)
     else:

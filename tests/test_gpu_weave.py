@@ -327,7 +327,7 @@ def test_woven_lists_of_cut_rows_stay_ranked(dev):
     _run(_weave(prov), q, k, v, lay, 1, cap)
     sel, cnt = cap["selected"].cpu().long(), cap["counts"].cpu()
     n = sel.shape[2]
-    assert ops.split_rows(1, 1, n * 128, 128, sel.shape[3]) == "all"
+    assert ops.planned_split(1, 1, n * 128, 128, sel.shape[3], "test") > 1
     local = rlayout.local_stencil(n, 6, 5)
     for r in range(n):
         near = torch.nonzero(local[r]).flatten().tolist()
