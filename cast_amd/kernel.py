@@ -93,8 +93,8 @@ def longcat_asymmetric(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor,
         bits = None
         if ready is not None:
             indices, counts, bits = ready
-        elif indices.ndim == 4 and _bits_pay(q, k, query_block_size, key_block_size,
-                                             indices.shape[3]):
+        elif indices.ndim == 4 and valid.device == k.device \
+                and _bits_pay(q, k, query_block_size, key_block_size, indices.shape[3]):
             bits = ops.valid_bits(valid, key_block_size)
         if bits is not None:  # (a few blocks: the bytes, without another launch)
             return ops.sparse_attn_bf16(q, k, v, indices, counts, None,

@@ -223,3 +223,20 @@ def test_order_rule(bm, H, Lq, nkb, K, int8, pays):
     if torch.cuda.get_device_properties(0).multi_processor_count != 256:
         pytest.skip("sizes for 256 compute units")
     assert ops.order_pays(H, Lq, nkb * 128, (3 if int8 else 4) * 128, bm, 128, K, int8) == pays
+
+
+def test_asymmetric_flags_from_the_host():
+    """Key flags in host memory are taken whatever the size of the call."""
+    from cast_amd import kernel
+    g = torch.Generator(device="cuda").manual_seed(8)
+    H, D, nkb, Lq, K = 8, 128, 80, 1792, 20
+    assert kernel.ops.listed_bytes(H, Lq, 4 * D, 64, 128, K) > 28 << 20
+    q, k, v = (torch.randn(1, H, n, D, device="cuda", generator=g).bfloat16()
+               for n in (Lq, nkb * 128, nkb * 128))
+    idx = torch.rand(1, H, Lq // 64, nkb, device="cuda", generator=g).argsort(-1)[..., :K].int()
+    cnt = torch.full((1, H, Lq // 64), K, dtype=torch.int32, device="cuda")
+    flags = torch.rand(nkb * 128, device="cuda", generator=g) > 0.1
+    run = lambda f: kernel.longcat_asymmetric(q, k, v, idx.contiguous(), cnt, f,
+                                              query_block_size=64, key_block_size=128)
+    torch.testing.assert_close(run(flags.cpu()).float(), run(flags).float(), rtol=2.0 ** -7,
+                               atol=2.0 ** -9)
